@@ -1,0 +1,693 @@
+// nd_factor.hip -- multifrontal Cholesky factor of the shell matrices under a
+// nested-dissection order.
+//
+// The mesh graph is cut by short separators (nd_order.h); every separator
+// and every leaf is a front of ns pivot dofs and nb boundary dofs, m = ns +
+// nb.  The fronts of one distance from the root form a level and are factored
+// together, deepest level first, for several designs at once.  The factor of
+// a front is the m x ns panel
+//
+//   M = [ X ; -W ],   X = L^{-1},  W = L21 L^{-1},   F11 = L L^T, L21 = F21 X^T,
+//
+// so a solve needs one product with M per front and sweep:
+//   up:   y = X v_J,  u_B = v_B - W v_J          (v = b plus the children's u)
+//   down: x_J = X^T y - W^T x_B = M^T [y ; x_B].
+//
+// Factoring a level takes the pivots in blocks of 64.  At block k the panel's
+// columns left of k already hold forward-eliminated columns Y of the identity
+// (rows below the pivots: of zero), the columns right of it what is left of
+// F.  With X_k the inverse Cholesky factor of the diagonal block and
+//   Q_k = [ (X_k Y_k)^T ; X_k^T ; F_ik X_k^T ]   (rows before, at, after k)
+// one update C_ij -= Q_ik Q_jk^T serves both: for columns j < k it goes on
+// eliminating Y, for j = k it starts the identity's column (C_ik = 0), for j
+// > k it is the Cholesky update.  After the last block the panel is M, and
+// the rows of Q at the boundary are L21: the Schur complement of the front is
+// one product S = (children's S) - L21 L21^T.
+//
+// The short separators are what this form is for: a band (level) order of the
+// 200 x 400 cylinder stores 27.7 GB and needs 10.6 Tflop, this order 1.45 GB
+// and 0.17 Tflop, and the largest front has 2,400 pivots.  A factorisation is
+// bound by the chain of about 100 pivot blocks of its levels (latency), a
+// solve by the two reads of M and the chain of 2 x 14 levels.
+//
+// Every sum has a fixed order (no atomics): a factor and its solves are
+// reproducible bit for bit.
+#include "nd_factor.h"
+
+#include <algorithm>
+
+#include "nd_layout.h"
+
+namespace shellgpu {
+
+namespace {
+
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(1))) const double gcdouble;
+typedef __attribute__((address_space(1))) double gdouble;
+
+constexpr int kB = 64;  // pivot block
+// leaves of the dissection: 24 nodes (144 dofs).  Fewer, larger leaves give
+// fewer fronts but more fill (200 x 400 cylinder: 1.45 GB at 24 nodes, 1.33
+// at 16 with a third more fronts, 1.79 at 48)
+constexpr int kLeafNodes = 24;
+
+struct LevelArgs {
+  const NdDev *fronts;  // the level's first front
+  const NdDev *all;     // front 0
+  const int *lists;
+  double *M;
+  double *Q;
+  double *S;        // the level's Schur complements
+  const double *Sc; // the children's
+  long sM, sQ, sS, sSc;  // per design
+  int k;            // pivot block
+  int tr, tc;       // tiles per front along rows and columns
+};
+
+// one 32 x 32 block of acc += A B^T: A rows ra (clamped by the caller), B rows
+// rb, columns 0 .. n of both (column stride ld); D^T layout of
+// v_mfma_f64_16x16x4f64 as measured on gfx950 (gemm_f64.hip): lane l, element
+// e hold row l % 16, column 4 e + l / 16
+struct Frag {
+  v4d c[2][2];
+};
+
+// 16 columns at a time, the loads of the next 16 in flight during the matrix
+// instructions of the current; columns past n count as zero
+template <typename FA, typename FB>
+__device__ __forceinline__ void mma32(Frag &f, int n, FA a_at, FB b_at) {
+  const int lk = (threadIdx.x & 63) >> 4;
+  double a[2][4][2], b[2][4][2];
+  auto load = [&](int buf, int k0) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int kk = k0 + 4 * q + lk, kc = min(kk, n - 1);
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const double v = a_at(i, kc);
+        a[buf][q][i] = kk < n ? v : 0.0;
+        b[buf][q][i] = b_at(i, kc);
+      }
+    }
+  };
+  auto mul = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          f.c[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[buf][q][j], a[buf][q][i], f.c[i][j], 0, 0, 0);
+  };
+  load(0, 0);
+  for (int k0 = 0; k0 < n; k0 += 32) {
+    load(1, k0 + 16);
+    mul(0);
+    if (k0 + 16 >= n) break;
+    load(0, k0 + 32);
+    mul(1);
+  }
+}
+
+__device__ __forceinline__ void clear(Frag &f) {
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) f.c[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+}
+
+// matrix blocks -> panels (zeroed before): block p of the pattern goes to
+// base[p] with leading dimension ld[p] (base -1: the transposed block is
+// stored).  flag[p]: bits 6 + c mark BC columns, zeroed for the symmetric
+// elimination (BC rows already are), bit 12 a diagonal block, of which the
+// lower triangle is stored: nothing above the diagonal of a panel is written
+// before its pivot block is, and solves count it as zero.
+__global__ __launch_bounds__(256) void nd_scatter_kernel(int nnzb, const double *__restrict__ vals, long vstride,
+                                                         const long *__restrict__ base, const int *__restrict__ ld,
+                                                         const int *__restrict__ flag, double *__restrict__ M,
+                                                         long stride) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= 36L * nnzb) return;
+  const int p = (int)(i / 36), e = (int)(i % 36), r = e / 6, c = e % 6;
+  if (base[p] < 0) return;
+  const int fl = flag[p];
+  const bool diag = (fl >> 12) & 1;
+  if (diag && c > r) return;
+  double v = vals[blockIdx.y * vstride + i];
+  if (((fl >> (6 + c)) & 1) && !(diag && r == c)) v = 0.0;
+  M[blockIdx.y * stride + base[p] + (long)c * ld[p] + r] = v;
+}
+
+// panel columns of a front += its children's Schur complements
+__global__ __launch_bounds__(256) void nd_gather_kernel(LevelArgs a) {
+  const int f = blockIdx.x / (a.tr * a.tc), t = blockIdx.x - f * a.tr * a.tc;
+  const NdDev d = a.fronts[f];
+  const int i = kB * (t % a.tr) + (threadIdx.x & 63), c0 = kB * (t / a.tr);
+  if (d.child[0] < 0 || c0 >= d.ns || i >= d.m || kB * (t % a.tr) + kB <= c0) return;
+  const int mn = d.m / 6, ri = i / 6, rr = i - 6 * ri;
+  const int *lists = a.lists + d.lists;
+  gdouble *C = (gdouble *)(a.M + blockIdx.y * a.sM + d.M);
+  int ir[2], ldc[2];
+  gcdouble *Sc[2];
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    ir[c] = -1;
+    if (d.child[c] >= 0) {
+      const NdDev ch = a.all[d.child[c]];
+      ir[c] = lists[(1 + c) * mn + ri];
+      ldc[c] = ch.m - ch.ns;
+      Sc[c] = (gcdouble *)(a.Sc + blockIdx.y * a.sSc + ch.S);
+    }
+  }
+  if (ir[0] < 0 && ir[1] < 0) return;
+  for (int j = c0 + (threadIdx.x >> 6); j < min(c0 + kB, min(d.ns, i + 1)); j += 4) {
+    const int cj = j / 6, cc = j - 6 * cj;
+    double v = 0.0;
+    bool any = false;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      if (ir[c] < 0) continue;
+      const int ic = lists[(1 + c) * mn + cj];
+      if (ic < 0) continue;
+      v += Sc[c][6 * ir[c] + rr + (long)(6 * ic + cc) * ldc[c]];
+      any = true;
+    }
+    if (any) C[i + (long)j * d.m] += v;
+  }
+}
+
+// diagonal block k: X_k = chol(C_kk)^{-1} into C_kk (zero above the
+// diagonal) and its transpose into Q_kk; one workgroup per front and design
+constexpr int kDiagThreads = 256;
+__global__ __launch_bounds__(kDiagThreads) void nd_diag_kernel(LevelArgs a, int *info) {
+  constexpr int ld = kB + 1;
+  __shared__ double L[kB * ld], Y[kB * ld], piv[kB];
+  const NdDev d = a.fronts[blockIdx.x];
+  const int k0 = kB * a.k;
+  if (k0 >= d.ns) return;
+  const int n = min(kB, d.ns - k0), t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  gdouble *C = (gdouble *)(a.M + blockIdx.y * a.sM + d.M + k0 + (long)k0 * d.m);
+  gdouble *Q = (gdouble *)(a.Q + blockIdx.y * a.sQ + d.Q + k0 + (long)k0 * d.m);
+  for (int e = t; e < kB * kB; e += kDiagThreads) {
+    const int i = e % kB, j = e / kB;
+    L[i * ld + j] = i < n && j <= i ? C[i + (long)j * d.m] : 0.0;
+    Y[i * ld + j] = i == j ? 1.0 : 0.0;
+  }
+  __syncthreads();
+  bool bad = false;
+  for (int j = 0; j < n; j++) {
+    double p = L[j * ld + j];
+    if (!(p > 0.0)) {
+      bad = true;
+      p = 1.0;
+    }
+    if (t == 0) piv[j] = p;
+    const double rp = 1.0 / p;
+    // lane: trailing column (lane > j) or column of the inverse (lane <= j)
+    const double *src = lane > j ? L : Y;
+    const double top = lane > j ? L[lane * ld + j] : Y[j * ld + lane];
+    double r[16], v[16];
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+      const int i = j + 1 + wave + 4 * s;
+      r[s] = v[s] = 0.0;
+      if (i < n) {
+        r[s] = L[i * ld + j] * rp;
+        if (lane <= i) v[s] = src[i * ld + lane];
+      }
+    }
+    double *dst = lane > j ? L : Y;
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+      const int i = j + 1 + wave + 4 * s;
+      if (i < n && lane <= i) dst[i * ld + lane] = v[s] - r[s] * top;
+    }
+    __syncthreads();
+  }
+  for (int e = t; e < n * n; e += kDiagThreads) {
+    const int i = e % n, c = e / n;
+    const double x = i >= c ? Y[i * ld + c] / sqrt(piv[i]) : 0.0;
+    C[i + (long)c * d.m] = x;
+  }
+  for (int e = t; e < n * n; e += kDiagThreads) {
+    const int c = e % n, i = e / n;
+    Q[c + (long)i * d.m] = i >= c ? Y[i * ld + c] / sqrt(piv[i]) : 0.0;
+  }
+  if (t == 0 && bad) info[blockIdx.y] = 1;
+}
+
+// Q_ik = C_ik X_k^T for the rows after block k (tiles 0 .. tr), and the row
+// block itself, C_kj = X_k C_kj and Q_jk = C_kj^T, for the columns before it
+// (tiles tr .. tr + k)
+__global__ __launch_bounds__(256) void nd_scale_kernel(LevelArgs a) {
+  const int tiles = a.tr + a.k;
+  const int f = blockIdx.x / tiles, t = blockIdx.x - f * tiles;
+  const NdDev d = a.fronts[f];
+  const int k0 = kB * a.k;
+  if (k0 >= d.ns) return;
+  const int n = min(kB, d.ns - k0), m = d.m;
+  gdouble *C = (gdouble *)(a.M + blockIdx.y * a.sM + d.M);
+  gdouble *Q = (gdouble *)(a.Q + blockIdx.y * a.sQ + d.Q);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int wm = 32 * (wave & 1), wn = 32 * (wave >> 1);
+  Frag acc;
+  clear(acc);
+  if (t < a.tr) {
+    const int r0 = k0 + n + kB * t + wm;
+    if (r0 >= m || wn >= n) return;
+    long ra[2], rb[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      ra[i] = min(r0 + 16 * i + lr, m - 1) + (long)k0 * m;
+      rb[i] = k0 + min(wn + 16 * i + lr, n - 1) + (long)k0 * m;
+    }
+    mma32(acc, n, [&](int i, int kk) { return C[ra[i] + (long)kk * m]; },
+          [&](int i, int kk) { return C[rb[i] + (long)kk * m]; });
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int r = r0 + 16 * i + lr;
+      if (r >= m) continue;
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int c = wn + 16 * j + 4 * e + lk;
+          if (c < n) Q[r + (long)(k0 + c) * m] = acc.c[i][j][e];
+        }
+    }
+    return;
+  }
+  // rows of block k (n of them), columns of block j < k (64 of them)
+  const int c0 = kB * (t - a.tr);
+  long ra[2], rb[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    ra[i] = k0 + min(wm + 16 * i + lr, n - 1) + (long)k0 * m;
+    rb[i] = k0 + (long)(c0 + wn + 16 * i + lr) * m;
+  }
+  mma32(acc, n, [&](int i, int kk) { return C[ra[i] + (long)kk * m]; },
+        [&](int i, int kk) { return C[rb[i] + kk]; });
+  __syncthreads();  // the tile is read in full by both row halves
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int r = wm + 16 * i + lr;
+    if (r >= n) continue;
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int c = c0 + wn + 16 * j + 4 * e + lk;
+        C[k0 + r + (long)c * m] = acc.c[i][j][e];
+        Q[c + (long)(k0 + r) * m] = acc.c[i][j][e];
+      }
+  }
+}
+
+// C_ij -= Q_ik Q_jk^T for the rows after block k: columns before k, column
+// block k (from zero), and the trailing lower triangle
+__global__ __launch_bounds__(256) void nd_update_kernel(LevelArgs a) {
+  const int f = blockIdx.x / (a.tr * a.tc), t = blockIdx.x - f * a.tr * a.tc;
+  const NdDev d = a.fronts[f];
+  const int k0 = kB * a.k, ns = d.ns, m = d.m;
+  if (k0 >= ns) return;
+  const int n = min(kB, ns - k0), rs = k0 + n, tj = t / a.tr;
+  const int r0 = rs + kB * (t % a.tr);
+  const int c0 = tj <= a.k ? kB * tj : rs + kB * (tj - a.k - 1);
+  if (r0 >= m || c0 >= ns || r0 + kB <= c0) return;
+  const int cw = tj == a.k ? n : min(kB, ns - c0);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int wm = 32 * (wave & 1), wn = 32 * (wave >> 1);
+  if (r0 + wm >= m || wn >= cw) return;
+  gdouble *C = (gdouble *)(a.M + blockIdx.y * a.sM + d.M);
+  gcdouble *Q = (gcdouble *)(a.Q + blockIdx.y * a.sQ + d.Q + (long)k0 * m);
+  Frag acc;
+  clear(acc);
+  long ra[2], rb[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    ra[i] = min(r0 + wm + 16 * i + lr, m - 1);
+    rb[i] = c0 + min(wn + 16 * i + lr, cw - 1);
+  }
+  mma32(acc, n, [&](int i, int kk) { return Q[ra[i] + (long)kk * m]; },
+        [&](int i, int kk) { return Q[rb[i] + (long)kk * m]; });
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int r = r0 + wm + 16 * i + lr;
+    if (r >= m) continue;
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int c = wn + 16 * j + 4 * e + lk;
+        if (c >= cw) continue;
+        gdouble *p = C + r + (long)(c0 + c) * m;
+        *p = tj == a.k ? -acc.c[i][j][e] : *p - acc.c[i][j][e];
+      }
+  }
+}
+
+// Schur complements: S = children's S - L21 L21^T, lower tiles
+__global__ __launch_bounds__(256) void nd_schur_kernel(LevelArgs a) {
+  const int nt = a.tr * (a.tr + 1) / 2;
+  const int f = blockIdx.x / nt, t = blockIdx.x - f * nt;
+  int ti = (int)((sqrtf(8.0f * t + 1.0f) - 1.0f) * 0.5f);
+  while ((ti + 1) * (ti + 2) / 2 <= t) ti++;
+  while (ti * (ti + 1) / 2 > t) ti--;
+  const int tj = t - ti * (ti + 1) / 2;
+  const NdDev d = a.fronts[f];
+  const int ns = d.ns, m = d.m, nb = m - ns;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int r0 = kB * ti + 32 * (wave & 1), c0 = kB * tj + 32 * (wave >> 1);
+  if (r0 >= nb || c0 >= nb || r0 + 32 <= c0) return;
+  gcdouble *Q = (gcdouble *)(a.Q + blockIdx.y * a.sQ + d.Q + ns);
+  gdouble *S = (gdouble *)(a.S + blockIdx.y * a.sS + d.S);
+  Frag acc;
+  clear(acc);
+  long ra[2], rb[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    ra[i] = min(r0 + 16 * i + lr, nb - 1);
+    rb[i] = min(c0 + 16 * i + lr, nb - 1);
+  }
+  mma32(acc, ns, [&](int i, int kk) { return Q[ra[i] + (long)kk * m]; },
+        [&](int i, int kk) { return Q[rb[i] + (long)kk * m]; });
+  const int mn = m / 6;
+  const int *lists = a.lists + d.lists;
+  gcdouble *Sc[2];
+  int ldc[2];
+#pragma unroll
+  for (int c = 0; c < 2; c++)
+    if (d.child[c] >= 0) {
+      const NdDev ch = a.all[d.child[c]];
+      ldc[c] = ch.m - ch.ns;
+      Sc[c] = (gcdouble *)(a.Sc + blockIdx.y * a.sSc + ch.S);
+    }
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int r = r0 + 16 * i + lr;
+    if (r >= nb) continue;
+    const int rn = (ns + r) / 6, rr = r % 6;  // ns is a multiple of 6
+    int ir[2] = {-1, -1};
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+      if (d.child[c] >= 0) ir[c] = lists[(1 + c) * mn + rn];
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int col = c0 + 16 * j + 4 * e + lk;
+        if (col > r) continue;
+        const int cn = (ns + col) / 6, cc = col % 6;
+        double v = 0.0;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+          if (ir[c] < 0) continue;
+          const int ic = lists[(1 + c) * mn + cn];
+          if (ic >= 0) v += Sc[c][6 * ir[c] + rr + (long)(6 * ic + cc) * ldc[c]];
+        }
+        S[r + (long)col * nb] = v - acc.c[i][j][e];
+      }
+  }
+}
+
+struct SolveArgs {
+  const NdDev *fronts, *all;
+  const int *lists;
+  const double *M;
+  double *V;
+  const double *b;
+  double *x;
+  long sM, sV, n;
+  int nd;          // designs: entry e is vector e / nd of design e % nd
+  const int *act;  // entries, or null
+  int tiles;       // per front
+};
+
+constexpr int kStage = 1024;  // vector entries staged at once
+
+// upward sweep: y = X v_J and u_B = v_B - W v_J, 128 rows per workgroup (two
+// per lane), the columns split over the NW wavefronts
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void nd_up_kernel(SolveArgs a) {
+  __shared__ double vj[kStage];
+  __shared__ v2d red[NW][64];
+  const int f = blockIdx.x / a.tiles, r0 = 128 * (blockIdx.x - f * a.tiles);
+  const NdDev d = a.fronts[f];
+  if (r0 >= d.m) return;
+  const int e = a.act ? a.act[blockIdx.y] : blockIdx.y, des = e % a.nd;
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, mn = d.m / 6;
+  const int *lists = a.lists + d.lists;
+  double *V = a.V + e * a.sV;
+  const double *b = a.b + e * a.n;
+  const double *u[2] = {nullptr, nullptr};
+#pragma unroll
+  for (int c = 0; c < 2; c++)
+    if (d.child[c] >= 0) {
+      const NdDev ch = a.all[d.child[c]];
+      u[c] = V + ch.V + ch.ns;
+    }
+  // entry i of the front's vector from the children
+  auto from_children = [&](int i) {
+    const int q = i / 6, w = i - 6 * q;
+    double s = 0.0;
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+      if (u[c]) {
+        const int p = lists[(1 + c) * mn + q];
+        if (p >= 0) s += u[c][6 * p + w];
+      }
+    return s;
+  };
+  const int cend = min(d.ns, r0 + 128);
+  const int row = min(r0 + 2 * lane, d.m - 2);
+  gcdouble *M = (gcdouble *)(a.M + des * a.sM + d.M + row);
+  v2d acc = {0.0, 0.0};
+  for (int s0 = 0; s0 < cend; s0 += kStage) {
+    const int sn = min(kStage, cend - s0);
+    if (s0) __syncthreads();
+    for (int i = t; i < sn; i += 64 * NW) {
+      const int q = (s0 + i) / 6, w = s0 + i - 6 * q;
+      vj[i] = b[6L * lists[q] + w] + from_children(s0 + i);
+    }
+    __syncthreads();
+#pragma unroll 8
+    for (int j = wave; j < sn; j += NW) {
+      const v2d c = *(__attribute__((address_space(1))) const v2d *)(M + (long)(s0 + j) * d.m);
+      acc += c * vj[j];
+    }
+  }
+  red[wave][lane] = acc;
+  __syncthreads();
+  if (wave) return;
+#pragma unroll
+  for (int w = 1; w < NW; w++) acc += red[w][lane];
+  const int r = r0 + 2 * lane;
+  if (r >= d.m) return;
+  if (r >= d.ns) {
+    acc.x += from_children(r);
+    acc.y += from_children(r + 1);
+  }
+  V[d.V + r] = acc.x;
+  V[d.V + r + 1] = acc.y;
+}
+
+// downward sweep: x_J = M^T [y ; x_B], CW columns per wavefront and pass,
+// lanes along the rows (two per lane)
+template <int CW>
+__global__ __launch_bounds__(256) void nd_down_kernel(SolveArgs a) {
+  __shared__ double z[2 * kStage];
+  const int f = blockIdx.x / a.tiles, c0 = 4 * CW * (blockIdx.x - f * a.tiles);
+  const NdDev d = a.fronts[f];
+  if (c0 >= d.ns) return;
+  const int e = a.act ? a.act[blockIdx.y] : blockIdx.y, des = e % a.nd;
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  const int *lists = a.lists + d.lists;
+  const double *V = a.V + e * a.sV + d.V;
+  double *x = a.x + e * a.n;
+  const int cw = c0 + CW * wave;
+  gcdouble *M = (gcdouble *)(a.M + des * a.sM + d.M);
+  v2d acc[CW];
+#pragma unroll
+  for (int c = 0; c < CW; c++) acc[c] = v2d{0.0, 0.0};
+  const int s1 = c0 & ~1;  // rows before the first column are zero
+  for (int s0 = s1; s0 < d.m; s0 += 2 * kStage) {
+    const int sn = min(2 * kStage, d.m - s0);
+    if (s0 != s1) __syncthreads();
+    for (int i = t; i < sn; i += 256) {
+      const int r = s0 + i, q = r / 6;
+      z[i] = r < d.ns ? V[r] : x[6L * lists[q] + r - 6 * q];
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int i = 2 * lane; i < sn; i += 128) {
+      const v2d zz = {z[i], z[i + 1]};
+#pragma unroll
+      for (int c = 0; c < CW; c++) {
+        const int col = min(cw + c, d.ns - 1);
+        acc[c] += *(__attribute__((address_space(1))) const v2d *)(M + s0 + i + (long)col * d.m) * zz;
+      }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < CW; c++) {
+    double s = acc[c].x + acc[c].y;
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) s += __shfl_xor(s, w, 64);
+    const int col = cw + c;
+    if (lane == c && col < d.ns) {
+      const int q = col / 6;
+      x[6L * lists[q] + col - 6 * q] = s;
+    }
+  }
+}
+
+template <typename T>
+hipError_t upload(T **dst, const std::vector<T> &src) {
+  hipError_t e = hipMalloc((void **)dst, sizeof(T) * std::max<size_t>(1, src.size()));
+  if (e == hipSuccess && !src.empty()) e = hipMemcpy(*dst, src.data(), sizeof(T) * src.size(), hipMemcpyHostToDevice);
+  return e;
+}
+
+}  // namespace
+
+std::string nd_create(int nn, const std::vector<int> &rowp, const std::vector<int> &cols, const double *X, int nbatch,
+                      int nrhs, NdFactor &F, std::vector<long> &blk_base, std::vector<int> &blk_ld) {
+  NdLayout L = nd_layout(nn, rowp, cols, X, kLeafNodes);
+  F.nbatch = nbatch;
+  F.levels = std::move(L.levels);
+  F.per_design = L.per_design;
+  F.v_len = L.v_len;
+  F.q_len = L.q_len;
+  F.s_len[0] = L.s_len[0];
+  F.s_len[1] = L.s_len[1];
+  blk_base = std::move(L.blk_base);
+  blk_ld = std::move(L.blk_ld);
+  // workspace copies: as many designs at once as 4 GiB hold (16 designs of
+  // the 100 x 200 cylinder), which leaves no level short of workgroups
+  const double ws = 8.0 * (F.q_len + F.s_len[0] + F.s_len[1]);
+  F.chunk = std::max(1, (int)std::min<double>(nbatch, 4294967296.0 / ws));
+  F.rhs_cap = std::max(1, nrhs);
+  hipError_t e = upload(&F.d_fronts, L.fronts);
+  if (e == hipSuccess) e = upload(&F.d_lists, L.lists);
+  if (e == hipSuccess) e = hipMalloc((void **)&F.M, sizeof(double) * (size_t)F.per_design * nbatch);
+  if (e == hipSuccess) e = hipMalloc((void **)&F.Q, sizeof(double) * (size_t)F.q_len * F.chunk);
+  for (int k = 0; k < 2 && e == hipSuccess; k++)
+    e = hipMalloc((void **)&F.S[k], sizeof(double) * (size_t)F.s_len[k] * F.chunk);
+  if (e == hipSuccess) e = hipMalloc((void **)&F.V, sizeof(double) * (size_t)F.v_len * nbatch * F.rhs_cap);
+  if (e != hipSuccess)
+    return std::string("factor allocation (") + std::to_string((long)(8.0 * F.per_design * nbatch) >> 20) +
+           " MiB): " + hipGetErrorString(e);
+  return "";
+}
+
+void nd_destroy(NdFactor &F) {
+  void *bufs[] = {F.d_fronts, F.d_lists, F.M, F.Q, F.S[0], F.S[1], F.V};
+  for (void *p : bufs)
+    if (p) (void)hipFree(p);
+  F = NdFactor();
+}
+
+hipError_t nd_reserve(NdFactor &F, int nrhs) {
+  if (nrhs <= F.rhs_cap) return hipSuccess;
+  hipError_t e = hipFree(F.V);
+  F.V = nullptr;
+  F.rhs_cap = 0;
+  if (e == hipSuccess) e = hipMalloc((void **)&F.V, sizeof(double) * (size_t)F.v_len * F.nbatch * nrhs);
+  if (e == hipSuccess) F.rhs_cap = nrhs;
+  return e;
+}
+
+hipError_t nd_compute(NdFactor &F, int nnzb, const double *vals, const long *blk_base, const int *blk_ld,
+                      const int *blk_flag, int *info, hipStream_t stream) {
+  hipError_t e = hipMemsetAsync(F.M, 0, sizeof(double) * (size_t)F.per_design * F.nbatch, stream);
+  if (e == hipSuccess) e = hipMemsetAsync(info, 0, sizeof(int) * F.nbatch, stream);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(nd_scatter_kernel, dim3((unsigned)((36L * nnzb + 255) / 256), F.nbatch), dim3(256), 0, stream,
+                     nnzb, vals, 36L * nnzb, blk_base, blk_ld, blk_flag, F.M, F.per_design);
+  for (int d0 = 0; d0 < F.nbatch; d0 += F.chunk) {
+    const unsigned nd = (unsigned)std::min(F.chunk, F.nbatch - d0);
+    for (size_t l = 0; l < F.levels.size(); l++) {
+      const NdLevel &lv = F.levels[l];
+      LevelArgs a;
+      a.all = F.d_fronts;
+      a.fronts = F.d_fronts + lv.f0;
+      a.lists = F.d_lists;
+      a.M = F.M + (size_t)d0 * F.per_design;
+      a.Q = F.Q;
+      a.S = F.S[l & 1];
+      a.Sc = F.S[(l & 1) ^ 1];
+      a.sM = F.per_design;
+      a.sQ = F.q_len;
+      a.sS = F.s_len[l & 1];
+      a.sSc = F.s_len[(l & 1) ^ 1];
+      const int tm = (lv.max_m + kB - 1) / kB, tn = (lv.max_ns + kB - 1) / kB;
+      if (lv.inner) {
+        a.tr = tm;
+        a.tc = tn;
+        hipLaunchKernelGGL(nd_gather_kernel, dim3((unsigned)lv.nf * tm * tn, nd), dim3(256), 0, stream, a);
+      }
+      for (a.k = 0; a.k < tn; a.k++) {
+        hipLaunchKernelGGL(nd_diag_kernel, dim3(lv.nf, nd), dim3(kDiagThreads), 0, stream, a, info + d0);
+        // rows after block k of the tallest front (a front whose block k is
+        // its last, of n < 64 pivots, has its boundary left)
+        a.tr = std::max((lv.max_m - kB * (a.k + 1) + kB - 1) / kB, (lv.max_nb + kB - 1) / kB);
+        a.tc = tn;
+        if (a.tr + a.k > 0)
+          hipLaunchKernelGGL(nd_scale_kernel, dim3((unsigned)lv.nf * (a.tr + a.k), nd), dim3(256), 0, stream, a);
+        if (a.tr > 0)
+          hipLaunchKernelGGL(nd_update_kernel, dim3((unsigned)lv.nf * a.tr * a.tc, nd), dim3(256), 0, stream, a);
+      }
+      if (lv.max_nb > 0) {
+        a.tr = (lv.max_nb + kB - 1) / kB;
+        hipLaunchKernelGGL(nd_schur_kernel, dim3((unsigned)lv.nf * (a.tr * (a.tr + 1) / 2), nd), dim3(256), 0, stream,
+                           a);
+      }
+    }
+  }
+  return hipGetLastError();
+}
+
+hipError_t nd_solve(const NdFactor &F, const double *b, double *x, long n, int nrhs, const int *act, int nact,
+                    hipStream_t stream) {
+  SolveArgs a;
+  a.all = F.d_fronts;
+  a.lists = F.d_lists;
+  a.M = F.M;
+  a.V = F.V;
+  a.b = b;
+  a.x = x;
+  a.sM = F.per_design;
+  a.sV = F.v_len;
+  a.n = n;
+  a.nd = F.nbatch;
+  a.act = act;
+  const unsigned ne = (unsigned)(act ? nact : F.nbatch * nrhs);
+  for (const NdLevel &lv : F.levels) {
+    a.fronts = F.d_fronts + lv.f0;
+    a.tiles = (lv.max_m + 127) / 128;
+    const long groups = (long)lv.nf * a.tiles * ne;
+    // few row tiles (the fronts near the root): more wavefronts share a
+    // tile's columns, so that enough loads are in flight
+    if (groups < 1024)
+      hipLaunchKernelGGL(nd_up_kernel<16>, dim3((unsigned)(lv.nf * a.tiles), ne), dim3(1024), 0, stream, a);
+    else
+      hipLaunchKernelGGL(nd_up_kernel<4>, dim3((unsigned)(lv.nf * a.tiles), ne), dim3(256), 0, stream, a);
+  }
+  for (size_t l = F.levels.size(); l-- > 0;) {
+    const NdLevel &lv = F.levels[l];
+    a.fronts = F.d_fronts + lv.f0;
+    const long cols = (long)lv.nf * lv.max_ns * ne;
+    if (cols >= 32768) {
+      a.tiles = (lv.max_ns + 31) / 32;
+      hipLaunchKernelGGL(nd_down_kernel<8>, dim3((unsigned)(lv.nf * a.tiles), ne), dim3(256), 0, stream, a);
+    } else {
+      a.tiles = (lv.max_ns + 15) / 16;
+      hipLaunchKernelGGL(nd_down_kernel<4>, dim3((unsigned)(lv.nf * a.tiles), ne), dim3(256), 0, stream, a);
+    }
+  }
+  return hipGetLastError();
+}
+
+}  // namespace shellgpu

@@ -1,0 +1,240 @@
+// nd_order.h -- nested-dissection order of a mesh graph and the symbolic
+// structure of its multifrontal Cholesky factor (host code, no device calls).
+//
+// A node set is cut by a vertex separator found along one of four sweeps of
+// the set: the three coordinates (shell meshes are surfaces, so a plane cuts
+// them in short lines) and the breadth-first distance from a far node (which
+// needs no coordinates).  For a sweep the separator of every cut position
+// comes from two prefix sums over the edges, so all positions between 30 and
+// 70 per cent of the set are compared, not only the median.  The two sides
+// are cut again down to leaves of at most `leaf` nodes; a leaf and every
+// separator is one front.
+#pragma once
+
+#include <algorithm>
+#include <cmath>
+#include <utility>
+#include <vector>
+
+namespace shellgpu {
+
+struct NdFront {
+  int j0 = 0;      // first pivot node (elimination position)
+  int ns = 0;      // pivot nodes
+  int parent = -1;
+  int child[2] = {-1, -1};
+  int depth = 0;            // distance from the root
+  std::vector<int> bnd;     // boundary nodes: elimination positions, ascending
+};
+
+struct NdTree {
+  std::vector<int> perm;       // elimination position -> node
+  std::vector<int> pos;        // node -> elimination position
+  std::vector<NdFront> fronts; // children before parents
+  int ndepth = 0;
+};
+
+class NdBuilder {
+ public:
+  NdBuilder(int nn, const int *rowp, const int *cols, const double *X, int leaf)
+      : nn_(nn), rowp_(rowp), cols_(cols), leaf_(leaf), where_(nn, -1), rank_(nn), dist_(nn), side_(nn) {
+    // the whole mesh along each coordinate; the sets below keep these orders
+    // (a stable partition), so nothing is sorted again
+    for (int d = 0; d < 3; d++) {
+      std::vector<std::pair<double, int>> key(nn);
+      for (int i = 0; i < nn; i++) key[i] = {X[3 * i + d], i};
+      std::sort(key.begin(), key.end());
+      all_.along[d].resize(nn);
+      for (int i = 0; i < nn; i++) all_.along[d][i] = key[i].second;
+    }
+  }
+
+  NdTree build() {
+    t_.perm.clear();
+    t_.pos.assign(nn_, -1);
+    cut(all_, 0);
+    for (int p = 0; p < nn_; p++) t_.pos[t_.perm[p]] = p;
+    symbolic();
+    return std::move(t_);
+  }
+
+ private:
+  struct Set {
+    std::vector<int> along[3];  // the same nodes along the three coordinates
+  };
+  struct Cut {
+    double cost = -1.0;
+    bool right = false;  // the separator is taken from the nodes after the cut
+    int at = 0, sweep = -1;
+  };
+
+  int nn_;
+  const int *rowp_, *cols_;
+  int leaf_;
+  // by node: stamp of its set, rank in the sweep, BFS distance, side of the cut
+  std::vector<int> where_, rank_, dist_;
+  std::vector<signed char> side_;
+  std::vector<int> left_, right_;
+  int stamp_ = 0;
+  Set all_;
+  NdTree t_;
+
+  // best cut of the current set (where_[] == stamp_) along an order
+  void sweep(const std::vector<int> &order, int which, Cut &best) {
+    const int n = (int)order.size();
+    for (int k = 0; k < n; k++) rank_[order[k]] = k;
+    left_.assign(n + 2, 0);
+    right_.assign(n + 2, 0);
+    for (int k = 0; k < n; k++) {
+      const int v = order[k];
+      int lo = k, hi = k;
+      for (int p = rowp_[v]; p < rowp_[v + 1]; p++) {
+        const int w = cols_[p];
+        if (where_[w] != stamp_) continue;
+        lo = std::min(lo, rank_[w]);
+        hi = std::max(hi, rank_[w]);
+      }
+      // v is in the separator of cut c when it lies before (after) the cut
+      // and has a neighbour after (before) it: k < c <= hi, lo < c <= k
+      left_[k + 1]++;
+      left_[hi + 1]--;
+      right_[lo + 1]++;
+      right_[k + 1]--;
+    }
+    const int c0 = std::max(1, (3 * n) / 10), c1 = std::min(n - 1, n - (3 * n) / 10);
+    int l = 0, r = 0;
+    for (int c = 1; c <= c1; c++) {
+      l += left_[c];
+      r += right_[c];
+      if (c < c0) continue;
+      const double b = 2.0 * c / n - 1.0, pen = 1.0 + 2.0 * b * b;
+      for (int side = 0; side < 2; side++) {
+        const double cost = (side ? r : l) * pen;
+        if (best.cost < 0.0 || cost < best.cost) best = {cost, side == 1, c, which};
+      }
+    }
+  }
+
+  // cut the set; returns its front (children first), or -1 for an empty set
+  int cut(Set &set, int depth) {
+    const int n = (int)set.along[0].size();
+    if (n == 0) return -1;
+    if (n <= leaf_) return front(set.along[0], -1, -1, depth);
+    stamp_++;
+    for (int v : set.along[0]) where_[v] = stamp_;
+    Cut best;
+    for (int d = 0; d < 3; d++) sweep(set.along[d], d, best);
+    // breadth-first sweep where planes do not find the short lines of a
+    // surface (coordinates that coincide or fold)
+    std::vector<int> order;
+    if (best.cost > 3.0 * std::sqrt((double)n)) {
+      bfs(set.along[0], order);
+      sweep(order, 3, best);
+    }
+    const std::vector<int> &along = best.sweep == 3 ? order : set.along[best.sweep];
+    for (int k = 0; k < n; k++) side_[along[k]] = k >= best.at;
+    // the separator: nodes of one side with a neighbour on the other
+    std::vector<int> s;
+    for (int k = 0; k < n; k++) {
+      const int v = along[k];
+      if ((k >= best.at) != best.right) continue;
+      for (int p = rowp_[v]; p < rowp_[v + 1]; p++) {
+        const int w = cols_[p];
+        if (where_[w] == stamp_ && (side_[w] & 1) != (int)best.right) {
+          s.push_back(v);
+          break;
+        }
+      }
+    }
+    // disconnected sides: any node keeps the tree binary
+    if (s.empty()) s.push_back(along[best.right ? n - 1 : 0]);
+    for (int v : s) side_[v] = 2 + (side_[v] & 1);
+    int id[2] = {-1, -1};
+    Set part[2];
+    for (int d = 0; d < 3; d++) {
+      for (int k = 0; k < 2; k++) part[k].along[d].reserve(n / 2 + 1);
+      for (int v : set.along[d])
+        if (side_[v] < 2) part[(int)side_[v]].along[d].push_back(v);
+      std::vector<int>().swap(set.along[d]);
+    }
+    std::vector<int>().swap(order);
+    for (int k = 0; k < 2; k++) id[k] = cut(part[k], depth + 1);
+    return front(s, id[0], id[1], depth);
+  }
+
+  // the set in breadth-first order from a far node (components one after another)
+  void bfs(const std::vector<int> &set, std::vector<int> &order) {
+    int start = set[0];
+    for (int it = 0; it < 3; it++) {
+      for (int v : set) dist_[v] = -1;
+      order.clear();
+      size_t next = 0;
+      int root = start;
+      while (order.size() < set.size()) {
+        size_t h = order.size();
+        dist_[root] = 0;
+        order.push_back(root);
+        for (; h < order.size(); h++) {
+          const int v = order[h];
+          for (int p = rowp_[v]; p < rowp_[v + 1]; p++) {
+            const int w = cols_[p];
+            if (where_[w] == stamp_ && dist_[w] < 0) {
+              dist_[w] = dist_[v] + 1;
+              order.push_back(w);
+            }
+          }
+        }
+        while (next < set.size() && dist_[set[next]] >= 0) next++;
+        if (next < set.size()) root = set[next];
+      }
+      start = order.back();
+    }
+  }
+
+  int front(const std::vector<int> &nodes, int ca, int cb, int depth) {
+    NdFront f;
+    f.j0 = (int)t_.perm.size();
+    f.ns = (int)nodes.size();
+    f.depth = depth;
+    if (ca < 0) std::swap(ca, cb);
+    f.child[0] = ca;
+    f.child[1] = cb;
+    for (int v : nodes) t_.perm.push_back(v);
+    const int id = (int)t_.fronts.size();
+    if (ca >= 0) t_.fronts[ca].parent = id;
+    if (cb >= 0) t_.fronts[cb].parent = id;
+    t_.fronts.push_back(f);
+    t_.ndepth = std::max(t_.ndepth, depth + 1);
+    return id;
+  }
+
+  // boundary of a front: later neighbours of its pivots and of its children's
+  // boundaries
+  void symbolic() {
+    std::vector<int> mark(nn_, -1);
+    for (size_t s = 0; s < t_.fronts.size(); s++) {
+      NdFront &f = t_.fronts[s];
+      const int end = f.j0 + f.ns;
+      for (int j = f.j0; j < end; j++) {
+        const int v = t_.perm[j];
+        for (int p = rowp_[v]; p < rowp_[v + 1]; p++) {
+          const int q = t_.pos[cols_[p]];
+          if (q >= end && mark[q] != (int)s) {
+            mark[q] = (int)s;
+            f.bnd.push_back(q);
+          }
+        }
+      }
+      for (int c : f.child)
+        if (c >= 0)
+          for (int q : t_.fronts[c].bnd)
+            if (q >= end && mark[q] != (int)s) {
+              mark[q] = (int)s;
+              f.bnd.push_back(q);
+            }
+      std::sort(f.bnd.begin(), f.bnd.end());
+    }
+  }
+};
+
+}  // namespace shellgpu

@@ -2,8 +2,10 @@
 //
 // Direct solver.  The reference factors K and K + sigma G with an
 // AMD-ordered complete block LU on the CPU (TACSSchurPc with levFill = 1e6,
-// src/bpmat/TACSSchurMat.cpp:944-1652).  Here the nodes are ordered by
-// breadth-first level sets from a seed set (a whole end ring of the
+// src/bpmat/TACSSchurMat.cpp:944-1652).  Here the default is a multifrontal
+// Cholesky factor under a nested-dissection order (nd_factor.hip).  Two
+// level forms remain behind SHELLGPU_FACTOR=thomas and =cr: the nodes are
+// ordered by breadth-first level sets from a seed set (a whole end ring of the
 // cylinder, or a pseudo-peripheral node), which makes every shell mesh
 // block-tridiagonal in level blocks: a node couples only to nodes of its own
 // and the neighbouring levels.  Boundary conditions are eliminated
@@ -35,7 +37,7 @@
 // Block cyclic reduction (below) for a few designs of long level chains.
 //
 // A failed Cholesky (non-positive pivot) reports a shift above the first
-// eigenvalue.  The solve is exact for right-hand sides that vanish on BC
+// eigenvalue, in every form.  The solve is exact for right-hand sides that vanish on BC
 // dofs (all solves of the buckling path); GMRES corrects the remainder.
 //
 // GMRES.  Right-preconditioned restarted GMRES with Givens rotations
@@ -62,6 +64,7 @@
 #include <string>
 #include <vector>
 
+#include "nd_factor.h"
 #include "shellgpu.h"
 #include "shellgpu_ctx.h"
 
@@ -141,6 +144,9 @@ struct shellgpu_factor {
   double *crm_b = nullptr, *crm_z = nullptr, *crm_x = nullptr, *crm_part = nullptr;
   int *d_crm_act = nullptr;
   bool factored = false;
+  // nested-dissection multifrontal form (nd_factor.hip): the default
+  bool nd = false;
+  NdFactor ndf;
   long nv = 0;               // level-ordered vector length per design
   // block cyclic reduction over uniform (padded) levels of M dofs: per
   // design, blocks D_i (-> C_i^{-1}), B_i (coupling to the left active
@@ -174,6 +180,8 @@ struct shellgpu_factor {
 };
 
 namespace {
+
+constexpr int kMaxRhs = 16;  // vectors per design of one solve
 
 int ferr(shellgpu_ctx *ctx, int code, const std::string &msg) {
   if (ctx) ctx->err = msg;
@@ -1053,6 +1061,50 @@ int setup_plan(shellgpu_factor *F) {
     F->maxm = std::max(F->maxm, F->m[l]);
   }
 
+  // BC dofs (symmetric elimination)
+  std::vector<int> isbc(F->n, 0);
+  for (size_t b = 0; b < ctx->h_bc_nodes.size(); b++)
+    for (int r = 0; r < 6; r++)
+      if (ctx->h_bc_mask[b] & (1 << r)) isbc[6 * ctx->h_bc_nodes[b] + r] = 1;
+  // per BSR block: BC rows (bit r), BC columns (bit 6 + c), diagonal (bit 12)
+  auto block_flag = [&](int i, int j) {
+    int mask = 0;
+    for (int d = 0; d < 6; d++) mask |= (isbc[6 * i + d] << d) | (isbc[6 * j + d] << (6 + d));
+    return i == j ? mask | 1 << 12 : mask;
+  };
+
+  // The nested-dissection form (nd_factor.hip) for every mesh and batch; the
+  // level forms below only where SHELLGPU_FACTOR asks for one of them.
+  // Factor and solve of one design, this form against the faster level form:
+  // 200 x 400 cylinder 24 and 0.67 ms against 340 and 4.3 ms (cyclic
+  // reduction), 16 designs of 61 x 119 15 against 110 ms, of 100 x 200 2.4
+  // against 4.0 ms per solve (sequential), and the whole analysis of a 20 x
+  // 40 cylinder 17 against 25 ms: no size was found where a level form wins.
+  {
+    const char *env = getenv("SHELLGPU_FACTOR");
+    F->nd = !(env && (strcmp(env, "thomas") == 0 || strcmp(env, "cr") == 0));
+  }
+  if (F->nd) {
+    std::vector<double> X(3 * (size_t)nn);
+    HIPCALL(ctx, hipMemcpyAsync(X.data(), ctx->d_X, sizeof(double) * X.size(), hipMemcpyDeviceToHost, ctx->stream));
+    HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
+    std::vector<long> base;
+    std::vector<int> ld, flag(ctx->nnzb);
+    const std::string err =
+        nd_create(nn, rowp, cols, X.data(), F->nbatch, F->nbatch == 1 ? std::min(kMaxRhs, ctx->nbatch) : 1, F->ndf, base, ld);
+    if (!err.empty()) return ferr(ctx, 2, err);
+    F->per_design = F->ndf.per_design;
+    for (int i = 0; i < nn; i++)
+      for (int p = rowp[i]; p < rowp[i + 1]; p++) flag[p] = block_flag(i, cols[p]);
+    HIPCALL(ctx, hipMalloc((void **)&F->d_bcflag, sizeof(int) * ctx->nnzb));
+    HIPCALL(ctx, hipMalloc((void **)&F->d_blk_base, sizeof(long) * ctx->nnzb));
+    HIPCALL(ctx, hipMalloc((void **)&F->d_blk_ld, sizeof(int) * ctx->nnzb));
+    HIPCALL(ctx, hipMemcpy(F->d_bcflag, flag.data(), sizeof(int) * ctx->nnzb, hipMemcpyHostToDevice));
+    HIPCALL(ctx, hipMemcpy(F->d_blk_base, base.data(), sizeof(long) * ctx->nnzb, hipMemcpyHostToDevice));
+    HIPCALL(ctx, hipMemcpy(F->d_blk_ld, ld.data(), sizeof(int) * ctx->nnzb, hipMemcpyHostToDevice));
+    return 0;
+  }
+
   // Block cyclic reduction when the padded factor (three M x M blocks per
   // level and design) fits in 85 % of the free device memory, padding the
   // levels to M adds at most half the unknowns, and the factor holds few
@@ -1187,12 +1239,6 @@ int setup_plan(shellgpu_factor *F) {
     }
   }
 
-  // BC dofs (symmetric elimination)
-  std::vector<int> isbc(F->n, 0);
-  for (size_t b = 0; b < ctx->h_bc_nodes.size(); b++)
-    for (int r = 0; r < 6; r++)
-      if (ctx->h_bc_mask[b] & (1 << r)) isbc[6 * ctx->h_bc_nodes[b] + r] = 1;
-
   // dof permutation (level order, padded to M per level under cyclic
   // reduction) and block scatter map
   std::vector<int> pos2dof(F->nv, -1);
@@ -1210,10 +1256,7 @@ int setup_plan(shellgpu_factor *F) {
     for (int p = rowp[i]; p < rowp[i + 1]; p++) {
       const int j = cols[p], lj = level[j];
       const long cl = 6L * (node_pos[j] - noff[lj]);
-      int mask = 0;
-      for (int d = 0; d < 6; d++) mask |= (isbc[6 * i + d] << d) | (isbc[6 * j + d] << (6 + d));
-      if (i == j) mask |= 1 << 12;
-      colbc[p] = mask;
+      colbc[p] = block_flag(i, j);
       ld[p] = F->cr ? F->M : F->m[li];
       if (lj == li) {
         base[p] = F->cr ? (long)li * M2 + cl * F->M + rl : F->S_off[li] + cl * F->m[li] + rl;
@@ -1467,10 +1510,19 @@ int factor_create(shellgpu_ctx *ctx, int nbatch, shellgpu_factor **out) {
   F->ctx = ctx;
   F->nbatch = nbatch;
   if ((rc = setup_plan(F))) {
-    delete F;
+    shellgpu_factor_destroy(F);
     return rc;
   }
   const int nb = F->nbatch;
+  if (F->nd) {
+    if (hipMalloc((void **)&F->info, sizeof(int) * nb) != hipSuccess ||
+        hipMalloc((void **)&F->d_act, sizeof(int) * nb) != hipSuccess) {
+      shellgpu_factor_destroy(F);
+      return ferr(ctx, 2, "out of device memory (factor)");
+    }
+    *out = F;
+    return 0;
+  }
   const size_t bytes = sizeof(double) * (size_t)F->per_design * nb;
   hipError_t e = hipMalloc((void **)&F->buf, bytes);
   if (e == hipSuccess && !F->cr)
@@ -1525,6 +1577,7 @@ void shellgpu_factor_destroy(shellgpu_factor *F) {
                   F->crm_z,    F->crm_x,     F->crm_part,  F->d_crm_act};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
+  nd_destroy(F->ndf);
   delete F;
 }
 
@@ -1550,6 +1603,21 @@ int shellgpu_factor_compute(shellgpu_factor *F, shellgpu_mat *A) {
   const int nb = F->nbatch;
   const long ps = F->per_design;
   F->factored = false;
+  auto not_spd = [&](int b) {
+    return ferr(ctx, 5, "matrix not positive definite in the level Cholesky (design " + std::to_string(b) +
+                            "): for K + sigma G the shift is above the first buckling load");
+  };
+  if (F->nd) {
+    HIPCALL(ctx, nd_compute(F->ndf, ctx->nnzb, A->vals, F->d_blk_base, F->d_blk_ld, F->d_bcflag, F->info,
+                            ctx->stream));
+    std::vector<int> info(nb);
+    HIPCALL(ctx, hipMemcpyAsync(info.data(), F->info, sizeof(int) * nb, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
+    for (int b = 0; b < nb; b++)
+      if (info[b] != 0) return not_spd(b);
+    F->factored = true;
+    return 0;
+  }
   HIPCALL(ctx, hipMemsetAsync(F->buf, 0, sizeof(double) * (size_t)ps * nb, ctx->stream));
   {
     const long nthreads = 36L * ctx->nnzb;
@@ -1567,9 +1635,7 @@ int shellgpu_factor_compute(shellgpu_factor *F, shellgpu_mat *A) {
     if (all[q] != 0) info[q % nb] = 1;
   HIPCALL(ctx, hipMemcpy(F->info, info.data(), sizeof(int) * nb, hipMemcpyHostToDevice));
   for (int b = 0; b < nb; b++)
-    if (info[b] != 0)
-      return ferr(ctx, 5, "matrix not positive definite in the level Cholesky (design " + std::to_string(b) +
-                              "): for K + sigma G the shift is above the first buckling load");
+    if (info[b] != 0) return not_spd(b);
   F->factored = true;
   return 0;
 }
@@ -1610,7 +1676,6 @@ static int gemv_batch(shellgpu_factor *F, bool trans, int m, int n, const double
 // level l of the sequential factorisation; vector entries e = r nb + d of
 // stride nv): one vector per design reads half of P, several read it in
 // full once for all (nrhs <= 8 or 16)
-constexpr int kMaxRhs = 16;
 // vectors per pass when a factor of one design solves n vectors: 16 while
 // there are that many (P read once for 16), else up to 8
 inline int rhs_chunk(int n) { return n >= kMaxRhs ? kMaxRhs : std::min(8, n); }
@@ -2173,29 +2238,40 @@ namespace {
 // replayed.  It is opt-in: the solves are bound by the GPU, not by their
 // launches (no wall-time change measured), and rocprofv3's kernel tracing
 // crashes in the capture.
-int solve_body(shellgpu_factor *F) { return F->cr ? apply_cr(F) : apply_schur(F, 1); }
+int solve_body(shellgpu_factor *F) {
+  if (F->nd) {
+    HIPCALL(F->ctx, nd_solve(F->ndf, F->vb, F->vx, F->n, 1, nullptr, 0, F->ctx->stream));
+    return 0;
+  }
+  return F->cr ? apply_cr(F) : apply_schur(F, 1);
+}
+
+// whether single-vector solves go through the captured graph (decided at a
+// factor's first solve)
+bool solve_captured(shellgpu_factor *F) {
+  if (!F->solve_graph && !F->graph_off) {
+    const char *env = getenv("SHELLGPU_GRAPH");
+    F->graph_off = !env || strcmp(env, "1") != 0;
+  }
+  return !F->graph_off;
+}
 
 int run_solve_body(shellgpu_factor *F) {
   shellgpu_ctx *ctx = F->ctx;
-  if (!F->solve_graph && !F->graph_off) {
-    const char *env = getenv("SHELLGPU_GRAPH");
-    if (!env || strcmp(env, "1") != 0) {
-      F->graph_off = true;
-    } else {
-      hipGraph_t g = nullptr;
-      HIPCALL(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-      const int rc = solve_body(F);
-      const hipError_t e = hipStreamEndCapture(ctx->stream, &g);
-      if (rc != 0 || e != hipSuccess) {
-        if (g) (void)hipGraphDestroy(g);
-        return rc ? rc : ferr(ctx, 2, std::string("solve capture: ") + hipGetErrorString(e));
-      }
-      const hipError_t ei = hipGraphInstantiate(&F->solve_graph, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      if (ei != hipSuccess) {
-        F->solve_graph = nullptr;
-        return ferr(ctx, 2, std::string("solve graph: ") + hipGetErrorString(ei));
-      }
+  if (solve_captured(F) && !F->solve_graph) {
+    hipGraph_t g = nullptr;
+    HIPCALL(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+    const int rc = solve_body(F);
+    const hipError_t e = hipStreamEndCapture(ctx->stream, &g);
+    if (rc != 0 || e != hipSuccess) {
+      if (g) (void)hipGraphDestroy(g);
+      return rc ? rc : ferr(ctx, 2, std::string("solve capture: ") + hipGetErrorString(e));
+    }
+    const hipError_t ei = hipGraphInstantiate(&F->solve_graph, g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    if (ei != hipSuccess) {
+      F->solve_graph = nullptr;
+      return ferr(ctx, 2, std::string("solve graph: ") + hipGetErrorString(ei));
     }
   }
   if (F->graph_off) return solve_body(F);
@@ -2213,6 +2289,30 @@ int apply_block(shellgpu_factor *F, const double *b, double *x, int nrhs, bool m
   // to the designs it has not converged yet (the others keep x unchanged)
   const int *act = (!F->cr && nrhs == 1 && F->nact >= 0) ? F->d_act : nullptr;
   if (act && F->nact == 0) return 0;
+  if (F->nd) {
+    if (nrhs > F->ndf.rhs_cap) {
+      if (!may_alloc) return ferr(ctx, 1, "the factor's vector buffers would have to grow");
+      HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
+      if (F->solve_graph) {  // captured on the buffer about to move
+        HIPCALL(ctx, hipGraphExecDestroy(F->solve_graph));
+        F->solve_graph = nullptr;
+      }
+      HIPCALL(ctx, nd_reserve(F->ndf, nrhs));
+    }
+    if (!act && nrhs == 1 && (may_alloc || F->solve_graph) && solve_captured(F)) {
+      // the captured body runs on vectors of its own
+      const size_t bytes = sizeof(double) * (size_t)n * nb;
+      if (!F->vb) HIPCALL(ctx, hipMalloc((void **)&F->vb, bytes));
+      if (!F->vx) HIPCALL(ctx, hipMalloc((void **)&F->vx, bytes));
+      HIPCALL(ctx, hipMemcpyAsync(F->vb, b, bytes, hipMemcpyDeviceToDevice, ctx->stream));
+      const int rc = run_solve_body(F);
+      if (rc) return rc;
+      HIPCALL(ctx, hipMemcpyAsync(x, F->vx, bytes, hipMemcpyDeviceToDevice, ctx->stream));
+      return 0;
+    }
+    HIPCALL(ctx, nd_solve(F->ndf, b, x, n, nrhs, act, F->nact, ctx->stream));
+    return 0;
+  }
   const dim3 pgrid((unsigned)((nv + 255) / 256), act ? F->nact : nb);
   int rc = 0;
   if (F->cr && nb == 1 && nrhs > 1 && (nrhs <= 8 || nrhs == kMaxRhs)) return apply_cr_multi(F, b, x, nrhs, may_alloc);
@@ -2288,7 +2388,7 @@ int factor_noalloc_ready(shellgpu_factor *F) {
   if (!F->factored) return ferr(ctx, 1, "factor not computed");
   if (F->nbatch == ctx->nbatch || F->cr) return 0;
   if (F->nbatch != 1) return ferr(ctx, 1, "factor batch size does not match the context's designs");
-  if (rhs_chunk(ctx->nbatch) > F->rhs_cap)
+  if (rhs_chunk(ctx->nbatch) > (F->nd ? F->ndf.rhs_cap : F->rhs_cap))
     return ferr(ctx, 1, "a factor shared by " + std::to_string(ctx->nbatch) +
                             " designs needs larger vector buffers: apply it once with shellgpu_factor_apply first");
   return 0;

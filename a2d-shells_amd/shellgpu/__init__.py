@@ -265,7 +265,7 @@ class Matrix:
 
 
 class Factor:
-    """Level-set block LU of a batch of matrices (TACSPc)."""
+    """Direct (multifrontal Cholesky) factor of a batch of matrices (TACSPc)."""
 
     def __init__(self, ctx):
         self.ctx = ctx

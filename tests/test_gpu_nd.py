@@ -1,0 +1,203 @@
+"""The multifrontal factor (the default SHELLGPU_FACTOR) on matrices of known
+solution: meshes of one front, fronts shorter and longer than a pivot block,
+last blocks of every remainder, fronts longer than the staged vector pieces,
+batches of designs, several vectors per design, and the captured solve."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import shellgpu as sg
+from shellgpu.problems import BoxBeam, Cylinder
+
+from helpers import random_mesh
+
+pytestmark = pytest.mark.gpu
+
+# diagonally dominant matrices with rows' off-diagonal sums at most 0.9 of
+# the diagonal, equilibrated to about 1: condition number below 40, so the
+# forward error of a backward stable solve is below ~ 40 eps times a modest
+# factor (100 here) of the depth of the sums
+TOL = 40 * 100 * 2.3e-16
+
+
+def spd_values(rowp, cols, seed):
+    """Symmetric diagonally dominant block values on a node pattern."""
+    rng = np.random.default_rng(seed)
+    n = len(rowp) - 1
+    rows = np.repeat(np.arange(n), np.diff(rowp))
+    v = rng.standard_normal((len(cols), 6, 6))
+    t = np.lexsort((rows, cols))  # position of the transposed block
+    up = rows < cols
+    v[up] = v[t[up]].transpose(0, 2, 1)
+    d = np.where(rows == cols)[0]
+    v[d] = v[d] + v[d].transpose(0, 2, 1)
+    off = np.zeros((n, 6))
+    np.add.at(off, rows, np.abs(v).sum(2))
+    i = np.arange(6)
+    v[d[:, None], i, i] = 0.0
+    off = np.zeros((n, 6))
+    np.add.at(off, rows, np.abs(v).sum(2))
+    v[d[:, None], i, i] = off / 0.9
+    return v / off.mean()
+
+
+def make(mesh, nb, bcs=True):
+    ctx = sg.Context(0)
+    ctx.set_mesh(mesh[0], mesh[1])
+    ctx.set_material(70e9, 0.3)
+    if bcs:
+        ctx.set_bcs(np.arange(0, len(mesh[1]), 7), np.arange(0, len(mesh[1]), 7) % 63 + 1)
+    ctx.set_designs(np.full((nb, len(mesh[0])), 0.002))
+    return ctx
+
+
+def bc_mask(nn):
+    m = np.zeros((nn, 6), bool)
+    nodes = np.arange(0, nn, 7)
+    for k in range(6):
+        m[nodes, k] = ((nodes % 63 + 1) >> k) & 1 == 1
+    return m.ravel()
+
+
+def system(ctx, nb, bcs, seed):
+    """Values of nb designs, and right-hand sides b of known x."""
+    rowp, cols = ctx.pattern()
+    nn = len(rowp) - 1
+    vals = np.stack([spd_values(rowp, cols, seed + d) for d in range(nb)])
+    x = np.random.default_rng(seed + 99).standard_normal((nb, 6 * nn))
+    b = np.empty_like(x)
+    for d in range(nb):
+        A = sp.bsr_matrix((vals[d], cols, rowp), shape=(6 * nn, 6 * nn))
+        if bcs:
+            m = bc_mask(nn)
+            b[d] = np.where(m, x[d], A @ np.where(m, 0.0, x[d]))
+        else:
+            b[d] = A @ x[d]
+    return vals, x, b
+
+
+MESHES = {
+    "1x3": lambda: (Cylinder(1, 3).conn, Cylinder(1, 3).Xpts),      # one front of 36 pivots
+    "4x8": lambda: (Cylinder(4, 8).conn, Cylinder(4, 8).Xpts),      # two leaves
+    "7x13": lambda: (Cylinder(7, 13).conn, Cylinder(7, 13).Xpts),
+    "plate9x10": lambda: random_mesh(9, 10, 3),
+    "33x65": lambda: (Cylinder(33, 65).conn, Cylinder(33, 65).Xpts),
+    "box": lambda: (lambda b: (b.conn, b.Xpts))(BoxBeam(ns=40, nc=12, nh=5, nribs=4)),  # junctions
+    "flat0": lambda: (Cylinder(12, 20).conn, 0.0 * Cylinder(12, 20).Xpts),  # coordinates say nothing
+    "201x402": lambda: (Cylinder(201, 402).conn, Cylinder(201, 402).Xpts),  # fronts of 2,400 pivots
+}
+
+
+@pytest.mark.parametrize("mesh,nb,bcs", [("1x3", 1, False), ("4x8", 2, True), ("7x13", 3, True),
+                                         ("plate9x10", 1, False), ("33x65", 2, True), ("box", 1, True),
+                                         ("flat0", 1, False), ("201x402", 1, True)])
+def test_known_solutions(mesh, nb, bcs):
+    ctx = make(MESHES[mesh](), nb, bcs)
+    vals, x, b = system(ctx, nb, bcs, 5)
+    A = ctx.matrix()
+    A.set_values(vals)
+    if bcs:
+        A.apply_bcs()
+    F = ctx.factor()
+    for _ in range(2):  # a second factor into the same buffers
+        F.compute(A)
+        y = ctx.vector()
+        F.apply(ctx.vector(b), y)
+        got = y.download().reshape(nb, -1)
+        assert np.linalg.norm(got - x) <= TOL * np.linalg.norm(x)
+    # in place
+    y = ctx.vector(b)
+    F.apply(y, y)
+    assert np.array_equal(y.download().reshape(nb, -1), got)
+    F.destroy()
+    ctx.close()
+
+
+def test_indefinite_matrix_is_refused_and_named():
+    mesh = MESHES["7x13"]()
+    ctx = make(mesh, 3, False)
+    vals, x, b = system(ctx, 3, False, 8)
+    rowp, cols = ctx.pattern()
+    diag = [rowp[i] + int(np.where(cols[rowp[i]:rowp[i + 1]] == i)[0][0]) for i in (40,)]
+    bad = vals.copy()
+    bad[1, diag[0], 2, 2] *= -1.0
+    A = ctx.matrix()
+    F = ctx.factor()
+    A.set_values(bad)
+    with pytest.raises(sg.ShellGPUError, match="design 1"):
+        F.compute(A)
+    with pytest.raises(sg.ShellGPUError):
+        F.apply(ctx.vector(b), ctx.vector())
+    A.set_values(vals)
+    F.compute(A)
+    y = ctx.vector()
+    F.apply(ctx.vector(b), y)
+    assert np.linalg.norm(y.download() - x.ravel()) <= TOL * np.linalg.norm(x)
+    ctx.close()
+
+
+def test_captured_solve_matches_direct(monkeypatch):
+    ctx = make(MESHES["7x13"](), 2)
+    vals, x, b = system(ctx, 2, True, 11)
+    A = ctx.matrix()
+    A.set_values(vals)
+    A.apply_bcs()
+    F, G = ctx.factor(), ctx.factor()
+    for f in (F, G):
+        f.compute(A)
+    y, z = ctx.vector(), ctx.vector()
+    F.apply(ctx.vector(b), y)
+    monkeypatch.setenv("SHELLGPU_GRAPH", "1")
+    for rep in range(4):
+        rhs = b * (rep + 1)
+        G.apply(ctx.vector(rhs), z)
+        F.apply(ctx.vector(rhs), y)  # eager work between the replays
+        assert np.array_equal(y.download(), z.download())
+    ctx.close()
+
+
+@pytest.mark.parametrize("cases", [1, 2, 5, 8, 11, 16, 19])
+def test_load_cases_share_one_factor(cases):
+    """Identical designs: a factor of one design solves all vectors (16, or up
+    to 8, at a time); every load case as if it were alone."""
+    cyl = Cylinder(9, 16)
+    rng = np.random.default_rng(3)
+    f = rng.standard_normal((cases, 6 * cyl.nnodes))
+    paths, lam = {}, {}
+    for nb in (1, cases):
+        ctx = sg.Context(0)
+        ctx.set_mesh(cyl.conn, cyl.Xpts)
+        ctx.set_material(70e9, 0.3)
+        ctx.set_bcs(*cyl.bcs())
+        ctx.set_designs(np.full((nb, cyl.nelems), 0.002))
+        p, v = [], []
+        for c in range(0, cases, nb):
+            B = ctx.buckling(sigma=0.0, nev=2, max_lanczos=90, tol=1e-10)
+            B.solve(force=f[c:c + nb])
+            p.append(B.info()["path"])
+            v.append(B.eigenvalues()[0])
+            B.destroy()
+        paths[nb], lam[nb] = np.concatenate(p), np.concatenate(v)
+        ctx.close()
+    # paths solved to 1e-12 by GMRES, condition ~ 1e6; loads to 1e-10
+    assert np.linalg.norm(paths[cases] - paths[1]) <= 1e-8 * np.linalg.norm(paths[1])
+    assert np.abs(lam[cases][:, 0] - lam[1][:, 0]).max() <= 1e-8 * np.abs(lam[1]).max()
+
+
+def test_block_lanczos_solves_blocks(monkeypatch):
+    cyl = Cylinder(10, 20)
+    thick = np.random.default_rng(2).uniform(0.0015, 0.0025, (2, cyl.nelems))
+    out = []
+    for block in ("1", "4"):
+        monkeypatch.setenv("SHELLGPU_LANCZOS_BLOCK", block)
+        ctx = sg.Context(0)
+        ctx.set_mesh(cyl.conn, cyl.Xpts)
+        ctx.set_material(70e9, 0.3)
+        ctx.set_bcs(*cyl.bcs())
+        ctx.set_designs(thick)
+        B = ctx.buckling(sigma=0.0, nev=3, max_lanczos=100, tol=1e-10)
+        B.solve(force=cyl.edge_load(1.0))
+        out.append(B.eigenvalues()[0])
+        B.destroy()
+        ctx.close()
+    assert np.abs(out[0] - out[1]).max() <= 1e-8 * np.abs(out[0]).max()
