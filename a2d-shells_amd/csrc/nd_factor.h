@@ -16,11 +16,13 @@ struct NdFactor {
   long per_design = 0;     // doubles of M per design
   long q_len = 0, s_len[2] = {0, 0}, v_len = 0;
   int chunk = 1;           // designs factored together (workspace copies)
-  int rhs_cap = 1;         // vectors per design that V holds
+  long n = 0;              // dofs
+  int rhs_cap = 0;         // vectors per design that V and W hold: 1 or 16
   std::vector<NdLevel> levels;  // deepest first
   NdDev *d_fronts = nullptr;
   int *d_lists = nullptr;
   double *M = nullptr, *Q = nullptr, *S[2] = {nullptr, nullptr}, *V = nullptr;
+  double *W = nullptr;  // interleaved right-hand sides and solutions of several vectors
 };
 
 // Order, structure and buffers for nbatch designs of the mesh graph; blk_base

@@ -46,6 +46,7 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 typedef double v2d __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(1))) const double gcdouble;
 typedef __attribute__((address_space(1))) double gdouble;
+typedef __attribute__((address_space(1))) const v2d gcv2d;
 
 constexpr int kB = 64;  // pivot block
 // leaves of the dissection: 24 nodes (144 dofs).  Fewer, larger leaves give
@@ -487,15 +488,51 @@ struct SolveArgs {
   const double *b;
   double *x;
   long sM, sV, n;
-  int nd;          // designs: entry e is vector e / nd of design e % nd
-  const int *act;  // entries, or null
+  const int *act;  // designs, or null: all
   int tiles;       // per front
 };
 
+// entry i of a front's vector from its children's u (and, for the pivots, b)
+struct FrontSource {
+  const int *lists;
+  const double *u[2];
+  int mn;
+  __device__ __forceinline__ FrontSource(const SolveArgs &a, const NdDev &d, const double *V, int nv)
+      : lists(a.lists + d.lists), u{nullptr, nullptr}, mn(d.m / 6) {
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+      if (d.child[c] >= 0) {
+        const NdDev ch = a.all[d.child[c]];
+        u[c] = V + (ch.V + ch.ns) * nv;
+      }
+  }
+  __device__ __forceinline__ double children(int i, int nv, int v) const {
+    const int q = i / 6, w = i - 6 * q;
+    double s = 0.0;
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+      if (u[c]) {
+        const int p = lists[(1 + c) * mn + q];
+        if (p >= 0) s += u[c][(6L * p + w) * nv + v];
+      }
+    return s;
+  }
+  __device__ __forceinline__ double pivot(const double *b, int i, int nv, int v) const {
+    const int q = i / 6;
+    return b[(6L * lists[q] + i - 6 * q) * nv + v] + children(i, nv, v);
+  }
+};
+
 constexpr int kStage = 1024;  // vector entries staged at once
+constexpr int kBatch = 8;     // columns of M per wavefront in flight
 
 // upward sweep: y = X v_J and u_B = v_B - W v_J, 128 rows per workgroup (two
-// per lane), the columns split over the NW wavefronts
+// per lane), the columns split over the NW wavefronts.  A level's launch is a
+// chain of memory latencies, so the loads of M (which need nothing of the
+// vector) and the children's part of the rows are issued before the vector is
+// staged, and each batch of columns before the products of the last: a solve
+// of the 200 x 400 cylinder 0.67 -> 0.61 ms (5.0 TB/s over both sweeps), of 16
+// designs of 100 x 200 2.39 -> 2.04 ms.
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void nd_up_kernel(SolveArgs a) {
   __shared__ double vj[kStage];
@@ -503,99 +540,96 @@ __global__ __launch_bounds__(64 * NW) void nd_up_kernel(SolveArgs a) {
   const int f = blockIdx.x / a.tiles, r0 = 128 * (blockIdx.x - f * a.tiles);
   const NdDev d = a.fronts[f];
   if (r0 >= d.m) return;
-  const int e = a.act ? a.act[blockIdx.y] : blockIdx.y, des = e % a.nd;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, mn = d.m / 6;
-  const int *lists = a.lists + d.lists;
+  const int e = a.act ? a.act[blockIdx.y] : blockIdx.y;
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
   double *V = a.V + e * a.sV;
   const double *b = a.b + e * a.n;
-  const double *u[2] = {nullptr, nullptr};
+  const int cend = min(d.ns, r0 + 128), r = r0 + 2 * lane;
+  gcdouble *M = (gcdouble *)(a.M + e * a.sM + d.M + min(r, d.m - 2));
+  v2d mv[2][kBatch];
+  auto load = [&](int buf, int j0) {
 #pragma unroll
-  for (int c = 0; c < 2; c++)
-    if (d.child[c] >= 0) {
-      const NdDev ch = a.all[d.child[c]];
-      u[c] = V + ch.V + ch.ns;
-    }
-  // entry i of the front's vector from the children
-  auto from_children = [&](int i) {
-    const int q = i / 6, w = i - 6 * q;
-    double s = 0.0;
-#pragma unroll
-    for (int c = 0; c < 2; c++)
-      if (u[c]) {
-        const int p = lists[(1 + c) * mn + q];
-        if (p >= 0) s += u[c][6 * p + w];
-      }
-    return s;
+    for (int q = 0; q < kBatch; q++) mv[buf][q] = *(gcv2d *)(M + (long)min(j0 + wave + NW * q, cend - 1) * d.m);
   };
-  const int cend = min(d.ns, r0 + 128);
-  const int row = min(r0 + 2 * lane, d.m - 2);
-  gcdouble *M = (gcdouble *)(a.M + des * a.sM + d.M + row);
+  load(0, 0);
+  const FrontSource src(a, d, V, 1);
   v2d acc = {0.0, 0.0};
-  for (int s0 = 0; s0 < cend; s0 += kStage) {
-    const int sn = min(kStage, cend - s0);
-    if (s0) __syncthreads();
-    for (int i = t; i < sn; i += 64 * NW) {
-      const int q = (s0 + i) / 6, w = s0 + i - 6 * q;
-      vj[i] = b[6L * lists[q] + w] + from_children(s0 + i);
+  if (wave == 0 && r >= d.ns && r < d.m) acc = v2d{src.children(r, 1, 0), src.children(r + 1, 1, 0)};
+  auto mul = [&](int buf, int j0) {
+#pragma unroll
+    for (int q = 0; q < kBatch; q++) acc += mv[buf][q] * vj[(j0 & (kStage - 1)) + wave + NW * q];
+  };
+  static_assert(kStage % (2 * kBatch * NW) == 0, "batches do not cross a staged piece");
+  for (int j0 = 0; j0 < cend; j0 += 2 * kBatch * NW) {
+    if ((j0 & (kStage - 1)) == 0) {
+      if (j0) __syncthreads();
+      // zero past the last column, to the end of the last batch
+      const int sn = min(kStage, (cend - j0 + 2 * kBatch * NW - 1) / (2 * kBatch * NW) * (2 * kBatch * NW));
+      for (int i = t; i < sn; i += 64 * NW) vj[i] = j0 + i < cend ? src.pivot(b, j0 + i, 1, 0) : 0.0;
+      __syncthreads();
     }
-    __syncthreads();
-#pragma unroll 8
-    for (int j = wave; j < sn; j += NW) {
-      const v2d c = *(__attribute__((address_space(1))) const v2d *)(M + (long)(s0 + j) * d.m);
-      acc += c * vj[j];
-    }
+    load(1, j0 + kBatch * NW);
+    mul(0, j0);
+    load(0, j0 + 2 * kBatch * NW);
+    mul(1, j0 + kBatch * NW);
   }
   red[wave][lane] = acc;
   __syncthreads();
   if (wave) return;
 #pragma unroll
   for (int w = 1; w < NW; w++) acc += red[w][lane];
-  const int r = r0 + 2 * lane;
   if (r >= d.m) return;
-  if (r >= d.ns) {
-    acc.x += from_children(r);
-    acc.y += from_children(r + 1);
-  }
   V[d.V + r] = acc.x;
   V[d.V + r + 1] = acc.y;
 }
 
-// downward sweep: x_J = M^T [y ; x_B], CW columns per wavefront and pass,
-// lanes along the rows (two per lane)
+// downward sweep: x_J = M^T [y ; x_B], CW columns per wavefront, lanes along
+// the rows (two per lane), the loads of M ahead of the vector as above
 template <int CW>
 __global__ __launch_bounds__(256) void nd_down_kernel(SolveArgs a) {
-  __shared__ double z[2 * kStage];
+  constexpr int kRows = 2 * kStage;
+  __shared__ __align__(16) double z[kRows];
   const int f = blockIdx.x / a.tiles, c0 = 4 * CW * (blockIdx.x - f * a.tiles);
   const NdDev d = a.fronts[f];
   if (c0 >= d.ns) return;
-  const int e = a.act ? a.act[blockIdx.y] : blockIdx.y, des = e % a.nd;
+  const int e = a.act ? a.act[blockIdx.y] : blockIdx.y;
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
   const int *lists = a.lists + d.lists;
   const double *V = a.V + e * a.sV + d.V;
   double *x = a.x + e * a.n;
   const int cw = c0 + CW * wave;
-  gcdouble *M = (gcdouble *)(a.M + des * a.sM + d.M);
-  v2d acc[CW];
+  // rows before the first column are zero (c0 is even)
+  gcdouble *M = (gcdouble *)(a.M + e * a.sM + d.M + c0);
+  const int rows = d.m - c0;
+  v2d mv[2][CW], acc[CW];
 #pragma unroll
   for (int c = 0; c < CW; c++) acc[c] = v2d{0.0, 0.0};
-  const int s1 = c0 & ~1;  // rows before the first column are zero
-  for (int s0 = s1; s0 < d.m; s0 += 2 * kStage) {
-    const int sn = min(2 * kStage, d.m - s0);
-    if (s0 != s1) __syncthreads();
-    for (int i = t; i < sn; i += 256) {
-      const int r = s0 + i, q = r / 6;
-      z[i] = r < d.ns ? V[r] : x[6L * lists[q] + r - 6 * q];
-    }
-    __syncthreads();
-#pragma unroll 2
-    for (int i = 2 * lane; i < sn; i += 128) {
-      const v2d zz = {z[i], z[i + 1]};
+  auto load = [&](int buf, int i) {
 #pragma unroll
-      for (int c = 0; c < CW; c++) {
-        const int col = min(cw + c, d.ns - 1);
-        acc[c] += *(__attribute__((address_space(1))) const v2d *)(M + s0 + i + (long)col * d.m) * zz;
+    for (int c = 0; c < CW; c++)
+      mv[buf][c] = *(gcv2d *)(M + min(i + 2 * lane, rows - 2) + (long)min(cw + c, d.ns - 1) * d.m);
+  };
+  auto mul = [&](int buf, int i) {
+    const v2d zz = *reinterpret_cast<const v2d *>(&z[(i & (kRows - 1)) + 2 * lane]);
+#pragma unroll
+    for (int c = 0; c < CW; c++) acc[c] += mv[buf][c] * zz;
+  };
+  load(0, 0);
+  for (int i0 = 0; i0 < rows; i0 += 256) {
+    if ((i0 & (kRows - 1)) == 0) {
+      if (i0) __syncthreads();
+      // zero past the last row, to the end of the last batch
+      const int sn = min(kRows, (rows - i0 + 255) & ~255);
+      for (int i = t; i < sn; i += 256) {
+        const int r = c0 + i0 + i, q = r / 6;
+        z[i] = r >= d.m ? 0.0 : r < d.ns ? V[r] : x[6L * lists[q] + r - 6 * q];
       }
+      __syncthreads();
     }
+    load(1, i0 + 128);
+    mul(0, i0);
+    load(0, i0 + 256);
+    mul(1, i0 + 128);
   }
 #pragma unroll
   for (int c = 0; c < CW; c++) {
@@ -608,6 +642,219 @@ __global__ __launch_bounds__(256) void nd_down_kernel(SolveArgs a) {
       x[6L * lists[q] + col - 6 * q] = s;
     }
   }
+}
+
+// ---- several vectors per design ------------------------------------------
+//
+// Load cases share one factor, so their vectors go through it together: the
+// panels are read once for up to 16 of them, as matrix products with 16
+// columns (v_mfma_f64_16x16x4f64).  The vectors are interleaved, entry i of
+// vector v at 16 i + v, so every gather along a node list moves whole 128-byte
+// lines.  16 vectors of a 32,000-quad box beam: 0.79 ms a solve (2.3 ms with
+// the single-vector kernels run once per vector).
+constexpr int kNv = 16;
+
+// n-vectors b (vector v of design d at (v nd + d) n) <-> interleaved w (n x 16
+// per design; the vectors past nrhs are zero)
+__global__ __launch_bounds__(256) void nd_interleave_kernel(long n, int nd, int nrhs, const double *__restrict__ b,
+                                                            double *__restrict__ w) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int d = blockIdx.y;
+  v2d *o = reinterpret_cast<v2d *>(w + ((long)d * n + i) * kNv);
+#pragma unroll
+  for (int v = 0; v < kNv; v += 2) {
+    v2d t;
+    t.x = v < nrhs ? b[((long)v * nd + d) * n + i] : 0.0;
+    t.y = v + 1 < nrhs ? b[((long)(v + 1) * nd + d) * n + i] : 0.0;
+    o[v / 2] = t;
+  }
+}
+__global__ __launch_bounds__(256) void nd_deinterleave_kernel(long n, int nd, int nrhs, const double *__restrict__ w,
+                                                              double *__restrict__ x) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int d = blockIdx.y;
+  const v2d *o = reinterpret_cast<const v2d *>(w + ((long)d * n + i) * kNv);
+#pragma unroll
+  for (int v = 0; v < kNv; v += 2) {
+    const v2d t = o[v / 2];
+    if (v < nrhs) x[((long)v * nd + d) * n + i] = t.x;
+    if (v + 1 < nrhs) x[((long)(v + 1) * nd + d) * n + i] = t.y;
+  }
+}
+
+constexpr int kStageM = 256;  // rows of 16 values staged at once
+
+// upward sweep, 32 RG rows per workgroup: a wavefront takes 32 rows (two per
+// lane, one 16-row matrix block of the even and one of the odd rows) and every
+// CS-th group of four columns
+template <int RG, int CS>
+__global__ __launch_bounds__(64 * RG * CS) void nd_up_multi_kernel(SolveArgs a) {
+  constexpr int NW = RG * CS, kU = 4, kStep = 4 * CS * kU;  // columns of a batch
+  constexpr int kLds = CS > 1 && NW * 512 > kStageM * 17 ? NW * 512 : kStageM * 17;
+  __shared__ double lds[kLds];
+  const int f = blockIdx.x / a.tiles, r0 = 32 * RG * (blockIdx.x - f * a.tiles);
+  const NdDev d = a.fronts[f];
+  if (r0 >= d.m) return;
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, lr = lane & 15, lk = lane >> 4;
+  const int rg = wave % RG, cs = wave / RG;
+  double *V = a.V + blockIdx.y * a.sV;
+  const double *b = a.x + blockIdx.y * a.n * kNv;
+  const int cend = min(d.ns, r0 + 32 * RG);
+  const int row = r0 + 32 * rg + 2 * lr;
+  gcdouble *M = (gcdouble *)(a.M + blockIdx.y * a.sM + d.M + min(row, d.m - 2));
+  v2d mv[2][kU];
+  auto load = [&](int buf, int c0) {
+#pragma unroll
+    for (int q = 0; q < kU; q++) mv[buf][q] = *(gcv2d *)(M + (long)min(c0 + 4 * (cs + CS * q) + lk, cend - 1) * d.m);
+  };
+  load(0, 0);
+  const FrontSource src(a, d, V, kNv);
+  v4d acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+  if (cs == 0) {
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+      if (row + h >= d.ns && row + h < d.m) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[h][e] = src.children(row + h, kNv, 4 * e + lk);
+      }
+  }
+  auto mul = [&](int buf, int c0) {
+#pragma unroll
+    for (int q = 0; q < kU; q++) {
+      const double bv = lds[17 * ((c0 & (kStageM - 1)) + 4 * (cs + CS * q) + lk) + lr];
+      acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv, mv[buf][q].x, acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv, mv[buf][q].y, acc[1], 0, 0, 0);
+    }
+  };
+  static_assert(kStageM % kStep == 0, "batches do not cross a staged piece");
+  for (int s0 = 0; s0 < cend; s0 += kStageM) {
+    if (s0) __syncthreads();
+    // zero past the last column, to the end of the last batch
+    const int sn = min(kStageM, (cend - s0 + kStep - 1) / kStep * kStep);
+    for (int e = t; e < kNv * sn; e += 64 * NW) {
+      const int i = e / kNv, v = e % kNv;
+      lds[17 * i + v] = s0 + i < cend ? src.pivot(b, s0 + i, kNv, v) : 0.0;
+    }
+    __syncthreads();
+    int c = s0;
+    for (; c + kStep < s0 + sn; c += 2 * kStep) {
+      load(1, c + kStep);
+      mul(0, c);
+      load(0, c + 2 * kStep);
+      mul(1, c + kStep);
+    }
+    if (c < s0 + sn) {  // one batch left: the piece is the last, or one batch
+      load(1, c + kStep);
+      mul(0, c);
+#pragma unroll
+      for (int q = 0; q < kU; q++) mv[0][q] = mv[1][q];
+    }
+  }
+  if (CS > 1) {  // the column parts of a row group, added in order
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) lds[512 * wave + 64 * (4 * h + e) + lane] = acc[h][e];
+    __syncthreads();
+    if (cs) return;
+#pragma unroll 1
+    for (int c = 1; c < CS; c++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[h][e] += lds[512 * (RG * c + rg) + 64 * (4 * h + e) + lane];
+  }
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int r = row + h;
+    if (r >= d.m) continue;
+#pragma unroll
+    for (int e = 0; e < 4; e++) V[(d.V + r) * kNv + 4 * e + lk] = acc[h][e];
+  }
+}
+
+// downward sweep, 16 CW columns per workgroup: a wavefront takes 16 columns
+// and every RS-th group of 16 rows (four consecutive rows per lane, the sum
+// over rows in any order)
+template <int CW, int RS>
+__global__ __launch_bounds__(64 * CW * RS) void nd_down_multi_kernel(SolveArgs a) {
+  constexpr int NW = CW * RS, kU = kStageM / (16 * RS) < 2 ? 1 : 2, kStep = 16 * RS * kU;  // rows of a batch
+  constexpr int kLds = RS > 1 && NW * 256 > kStageM * 17 ? NW * 256 : kStageM * 17;
+  __shared__ double lds[kLds];
+  const int f = blockIdx.x / a.tiles, t0 = 16 * CW * (blockIdx.x - f * a.tiles);
+  const NdDev d = a.fronts[f];
+  if (t0 >= d.ns) return;
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, lr = lane & 15, lk = lane >> 4;
+  const int cw = wave % CW, rs = wave / CW;
+  const int *lists = a.lists + d.lists;
+  const double *V = a.V + blockIdx.y * a.sV + d.V * kNv;
+  double *x = a.x + blockIdx.y * a.n * kNv;
+  const int col = t0 + 16 * cw + lr;
+  // rows before the first column are zero (t0 is even)
+  gcdouble *M = (gcdouble *)(a.M + blockIdx.y * a.sM + d.M + t0 + (long)min(col, d.ns - 1) * d.m);
+  const int rows = d.m - t0;
+  v4d acc = {0.0, 0.0, 0.0, 0.0};
+  v2d mv[2][kU][2];
+  auto load = [&](int buf, int i0) {
+#pragma unroll
+    for (int q = 0; q < kU; q++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        mv[buf][q][h] = *(gcv2d *)(M + min(i0 + 16 * (rs + RS * q) + 4 * lk + 2 * h, rows - 2));
+  };
+  auto mul = [&](int buf, int i0) {
+#pragma unroll
+    for (int q = 0; q < kU; q++)
+#pragma unroll
+      for (int h = 0; h < 4; h++)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(lds[17 * ((i0 & (kStageM - 1)) + 16 * (rs + RS * q) + 4 * lk + h) + lr],
+                                                   mv[buf][q][h >> 1][h & 1], acc, 0, 0, 0);
+  };
+  static_assert(kStageM % kStep == 0, "batches do not cross a staged piece");
+  load(0, 0);
+  for (int s0 = 0; s0 < rows; s0 += kStageM) {
+    if (s0) __syncthreads();
+    // zero past the last row, to the end of the last batch
+    const int sn = min(kStageM, (rows - s0 + kStep - 1) / kStep * kStep);
+    for (int e = t; e < kNv * sn; e += 64 * NW) {
+      const int i = e / kNv, v = e % kNv, r = t0 + s0 + i, q = r / 6;
+      lds[17 * i + v] = r >= d.m ? 0.0 : r < d.ns ? V[(long)r * kNv + v] : x[(6L * lists[q] + r - 6 * q) * kNv + v];
+    }
+    __syncthreads();
+    int i = s0;
+    for (; i + kStep < s0 + sn; i += 2 * kStep) {
+      load(1, i + kStep);
+      mul(0, i);
+      load(0, i + 2 * kStep);
+      mul(1, i + kStep);
+    }
+    if (i < s0 + sn) {  // one batch left
+      load(1, i + kStep);
+      mul(0, i);
+#pragma unroll
+      for (int q = 0; q < kU; q++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) mv[0][q][h] = mv[1][q][h];
+    }
+  }
+  if (RS > 1) {
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 4; e++) lds[256 * wave + 64 * e + lane] = acc[e];
+    __syncthreads();
+    if (rs) return;
+#pragma unroll
+    for (int c = 1; c < RS; c++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[e] += lds[256 * (CW * c + cw) + 64 * e + lane];
+  }
+  if (col >= d.ns) return;
+  const int q = col / 6;
+#pragma unroll
+  for (int e = 0; e < 4; e++) x[(6L * lists[q] + col - 6 * q) * kNv + 4 * e + lk] = acc[e];
 }
 
 template <typename T>
@@ -635,14 +882,14 @@ std::string nd_create(int nn, const std::vector<int> &rowp, const std::vector<in
   // the 100 x 200 cylinder), which leaves no level short of workgroups
   const double ws = 8.0 * (F.q_len + F.s_len[0] + F.s_len[1]);
   F.chunk = std::max(1, (int)std::min<double>(nbatch, 4294967296.0 / ws));
-  F.rhs_cap = std::max(1, nrhs);
+  F.n = 6L * nn;
   hipError_t e = upload(&F.d_fronts, L.fronts);
   if (e == hipSuccess) e = upload(&F.d_lists, L.lists);
   if (e == hipSuccess) e = hipMalloc((void **)&F.M, sizeof(double) * (size_t)F.per_design * nbatch);
   if (e == hipSuccess) e = hipMalloc((void **)&F.Q, sizeof(double) * (size_t)F.q_len * F.chunk);
   for (int k = 0; k < 2 && e == hipSuccess; k++)
     e = hipMalloc((void **)&F.S[k], sizeof(double) * (size_t)F.s_len[k] * F.chunk);
-  if (e == hipSuccess) e = hipMalloc((void **)&F.V, sizeof(double) * (size_t)F.v_len * nbatch * F.rhs_cap);
+  if (e == hipSuccess) e = nd_reserve(F, nrhs);
   if (e != hipSuccess)
     return std::string("factor allocation (") + std::to_string((long)(8.0 * F.per_design * nbatch) >> 20) +
            " MiB): " + hipGetErrorString(e);
@@ -650,19 +897,25 @@ std::string nd_create(int nn, const std::vector<int> &rowp, const std::vector<in
 }
 
 void nd_destroy(NdFactor &F) {
-  void *bufs[] = {F.d_fronts, F.d_lists, F.M, F.Q, F.S[0], F.S[1], F.V};
+  void *bufs[] = {F.d_fronts, F.d_lists, F.M, F.Q, F.S[0], F.S[1], F.V, F.W};
   for (void *p : bufs)
     if (p) (void)hipFree(p);
   F = NdFactor();
 }
 
 hipError_t nd_reserve(NdFactor &F, int nrhs) {
-  if (nrhs <= F.rhs_cap) return hipSuccess;
-  hipError_t e = hipFree(F.V);
-  F.V = nullptr;
+  // several vectors take the buffers of 16
+  const int cap = nrhs > 1 ? kNv : 1;
+  if (cap <= F.rhs_cap) return hipSuccess;
+  if (nrhs > kNv) return hipErrorInvalidValue;
   F.rhs_cap = 0;
-  if (e == hipSuccess) e = hipMalloc((void **)&F.V, sizeof(double) * (size_t)F.v_len * F.nbatch * nrhs);
-  if (e == hipSuccess) F.rhs_cap = nrhs;
+  for (double **p : {&F.V, &F.W}) {
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+  }
+  hipError_t e = hipMalloc((void **)&F.V, sizeof(double) * (size_t)F.v_len * F.nbatch * cap);
+  if (e == hipSuccess && cap > 1) e = hipMalloc((void **)&F.W, sizeof(double) * (size_t)F.n * F.nbatch * cap);
+  if (e == hipSuccess) F.rhs_cap = cap;
   return e;
 }
 
@@ -728,9 +981,53 @@ hipError_t nd_solve(const NdFactor &F, const double *b, double *x, long n, int n
   a.sM = F.per_design;
   a.sV = F.v_len;
   a.n = n;
-  a.nd = F.nbatch;
   a.act = act;
-  const unsigned ne = (unsigned)(act ? nact : F.nbatch * nrhs);
+  if (nrhs > 1 && !act) {
+    a.x = F.W;
+    a.sV = F.v_len * kNv;
+    const dim3 ig((unsigned)((n + 255) / 256), F.nbatch);
+    hipLaunchKernelGGL(nd_interleave_kernel, ig, dim3(256), 0, stream, n, F.nbatch, nrhs, b, F.W);
+    for (const NdLevel &lv : F.levels) {
+      a.fronts = F.d_fronts + lv.f0;
+      const long rows = (long)lv.nf * F.nbatch * ((lv.max_m + 31) / 32);
+      // 32-row pieces of the level: enough of them fill the GPU with whole
+      // columns, fewer split the columns over the wavefronts of a workgroup
+      if (rows >= 8192) {
+        a.tiles = (lv.max_m + 127) / 128;
+        hipLaunchKernelGGL((nd_up_multi_kernel<4, 1>), dim3((unsigned)(lv.nf * a.tiles), F.nbatch), dim3(256), 0,
+                           stream, a);
+      } else if (rows >= 1024) {
+        a.tiles = (lv.max_m + 63) / 64;
+        hipLaunchKernelGGL((nd_up_multi_kernel<2, 4>), dim3((unsigned)(lv.nf * a.tiles), F.nbatch), dim3(512), 0,
+                           stream, a);
+      } else {
+        a.tiles = (lv.max_m + 31) / 32;
+        hipLaunchKernelGGL((nd_up_multi_kernel<1, 16>), dim3((unsigned)(lv.nf * a.tiles), F.nbatch), dim3(1024), 0,
+                           stream, a);
+      }
+    }
+    for (size_t l = F.levels.size(); l-- > 0;) {
+      const NdLevel &lv = F.levels[l];
+      a.fronts = F.d_fronts + lv.f0;
+      const long cols = (long)lv.nf * F.nbatch * ((lv.max_ns + 15) / 16);
+      if (cols >= 4096) {
+        a.tiles = (lv.max_ns + 127) / 128;
+        hipLaunchKernelGGL((nd_down_multi_kernel<8, 1>), dim3((unsigned)(lv.nf * a.tiles), F.nbatch), dim3(512), 0,
+                           stream, a);
+      } else if (cols >= 512) {
+        a.tiles = (lv.max_ns + 31) / 32;
+        hipLaunchKernelGGL((nd_down_multi_kernel<2, 4>), dim3((unsigned)(lv.nf * a.tiles), F.nbatch), dim3(512), 0,
+                           stream, a);
+      } else {
+        a.tiles = (lv.max_ns + 15) / 16;
+        hipLaunchKernelGGL((nd_down_multi_kernel<1, 16>), dim3((unsigned)(lv.nf * a.tiles), F.nbatch), dim3(1024), 0,
+                           stream, a);
+      }
+    }
+    hipLaunchKernelGGL(nd_deinterleave_kernel, ig, dim3(256), 0, stream, n, F.nbatch, nrhs, F.W, x);
+    return hipGetLastError();
+  }
+  const unsigned ne = (unsigned)(act ? nact : F.nbatch);
   for (const NdLevel &lv : F.levels) {
     a.fronts = F.d_fronts + lv.f0;
     a.tiles = (lv.max_m + 127) / 128;
