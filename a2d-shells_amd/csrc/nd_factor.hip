@@ -186,124 +186,197 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
   return __longlong_as_double((long)hi << 32 | lo);
 }
 
-// diagonal block k: X_k = chol(C_kk)^{-1} into C_kk (zero above the
-// diagonal) and its transpose into Q_kk; one workgroup per front and design.
+// Diagonal block k: X_k = chol(C_kk)^{-1} into C_kk (zero above the
+// diagonal) and its transpose into Q_kk, by one workgroup.
 //
-// The chain of these launches is what bounds a factorisation, so the kernel
-// is built for latency: the block is cut in four column blocks of 16, one per
-// wavefront, lane i holding row i of it in registers.  A column block is
-// factored with the pivot row broadcast by v_readlane (no LDS round trip or
-// barrier per pivot), then written to LDS, where the wavefronts right of it
-// take their update from; four barriers in all.  The 16 x 16 inverses of the
-// diagonal blocks come the same way from the registers, beside those updates,
-// and the rest of X from matrix instructions: X_ij = -X_ii sum L_ik X_kj, one
-// column block per wavefront, whose results are already laid out as the
-// second operand of the next product.  Blocks shorter than 64 are padded
-// with the identity.  28 us per launch over a factor of the 200 x 400 cylinder
-// (106 launches; 112 us with one barrier and LDS round trip per pivot).
-constexpr int kDiagThreads = 256;
-__global__ __launch_bounds__(kDiagThreads) void nd_diag_kernel(LevelArgs a, int *info) {
-  constexpr int ld = kB + 1;
-  __shared__ double Lc[kB][ld];      // L by columns
-  __shared__ double Xd[4][16][17];   // inverses of the diagonal blocks, by rows
-  const NdDev d = a.fronts[blockIdx.x];
-  const int k0 = kB * a.k, m = d.m;
-  if (k0 >= d.ns) return;
-  const int n = min(kB, d.ns - k0), nblk = (n + 15) / 16;
+// The chain of these blocks is what bounds a factorisation near the root, so
+// the code is built for latency: the block lies in LDS as four column blocks
+// of 16; a wavefront takes a column block in registers, lane i holding row i,
+// and factors it with the pivot row broadcast by v_readlane (no LDS round trip
+// or barrier per pivot).  Between two panels all wavefronts update the
+// remaining 16 x 16 tiles with matrix instructions.  X follows two panels
+// behind, on the wavefronts the panel leaves idle: first the inverse of a
+// diagonal block, then the columns of X, Y_ij -= L_ib X_bj with X_bj = X_bb
+// Y_bj, whose tiles stay in registers (a result of the matrix instruction is
+// laid out as the second operand of the next).  Blocks shorter than 64 are
+// padded with the identity.  16 us a block near the root (25 us with the
+// inverses on the panels' path, 112 us with one barrier and LDS round trip per
+// pivot).
+struct DiagLds {
+  double L[kB][kB + 1];  // by columns; odd stride: constant offsets and no bank conflicts
+  double Xd[4][16][17];  // inverses of the diagonal blocks, by rows
+  double rs[kB];         // 1 / L_jj
+};
+
+// 1 / sqrt(p): the hardware's estimate and one third-order step (relative
+// error of the estimate below 2^-24: 5/16 of its cube is below 2^-53)
+__device__ __forceinline__ double inv_sqrt(double p) {
+  const double y = __builtin_amdgcn_rsq(p);
+  const double e = fma(-y * p, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// all 256 threads of a workgroup; returns true (in any lane of the panel's
+// wavefront) for a pivot that is not positive
+__device__ __forceinline__ bool diag_block(DiagLds &lds, gdouble *C, gdouble *Q, int n, int m) {
+  const int nblk = (n + 15) / 16;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  gdouble *C = (gdouble *)(a.M + blockIdx.y * a.sM + d.M + k0 + (long)k0 * m);
-  gdouble *Q = (gdouble *)(a.Q + blockIdx.y * a.sQ + d.Q + k0 + (long)k0 * m);
-  double r[16], rs[16];
+  const int lr = lane & 15, lk = lane >> 4;
+  double r[16];
 #pragma unroll
   for (int c = 0; c < 16; c++) {
     const int j = 16 * w + c;
     const double v = C[min(lane, n - 1) + (long)min(j, n - 1) * m];
     r[c] = lane < n && j < n ? v : (lane == j ? 1.0 : 0.0);
   }
+  if (w > 0 && lane >= 16 * w) {
+#pragma unroll
+    for (int c = 0; c < 16; c++) lds.L[16 * w + c][lane] = r[c];
+  }
+  // column block w of X: tile (w + t, w) in R[t], eliminated with block row b
+  v4d R[4];
+  auto eliminate = [&](int b) {
+    if (b == w) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) R[0][e] = lds.Xd[w][4 * e + lk][lr];
+    }
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      if (b - w != s) continue;
+      if (s > 0) {
+        v4d x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < 4; q++) x = __builtin_amdgcn_mfma_f64_16x16x4f64(lds.Xd[b][lr][4 * q + lk], R[s][q], x, 0, 0, 0);
+        R[s] = x;
+      }
+#pragma unroll
+      for (int t = s + 1; t < 4; t++) {
+        if (w + t >= nblk) continue;
+        if (s == 0) R[t] = v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          R[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-lds.L[16 * b + 4 * q + lk][16 * (w + t) + lr], R[s][q], R[t], 0,
+                                                      0, 0);
+      }
+    }
+  };
+  // inverse of diagonal block b by four rank-4 steps: with Z the inverse of
+  // the 4 x 4 block s, its rows become Z Y_s and the rows below take -L_is Z
+  // Y_s; lane: row lr and column lk of P_s = [Z; -L_is Z]
+  auto invert = [&](int b) {
+    const double *rs = &lds.rs[16 * b];
+    auto at = [&](int i, int j) { return lds.L[16 * b + j][16 * b + i]; };
+    double P[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const int o = 4 * s;
+      const double z0 = lk == 0 ? rs[o] : 0.0;
+      const double z1 = ((lk == 1 ? 1.0 : 0.0) - at(o + 1, o) * z0) * rs[o + 1];
+      const double z2 = ((lk == 2 ? 1.0 : 0.0) - at(o + 2, o) * z0 - at(o + 2, o + 1) * z1) * rs[o + 2];
+      const double z3 =
+          ((lk == 3 ? 1.0 : 0.0) - at(o + 3, o) * z0 - at(o + 3, o + 1) * z1 - at(o + 3, o + 2) * z2) * rs[o + 3];
+      const int i = lr - o;
+      const double in = i == 0 ? z0 : i == 1 ? z1 : i == 2 ? z2 : z3;
+      const double below = -(at(lr, o) * z0 + at(lr, o + 1) * z1 + at(lr, o + 2) * z2 + at(lr, o + 3) * z3);
+      P[s] = i < 0 ? 0.0 : i < 4 ? in : below;
+    }
+    v4d Y;
+#pragma unroll
+    for (int e = 0; e < 4; e++) Y[e] = 4 * e + lk == lr ? 1.0 : 0.0;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const double ys = Y[s];
+      Y[s] = 0.0;  // rows 4 s + lk: replaced, not added to (Z may be tiny beside the identity)
+      Y = __builtin_amdgcn_mfma_f64_16x16x4f64(P[s], ys, Y, 0, 0, 0);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) lds.Xd[b][4 * e + lk][lr] = Y[e];
+  };
   bool bad = false;
   for (int b = 0; b < nblk; b++) {
     if (w == b) {
+      if (b > 0) {
+#pragma unroll
+        for (int c = 0; c < 16; c++) r[c] = lds.L[16 * b + c][max(lane, 16 * b)];
+      }
+      double rs_lane = 0.0;
 #pragma unroll
       for (int j = 0; j < 16; j++) {
-        double p = lane_value(r[j], 16 * b + j);
-        if (!(p > 0.0)) {
-          bad = true;
-          p = 1.0;
-        }
-        rs[j] = rsqrt(p);
-        r[j] *= rs[j];
+        const double p = lane_value(r[j], 16 * b + j), rs = inv_sqrt(p);
+        bad = bad || !(p > 0.0);
+        r[j] *= rs;
+        rs_lane = lane == j ? rs : rs_lane;
 #pragma unroll
         for (int c = j + 1; c < 16; c++) r[c] -= r[j] * lane_value(r[j], 16 * b + c);
       }
+      if (lane >= 16 * b) {
 #pragma unroll
-      for (int j = 0; j < 16; j++) Lc[16 * b + j][lane] = r[j];
+        for (int j = 0; j < 16; j++) lds.L[16 * b + j][lane] = r[j];
+      }
+      if (lane < 16) lds.rs[16 * b + lane] = rs_lane;
+    } else if (w == b - 1) {
+      invert(b - 1);
+    } else if (w < b) {
+      eliminate(b - 2);
     }
     __syncthreads();
-    if (w == b) {
-      // column lane % 16 of the inverse of the diagonal block
-      double x[16];
+    // tiles (i, j) right of block b, dealt to the wavefronts
+    int q = w;
+    for (int j = b + 1; j < nblk; j++)
+      for (int i = j; i < nblk; i++, q--) {
+        if (q < 0) q = 3;
+        if (q != 0) continue;
+        v4d t;
 #pragma unroll
-      for (int i = 0; i < 16; i++) {
-        x[i] = (lane & 15) == i ? 1.0 : 0.0;
+        for (int e = 0; e < 4; e++) t[e] = -lds.L[16 * j + 4 * e + lk][16 * i + lr];
 #pragma unroll
-        for (int k = 0; k < i; k++) x[i] -= lane_value(r[k], 16 * b + i) * x[k];
-        x[i] *= rs[i];
+        for (int e = 0; e < 4; e++)
+          t = __builtin_amdgcn_mfma_f64_16x16x4f64(lds.L[16 * b + 4 * e + lk][16 * j + lr],
+                                                   lds.L[16 * b + 4 * e + lk][16 * i + lr], t, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; e++) lds.L[16 * j + 4 * e + lk][16 * i + lr] = -t[e];
       }
-      if (lane < 16) {
-#pragma unroll
-        for (int i = 0; i < 16; i++) Xd[b][i][lane] = x[i];
-      }
-    } else if (w > b && w < nblk) {
-#pragma unroll
-      for (int j = 0; j < 16; j++) {
-        const double l = Lc[16 * b + j][lane];
-#pragma unroll
-        for (int c = 0; c < 16; c++) r[c] -= l * lane_value(l, 16 * w + c);
-      }
-    }
+    if (b + 1 < nblk) __syncthreads();
   }
+  if (w == nblk - 1)
+    invert(w);
+  else if (w < nblk - 1)
+    eliminate(nblk - 2);
   __syncthreads();
   if (w < nblk) {
-    const int lr = lane & 15, lk = lane >> 4;
-    auto put = [&](int i, int e, double v) {  // entry (16 i + 4 e + lk, 16 w + lr) of X
-      const int row = 16 * i + 4 * e + lk, col = 16 * w + lr;
-      if (row >= n || col >= n) return;
-      C[row + (long)col * m] = v;
-      Q[col + (long)row * m] = v;
-    };
-    v4d R[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) R[0][e] = Xd[w][4 * e + lk][lr];
-#pragma unroll
-    for (int t = 1; t < 4; t++) {
-      const int i = w + t;
-      if (i >= nblk) continue;
-      v4d T = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int u = 0; u < t; u++)
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          T = __builtin_amdgcn_mfma_f64_16x16x4f64(Lc[16 * (w + u) + 4 * q + lk][16 * i + lr], R[u][q], T, 0, 0, 0);
-      R[t] = v4d{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-        R[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-Xd[i][lr][4 * q + lk], T[q], R[t], 0, 0, 0);
-    }
+    eliminate(nblk - 1);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       if (i >= nblk) continue;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        // R is indexed from the diagonal block: select without a register index
+        // entry (16 i + 4 e + lk, 16 w + lr) of X; R is indexed from the
+        // diagonal block: select without a register index
         double v = 0.0;
 #pragma unroll
         for (int t = 0; t < 4; t++)
           if (i - w == t) v = R[t][e];
-        put(i, e, v);
+        const int row = 16 * i + 4 * e + lk, col = 16 * w + lr;
+        if (row >= n || col >= n) continue;
+        C[row + (long)col * m] = v;
+        Q[col + (long)row * m] = v;
       }
     }
   }
-  if (bad && lane == 0) info[blockIdx.y] = 1;
+  return bad;
+}
+
+// pivot block k of every front (the first; the later ones too unless
+// nd_update_kernel has factored them)
+__global__ __launch_bounds__(256, 2) void nd_diag_kernel(LevelArgs a, int *info) {
+  __shared__ DiagLds lds;
+  const NdDev d = a.fronts[blockIdx.x];
+  const int k0 = kB * a.k;
+  if (k0 >= d.ns) return;
+  const long o = k0 + (long)k0 * d.m;
+  gdouble *C = (gdouble *)(a.M + blockIdx.y * a.sM + d.M + o);
+  gdouble *Q = (gdouble *)(a.Q + blockIdx.y * a.sQ + d.Q + o);
+  if (diag_block(lds, C, Q, min(kB, d.ns - k0), d.m) && (threadIdx.x & 63) == 0) info[blockIdx.y] = 1;
 }
 
 // Q_ik = C_ik X_k^T for the rows after block k (tiles 0 .. tr), and the row
@@ -374,45 +447,64 @@ __global__ __launch_bounds__(256) void nd_scale_kernel(LevelArgs a) {
 }
 
 // C_ij -= Q_ik Q_jk^T for the rows after block k: columns before k, column
-// block k (from zero), and the trailing lower triangle
-__global__ __launch_bounds__(256) void nd_update_kernel(LevelArgs a) {
-  const int f = blockIdx.x / (a.tr * a.tc), t = blockIdx.x - f * a.tr * a.tc;
+// block k (from zero), and the trailing lower triangle.  AHEAD: the workgroup
+// of the next diagonal block goes on to factor it, so that chain runs beside
+// the other tiles' updates (those tiles come first in the grid, for all
+// fronts).
+template <bool AHEAD>
+__global__ __launch_bounds__(256, AHEAD ? 2 : 4) void nd_update_kernel(LevelArgs a, int nf, int *info) {
+  const int f = blockIdx.x % nf, t = blockIdx.x / nf;
   const NdDev d = a.fronts[f];
   const int k0 = kB * a.k, ns = d.ns, m = d.m;
   if (k0 >= ns) return;
-  const int n = min(kB, ns - k0), rs = k0 + n, tj = t / a.tr;
+  const int n = min(kB, ns - k0), rs = k0 + n;
+  int tj = a.k + 1 + t / a.tr;  // column tiles from the next block on, then those before it
+  if (tj >= a.tc) tj -= a.tc;
   const int r0 = rs + kB * (t % a.tr);
   const int c0 = tj <= a.k ? kB * tj : rs + kB * (tj - a.k - 1);
   if (r0 >= m || c0 >= ns || r0 + kB <= c0) return;
   const int cw = tj == a.k ? n : min(kB, ns - c0);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
   const int wm = 32 * (wave & 1), wn = 32 * (wave >> 1);
-  if (r0 + wm >= m || wn >= cw) return;
   gdouble *C = (gdouble *)(a.M + blockIdx.y * a.sM + d.M);
-  gcdouble *Q = (gcdouble *)(a.Q + blockIdx.y * a.sQ + d.Q + (long)k0 * m);
-  Frag acc;
-  clear(acc);
-  long ra[2], rb[2];
+  gdouble *Qf = (gdouble *)(a.Q + blockIdx.y * a.sQ + d.Q);
+  if (r0 + wm < m && wn < cw) {
+    gcdouble *Q = Qf + (long)k0 * m;
+    // the tile enters as the negated sum, so its loads overlap the operands'
+    Frag acc;
+    long ra[2], rb[2];
 #pragma unroll
-  for (int i = 0; i < 2; i++) {
-    ra[i] = min(r0 + wm + 16 * i + lr, m - 1);
-    rb[i] = c0 + min(wn + 16 * i + lr, cw - 1);
+    for (int i = 0; i < 2; i++) {
+      ra[i] = min(r0 + wm + 16 * i + lr, m - 1);
+      rb[i] = c0 + min(wn + 16 * i + lr, cw - 1);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          acc.c[i][j][e] = tj == a.k ? 0.0 : -C[ra[i] + (long)(c0 + min(wn + 16 * j + 4 * e + lk, cw - 1)) * m];
+    mma32(acc, n, [&](int i, int kk) { return Q[ra[i] + (long)kk * m]; },
+          [&](int i, int kk) { return Q[rb[i] + (long)kk * m]; });
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int r = r0 + wm + 16 * i + lr;
+      if (r >= m) continue;
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int c = wn + 16 * j + 4 * e + lk;
+          if (c < cw) C[r + (long)(c0 + c) * m] = -acc.c[i][j][e];
+        }
+    }
   }
-  mma32(acc, n, [&](int i, int kk) { return Q[ra[i] + (long)kk * m]; },
-        [&](int i, int kk) { return Q[rb[i] + (long)kk * m]; });
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int r = r0 + wm + 16 * i + lr;
-    if (r >= m) continue;
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int c = wn + 16 * j + 4 * e + lk;
-        if (c >= cw) continue;
-        gdouble *p = C + r + (long)(c0 + c) * m;
-        *p = tj == a.k ? -acc.c[i][j][e] : *p - acc.c[i][j][e];
-      }
+  if (AHEAD && tj == a.k + 1 && r0 == c0) {  // the next diagonal block (the whole workgroup)
+    __shared__ DiagLds lds;
+    __syncthreads();
+    const long o = c0 + (long)c0 * m;
+    if (diag_block(lds, C + o, Qf + o, min(kB, ns - c0), m) && lane == 0) info[blockIdx.y] = 1;
   }
 }
 
@@ -431,6 +523,10 @@ __global__ __launch_bounds__(256) void nd_schur_kernel(LevelArgs a) {
   if (r0 >= nb || c0 >= nb || r0 + 32 <= c0) return;
   gcdouble *Q = (gcdouble *)(a.Q + blockIdx.y * a.sQ + d.Q + ns);
   gdouble *S = (gdouble *)(a.S + blockIdx.y * a.sS + d.S);
+  const int mn = m / 6;
+  const int *lists = a.lists + d.lists;
+  // the children's parts enter as the negated sum, so their loads overlap the
+  // operands'
   Frag acc;
   clear(acc);
   long ra[2], rb[2];
@@ -439,43 +535,47 @@ __global__ __launch_bounds__(256) void nd_schur_kernel(LevelArgs a) {
     ra[i] = min(r0 + 16 * i + lr, nb - 1);
     rb[i] = min(c0 + 16 * i + lr, nb - 1);
   }
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    if (d.child[c] < 0) continue;
+    const NdDev ch = a.all[d.child[c]];
+    const int ldc = ch.m - ch.ns, *place = lists + (1 + c) * mn + ns / 6;
+    gcdouble *Sc = (gcdouble *)(a.Sc + blockIdx.y * a.sSc + ch.S);
+    int ir[2], rr[2], ic[2][4], cc[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      rr[i] = (int)ra[i] % 6;
+      ir[i] = place[(int)ra[i] / 6];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int col = min(c0 + 16 * i + 4 * e + lk, nb - 1);
+        cc[i][e] = col % 6;
+        ic[i][e] = place[col / 6];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int pr = 6 * ir[i] + rr[i], pc = 6 * ic[j][e] + cc[j][e];
+          // entries above the diagonal of the child's block are not stored
+          if (ir[i] >= 0 && ic[j][e] >= 0 && pr >= pc) acc.c[i][j][e] -= Sc[pr + (long)pc * ldc];
+        }
+  }
   mma32(acc, ns, [&](int i, int kk) { return Q[ra[i] + (long)kk * m]; },
         [&](int i, int kk) { return Q[rb[i] + (long)kk * m]; });
-  const int mn = m / 6;
-  const int *lists = a.lists + d.lists;
-  gcdouble *Sc[2];
-  int ldc[2];
-#pragma unroll
-  for (int c = 0; c < 2; c++)
-    if (d.child[c] >= 0) {
-      const NdDev ch = a.all[d.child[c]];
-      ldc[c] = ch.m - ch.ns;
-      Sc[c] = (gcdouble *)(a.Sc + blockIdx.y * a.sSc + ch.S);
-    }
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     const int r = r0 + 16 * i + lr;
     if (r >= nb) continue;
-    const int rn = (ns + r) / 6, rr = r % 6;  // ns is a multiple of 6
-    int ir[2] = {-1, -1};
-#pragma unroll
-    for (int c = 0; c < 2; c++)
-      if (d.child[c] >= 0) ir[c] = lists[(1 + c) * mn + rn];
 #pragma unroll
     for (int j = 0; j < 2; j++)
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const int col = c0 + 16 * j + 4 * e + lk;
-        if (col > r) continue;
-        const int cn = (ns + col) / 6, cc = col % 6;
-        double v = 0.0;
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-          if (ir[c] < 0) continue;
-          const int ic = lists[(1 + c) * mn + cn];
-          if (ic >= 0) v += Sc[c][6 * ir[c] + rr + (long)(6 * ic + cc) * ldc[c]];
-        }
-        S[r + (long)col * nb] = v - acc.c[i][j][e];
+        if (col <= r) S[r + (long)col * nb] = -acc.c[i][j][e];
       }
   }
 }
@@ -948,8 +1048,15 @@ hipError_t nd_compute(NdFactor &F, int nnzb, const double *vals, const long *blk
         a.tc = tn;
         hipLaunchKernelGGL(nd_gather_kernel, dim3((unsigned)lv.nf * tm * tn, nd), dim3(256), 0, stream, a);
       }
+      // few fronts: the chain of pivot blocks bounds the level, and the update
+      // factors the next one; many: the updates' throughput does, and the
+      // registers of the pivot code would halve their occupancy (panels of a
+      // level of the 200 x 400 cylinder: 1 front 2,760 -> 1,870 us, 64 350 ->
+      // 314, 256 276 -> 268, 512 332 -> 344, 2,048 1,120 -> 1,445)
+      const bool ahead = (long)lv.nf * nd <= 256;
       for (a.k = 0; a.k < tn; a.k++) {
-        hipLaunchKernelGGL(nd_diag_kernel, dim3(lv.nf, nd), dim3(kDiagThreads), 0, stream, a, info + d0);
+        if (a.k == 0 || !ahead)
+          hipLaunchKernelGGL(nd_diag_kernel, dim3(lv.nf, nd), dim3(256), 0, stream, a, info + d0);
         // rows after block k of the tallest front (a front whose block k is
         // its last, of n < 64 pivots, has its boundary left)
         a.tr = std::max((lv.max_m - kB * (a.k + 1) + kB - 1) / kB, (lv.max_nb + kB - 1) / kB);
@@ -957,7 +1064,8 @@ hipError_t nd_compute(NdFactor &F, int nnzb, const double *vals, const long *blk
         if (a.tr + a.k > 0)
           hipLaunchKernelGGL(nd_scale_kernel, dim3((unsigned)lv.nf * (a.tr + a.k), nd), dim3(256), 0, stream, a);
         if (a.tr > 0)
-          hipLaunchKernelGGL(nd_update_kernel, dim3((unsigned)lv.nf * a.tr * a.tc, nd), dim3(256), 0, stream, a);
+          hipLaunchKernelGGL(ahead ? nd_update_kernel<true> : nd_update_kernel<false>,
+                             dim3((unsigned)lv.nf * a.tr * a.tc, nd), dim3(256), 0, stream, a, lv.nf, info + d0);
       }
       if (lv.max_nb > 0) {
         a.tr = (lv.max_nb + kB - 1) / kB;
