@@ -2,6 +2,7 @@
 // (host-side state shared by the translation units of the library).
 #pragma once
 
+#include <algorithm>
 #include <string>
 #include <utility>
 #include <vector>
@@ -31,8 +32,10 @@ struct shellgpu_ctx {
   // fit with the elements of most neighbours first (shellgpu_tune chooses)
   int coloring = 0;
   // compiled schedule of each element-kernel mode (launch_elem_kernel's
-  // variant; shellgpu_tune chooses) and the tuner's report
-  int elem_variant[32] = {0};
+  // variant) chosen by shellgpu_tune or shellgpu_set_elem_schedule, -1: by the
+  // launch's size; and the tuner's report
+  int elem_variant[32];
+  shellgpu_ctx() { std::fill(elem_variant, elem_variant + 32, -1); }
   std::string schedule;
 
   shellgpu::Material mat = shellgpu::make_material(70e9, 0.3, 2700.0, 0.0, 10.0);
