@@ -12,7 +12,10 @@
 #pragma once
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
+#include <future>
+#include <memory>
 #include <utility>
 #include <vector>
 
@@ -37,30 +40,43 @@ struct NdTree {
 class NdBuilder {
  public:
   NdBuilder(int nn, const int *rowp, const int *cols, const double *X, int leaf)
-      : nn_(nn), rowp_(rowp), cols_(cols), leaf_(leaf), where_(nn, -1), rank_(nn), dist_(nn), side_(nn) {
+      : nn_(nn), rowp_(rowp), cols_(cols), leaf_(leaf), where_(nn), rank_(nn), dist_(nn), side_(nn) {
+    for (auto &w : where_) w.store(-1, std::memory_order_relaxed);
     // the whole mesh along each coordinate; the sets below keep these orders
     // (a stable partition), so nothing is sorted again
-    for (int d = 0; d < 3; d++) {
-      std::vector<std::pair<double, int>> key(nn);
-      for (int i = 0; i < nn; i++) key[i] = {X[3 * i + d], i};
-      std::sort(key.begin(), key.end());
-      all_.along[d].resize(nn);
-      for (int i = 0; i < nn; i++) all_.along[d][i] = key[i].second;
-    }
+    all_.reset(new Part());
+    std::vector<std::future<void>> wait;
+    for (int d = 0; d < 3; d++)
+      wait.push_back(std::async(nn > kFork ? kThread : std::launch::deferred, [this, X, d] {
+        std::vector<std::pair<double, int>> key(nn_);
+        for (int i = 0; i < nn_; i++) key[i] = {X[3 * i + d], i};
+        std::sort(key.begin(), key.end());
+        all_->along[d].resize(nn_);
+        for (int i = 0; i < nn_; i++) all_->along[d][i] = key[i].second;
+      }));
+    for (auto &w : wait) w.get();
   }
 
   NdTree build() {
     t_.perm.clear();
     t_.pos.assign(nn_, -1);
-    cut(all_, 0);
+    cut(*all_, 0);
+    collect(*all_, 0);
     for (int p = 0; p < nn_; p++) t_.pos[t_.perm[p]] = p;
     symbolic();
     return std::move(t_);
   }
 
  private:
-  struct Set {
+  // sets of more nodes are cut on a thread of their own, 4 levels deep
+  static constexpr int kFork = 2000, kForkDepth = 4;
+  // a thread where the system has one to give, else in the caller's get()
+  static constexpr std::launch kThread = std::launch::async | std::launch::deferred;
+
+  struct Part {
     std::vector<int> along[3];  // the same nodes along the three coordinates
+    std::vector<int> sep;       // the separator, or a leaf's nodes
+    std::unique_ptr<Part> side[2];
   };
   struct Cut {
     double cost = -1.0;
@@ -71,41 +87,43 @@ class NdBuilder {
   int nn_;
   const int *rowp_, *cols_;
   int leaf_;
-  // by node: stamp of its set, rank in the sweep, BFS distance, side of the cut
-  std::vector<int> where_, rank_, dist_;
+  // by node: stamp of its set (neighbours of other sets, cut by other
+  // threads, are looked at too), rank in the sweep, BFS distance, side
+  std::vector<std::atomic<int>> where_;
+  std::vector<int> rank_, dist_;
   std::vector<signed char> side_;
-  std::vector<int> left_, right_;
-  int stamp_ = 0;
-  Set all_;
+  std::atomic<int> stamps_{0};
+  std::unique_ptr<Part> all_;
   NdTree t_;
 
-  // best cut of the current set (where_[] == stamp_) along an order
-  void sweep(const std::vector<int> &order, int which, Cut &best) {
+  bool in(int v, int stamp) const { return where_[v].load(std::memory_order_relaxed) == stamp; }
+
+  // best cut of a set along an order
+  void sweep(const std::vector<int> &order, int stamp, int which, Cut &best) {
     const int n = (int)order.size();
     for (int k = 0; k < n; k++) rank_[order[k]] = k;
-    left_.assign(n + 2, 0);
-    right_.assign(n + 2, 0);
+    std::vector<int> left(n + 2, 0), right(n + 2, 0);
     for (int k = 0; k < n; k++) {
       const int v = order[k];
       int lo = k, hi = k;
       for (int p = rowp_[v]; p < rowp_[v + 1]; p++) {
         const int w = cols_[p];
-        if (where_[w] != stamp_) continue;
+        if (!in(w, stamp)) continue;
         lo = std::min(lo, rank_[w]);
         hi = std::max(hi, rank_[w]);
       }
       // v is in the separator of cut c when it lies before (after) the cut
       // and has a neighbour after (before) it: k < c <= hi, lo < c <= k
-      left_[k + 1]++;
-      left_[hi + 1]--;
-      right_[lo + 1]++;
-      right_[k + 1]--;
+      left[k + 1]++;
+      left[hi + 1]--;
+      right[lo + 1]++;
+      right[k + 1]--;
     }
     const int c0 = std::max(1, (3 * n) / 10), c1 = std::min(n - 1, n - (3 * n) / 10);
     int l = 0, r = 0;
     for (int c = 1; c <= c1; c++) {
-      l += left_[c];
-      r += right_[c];
+      l += left[c];
+      r += right[c];
       if (c < c0) continue;
       const double b = 2.0 * c / n - 1.0, pen = 1.0 + 2.0 * b * b;
       for (int side = 0; side < 2; side++) {
@@ -115,32 +133,34 @@ class NdBuilder {
     }
   }
 
-  // cut the set; returns its front (children first), or -1 for an empty set
-  int cut(Set &set, int depth) {
+  // cut a set down to its leaves
+  void cut(Part &set, int depth) {
     const int n = (int)set.along[0].size();
-    if (n == 0) return -1;
-    if (n <= leaf_) return front(set.along[0], -1, -1, depth);
-    stamp_++;
-    for (int v : set.along[0]) where_[v] = stamp_;
+    if (n <= leaf_) {
+      set.sep.swap(set.along[0]);
+      return;
+    }
+    const int stamp = ++stamps_;
+    for (int v : set.along[0]) where_[v].store(stamp, std::memory_order_relaxed);
     Cut best;
-    for (int d = 0; d < 3; d++) sweep(set.along[d], d, best);
+    for (int d = 0; d < 3; d++) sweep(set.along[d], stamp, d, best);
     // breadth-first sweep where planes do not find the short lines of a
     // surface (coordinates that coincide or fold)
     std::vector<int> order;
     if (best.cost > 3.0 * std::sqrt((double)n)) {
-      bfs(set.along[0], order);
-      sweep(order, 3, best);
+      bfs(set.along[0], stamp, order);
+      sweep(order, stamp, 3, best);
     }
     const std::vector<int> &along = best.sweep == 3 ? order : set.along[best.sweep];
     for (int k = 0; k < n; k++) side_[along[k]] = k >= best.at;
     // the separator: nodes of one side with a neighbour on the other
-    std::vector<int> s;
+    std::vector<int> &s = set.sep;
     for (int k = 0; k < n; k++) {
       const int v = along[k];
       if ((k >= best.at) != best.right) continue;
       for (int p = rowp_[v]; p < rowp_[v + 1]; p++) {
         const int w = cols_[p];
-        if (where_[w] == stamp_ && (side_[w] & 1) != (int)best.right) {
+        if (in(w, stamp) && (side_[w] & 1) != (int)best.right) {
           s.push_back(v);
           break;
         }
@@ -149,21 +169,27 @@ class NdBuilder {
     // disconnected sides: any node keeps the tree binary
     if (s.empty()) s.push_back(along[best.right ? n - 1 : 0]);
     for (int v : s) side_[v] = 2 + (side_[v] & 1);
-    int id[2] = {-1, -1};
-    Set part[2];
+    for (auto &p : set.side) p.reset(new Part());
     for (int d = 0; d < 3; d++) {
-      for (int k = 0; k < 2; k++) part[k].along[d].reserve(n / 2 + 1);
+      for (auto &p : set.side) p->along[d].reserve(n / 2 + 1);
       for (int v : set.along[d])
-        if (side_[v] < 2) part[(int)side_[v]].along[d].push_back(v);
+        if (side_[v] < 2) set.side[(int)side_[v]]->along[d].push_back(v);
       std::vector<int>().swap(set.along[d]);
     }
     std::vector<int>().swap(order);
-    for (int k = 0; k < 2; k++) id[k] = cut(part[k], depth + 1);
-    return front(s, id[0], id[1], depth);
+    for (auto &p : set.side)
+      if (p->along[0].empty()) p.reset();
+    std::future<void> other;
+    if (n > kFork && depth < kForkDepth && set.side[0] && set.side[1])
+      other = std::async(kThread, [this, &set, depth] { cut(*set.side[0], depth + 1); });
+    else if (set.side[0])
+      cut(*set.side[0], depth + 1);
+    if (set.side[1]) cut(*set.side[1], depth + 1);
+    if (other.valid()) other.get();
   }
 
   // the set in breadth-first order from a far node (components one after another)
-  void bfs(const std::vector<int> &set, std::vector<int> &order) {
+  void bfs(const std::vector<int> &set, int stamp, std::vector<int> &order) {
     int start = set[0];
     for (int it = 0; it < 3; it++) {
       for (int v : set) dist_[v] = -1;
@@ -178,7 +204,7 @@ class NdBuilder {
           const int v = order[h];
           for (int p = rowp_[v]; p < rowp_[v + 1]; p++) {
             const int w = cols_[p];
-            if (where_[w] == stamp_ && dist_[w] < 0) {
+            if (in(w, stamp) && dist_[w] < 0) {
               dist_[w] = dist_[v] + 1;
               order.push_back(w);
             }
@@ -191,19 +217,26 @@ class NdBuilder {
     }
   }
 
-  int front(const std::vector<int> &nodes, int ca, int cb, int depth) {
+  // fronts and elimination order from the cut sets, children first
+  int collect(Part &set, int depth) {
+    int child[2] = {-1, -1};
+    for (int k = 0; k < 2; k++)
+      if (set.side[k]) {
+        child[k] = collect(*set.side[k], depth + 1);
+        set.side[k].reset();
+      }
+    if (child[0] < 0) std::swap(child[0], child[1]);
     NdFront f;
     f.j0 = (int)t_.perm.size();
-    f.ns = (int)nodes.size();
+    f.ns = (int)set.sep.size();
     f.depth = depth;
-    if (ca < 0) std::swap(ca, cb);
-    f.child[0] = ca;
-    f.child[1] = cb;
-    for (int v : nodes) t_.perm.push_back(v);
+    f.child[0] = child[0];
+    f.child[1] = child[1];
+    t_.perm.insert(t_.perm.end(), set.sep.begin(), set.sep.end());
     const int id = (int)t_.fronts.size();
-    if (ca >= 0) t_.fronts[ca].parent = id;
-    if (cb >= 0) t_.fronts[cb].parent = id;
-    t_.fronts.push_back(f);
+    for (int c : child)
+      if (c >= 0) t_.fronts[c].parent = id;
+    t_.fronts.push_back(std::move(f));
     t_.ndepth = std::max(t_.ndepth, depth + 1);
     return id;
   }
