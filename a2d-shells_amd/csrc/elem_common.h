@@ -88,8 +88,7 @@ __device__ __forceinline__ int field_slot(int f) {
   return f == kG11 ? 0 : (f == kG22 ? 3 : (f == kG12 ? 1 : (f == kG23 ? 4 : 2)));
 }
 
-// ---- 3x3 row-major algebra, generic in the scalar type S (double, or the
-// forward-mode Dual of dual.h for coordinate derivatives) ----
+// ---- 3x3 row-major algebra, generic in the scalar type S ----
 template <typename S>
 __device__ __forceinline__ void cross3(const S *a, const S *b, S *c) {
   c[0] = a[1] * b[2] - a[2] * b[1];

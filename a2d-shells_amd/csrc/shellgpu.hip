@@ -453,6 +453,28 @@ int run_colored(shellgpu_ctx *ctx, int mode, ElemArgs a) {
   return record_end(ctx, ctx->elem_ev);
 }
 
+// designs of one coordinate-derivative launch: as many as keep the element
+// gradients within 64 MiB (700,000 elements, many times what fills the GPU),
+// at least one
+static int xpt_designs(const shellgpu_ctx *ctx) {
+  const long n = (8L << 20) / (12L * ctx->nelems);
+  return (int)std::max(1L, std::min(n, (long)ctx->nbatch));
+}
+
+// the element gradients' buffer; sized with the designs, so that a
+// derivative call allocates nothing
+int reserve_xpt(shellgpu_ctx *ctx) {
+  const size_t need = 12L * ctx->nelems * xpt_designs(ctx);
+  if (need <= ctx->xg_doubles) return 0;
+  HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
+  if (ctx->d_xg) (void)hipFree(ctx->d_xg);
+  ctx->d_xg = nullptr;
+  ctx->xg_doubles = 0;
+  HIPCALL(ctx, hipMalloc((void **)&ctx->d_xg, sizeof(double) * need));
+  ctx->xg_doubles = need;
+  return 0;
+}
+
 int run_xpt(shellgpu_ctx *ctx, const double *phi, const double *u, const double *psi, const double *coef,
             int nonlin, int terms, double *dfdX) {
   XptArgs a{};
@@ -471,10 +493,20 @@ int run_xpt(shellgpu_ctx *ctx, const double *phi, const double *u, const double 
   a.dfdX = dfdX;
   a.dX_stride = 3L * ctx->nnodes;
   a.terms = terms;
-  for (int c = 0; c < ctx->ncolors; c++) {
-    a.elems = ctx->d_color_elems + ctx->h_color_ptr[c];
-    const int nb = ctx->h_color_ptr[c + 1] - ctx->h_color_ptr[c];
-    HIPCALL(ctx, launch_xpt_kernel(a, nb, ctx->nbatch, ctx->stream));
+  int rc = reserve_xpt(ctx);
+  if (rc) return rc;
+  const int nd = xpt_designs(ctx);
+  for (int d = 0; d < ctx->nbatch; d += nd) {
+    XptArgs b = a;
+    b.thick += (long)d * a.nelems;
+    if (b.temp) b.temp += (long)d * a.nelems;
+    if (b.phi) b.phi += d * a.stride;
+    if (b.u) b.u += d * a.stride;
+    if (b.psi) b.psi += d * a.stride;
+    b.coef += 4L * d;
+    b.dfdX += d * a.dX_stride;
+    HIPCALL(ctx, launch_xpt_kernel(b, ctx->nnodes, std::min(nd, ctx->nbatch - d), ctx->d_nptr, ctx->d_corner, ctx->d_xg,
+                                   ctx->stream));
   }
   return 0;
 }
@@ -513,7 +545,8 @@ void shellgpu_destroy(shellgpu_ctx *ctx) {
   (void)hipStreamSynchronize(ctx->stream);
   void *bufs[] = {ctx->d_conn, ctx->d_rowp,     ctx->d_cols,    ctx->d_blk, ctx->d_diag, ctx->d_tpos,
                   ctx->d_color_elems, ctx->d_X, ctx->d_bc_nodes, ctx->d_bc_mask,
-                  ctx->d_bc_vals, ctx->d_thick, ctx->d_temp, ctx->d_coef, ctx->d_first};
+                  ctx->d_bc_vals, ctx->d_thick, ctx->d_temp, ctx->d_coef, ctx->d_first,
+                  ctx->d_nptr, ctx->d_corner, ctx->d_xg};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   drop_events(ctx->elem_ev);
@@ -576,16 +609,15 @@ int shellgpu_set_mesh(shellgpu_ctx *ctx, int nnodes, int nelems, const int *conn
   for (int e = 0; e < nelems; e++)
     for (int k = 0; k < 4; k++) nep[conn[4 * e + k] + 1]++;
   for (int i = 0; i < nnodes; i++) nep[i + 1] += nep[i];
-  std::vector<int> n2e(nep[nnodes]), fill(nep.begin(), nep.end() - 1);
-  for (int e = 0; e < nelems; e++)
-    for (int k = 0; k < 4; k++) n2e[fill[conn[4 * e + k]]++] = e;
+  std::vector<int> n2c(nep[nnodes]), fill(nep.begin(), nep.end() - 1);
+  for (int c = 0; c < 4 * nelems; c++) n2c[fill[conn[c]]++] = c;
   ctx->h_rowp.assign(nnodes + 1, 0);
   ctx->h_cols.clear();
   std::vector<int> row;
   for (int i = 0; i < nnodes; i++) {
     row.clear();
     for (int p = nep[i]; p < nep[i + 1]; p++)
-      for (int k = 0; k < 4; k++) row.push_back(conn[4 * n2e[p] + k]);
+      for (int k = 0; k < 4; k++) row.push_back(conn[(n2c[p] & ~3) + k]);
     std::sort(row.begin(), row.end());
     row.erase(std::unique(row.begin(), row.end()), row.end());
     ctx->h_cols.insert(ctx->h_cols.end(), row.begin(), row.end());
@@ -621,6 +653,8 @@ int shellgpu_set_mesh(shellgpu_ctx *ctx, int nnodes, int nelems, const int *conn
   if (rc) return rc;
   if ((rc = upload(ctx, &ctx->d_conn, conn, 4L * nelems))) return rc;
   if ((rc = upload(ctx, &ctx->d_X, Xpts, 3L * nnodes))) return rc;
+  if ((rc = upload(ctx, &ctx->d_nptr, nep.data(), nep.size()))) return rc;
+  if ((rc = upload(ctx, &ctx->d_corner, n2c.data(), n2c.size()))) return rc;
   if ((rc = upload(ctx, &ctx->d_rowp, ctx->h_rowp.data(), ctx->h_rowp.size()))) return rc;
   if ((rc = upload(ctx, &ctx->d_cols, ctx->h_cols.data(), ctx->h_cols.size()))) return rc;
   if ((rc = upload(ctx, &ctx->d_blk, ctx->h_blk.data(), ctx->h_blk.size()))) return rc;
@@ -690,7 +724,7 @@ int shellgpu_set_designs(shellgpu_ctx *ctx, int nbatch, const double *thick, con
   if (ctx->d_coef) (void)hipFree(ctx->d_coef);
   ctx->d_coef = nullptr;
   HIPCALL(ctx, hipMalloc((void **)&ctx->d_coef, sizeof(double) * 4 * nbatch));
-  return 0;
+  return reserve_xpt(ctx);
 }
 
 int shellgpu_get_sizes(shellgpu_ctx *ctx, int *nnodes, int *nelems, int *nnzb, int *ncolors, int *nbatch) {

@@ -27,6 +27,9 @@ struct shellgpu_ctx {
   // repeats a node (two of its blocks coincide)
   int *d_first = nullptr;
   double *d_X = nullptr;
+  // per node n the places 4 element + corner where it stands, in element
+  // order: d_corner[d_nptr[n]..d_nptr[n + 1])
+  int *d_nptr = nullptr, *d_corner = nullptr;
 
   // element colouring: 0 greedy first fit in element order, 1 greedy first
   // fit with the elements of most neighbours first (shellgpu_tune chooses)
@@ -48,6 +51,10 @@ struct shellgpu_ctx {
   double *d_thick = nullptr, *d_temp = nullptr;
   bool same_designs = false;  // every design has the same thickness and temperature
   double *d_coef = nullptr;  // 4 * nbatch per-design kernel coefficients
+  // element gradients of run_xpt, 12 doubles per element for as many designs
+  // as xpt_designs() allows at a time
+  double *d_xg = nullptr;
+  size_t xg_doubles = 0;
   // timing
   bool timing = false;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> elem_ev, spmv_ev;
@@ -81,7 +88,7 @@ ElemArgs base_args(shellgpu_ctx *ctx, const double *u);
 // launch one element-kernel mode colour by colour (no two elements of a
 // launch share a node, so scatters need no atomics)
 int run_colored(shellgpu_ctx *ctx, int mode, ElemArgs a);
-// coordinate-derivative kernel over all colours; coef (device, 4 per
+// coordinate-derivative kernel over all elements; coef (device, 4 per
 // design), vectors with stride 6*nnodes, dfdX with stride 3*nnodes
 int run_xpt(shellgpu_ctx *ctx, const double *phi, const double *u, const double *psi, const double *coef,
             int nonlin, int terms, double *dfdX);

@@ -133,7 +133,6 @@ __host__ __device__ inline Section make_section_dt(const Material &m, double t) 
 // vectors and bilinear pairs those need.
 enum { kXptK = 1, kXptG = 2, kXptR = 4, kXptM = 8 };
 struct XptArgs {
-  const int *elems;
   const int *conn;
   const double *Xpts;
   const double *thick;
@@ -148,7 +147,10 @@ struct XptArgs {
   long dX_stride;
   int terms;
 };
-hipError_t launch_xpt_kernel(const XptArgs &args, int nel, int nbatch, hipStream_t stream);
+// work: 12 doubles per element and design; node_corner[node_ptr[n]..] lists
+// the places 4 element + corner of node n
+hipError_t launch_xpt_kernel(const XptArgs &args, int nnodes, int nbatch, const int *node_ptr, const int *node_corner,
+                             double *work, hipStream_t stream);
 
 // variant: the compiled schedule of the matrix modes (kModeKLin, kModeKNl,
 // kModeG, kModeJac*): bit 0 reads the BSR blocks at the scatter (default:

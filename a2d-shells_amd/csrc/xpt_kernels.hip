@@ -6,9 +6,9 @@
 // The reference differentiates these products with respect to Xpts by
 // central differences (TACSElement::addMatXptSensInnerProduct and
 // addAdjResXptProduct, src/elements/TACSElement.cpp:270-332, 434-507,
-// dh = 1e-7).  Here they are exact: one thread per (element, coordinate)
-// evaluates the scalars in forward-mode dual numbers seeded on that
-// coordinate.  The scalars are written through strains only,
+// dh = 1e-7).  Here they are exact, by the adjoint of the strain evaluation:
+// one backward sweep gives all 12 coordinates of an element.  The scalars are
+// written through strains only,
 //
 //   e(q) = e1(q) + Q(q, q) / 2           (Q symmetric bilinear)
 //   s_K = sum_qp det e1(phi)^T C e1(phi)
@@ -29,415 +29,696 @@
 // strains (TACSShellElementModel.h:32-77, 643-697) interpolated and
 // transformed at the quadrature points, bending strains from the
 // displacement gradients (TACSShellUtilities.h:361-422) and the natural
-// transform with its un-orthogonalised in-plane axis.  Elements run colour
-// by colour, so the 12 threads of an element add into distinct coordinates
-// and no two elements of a launch share a node.
-#include "dual.h"
+// transform with its un-orthogonalised in-plane axis.
+//
+// Four lanes share an element: lane p takes node p, quadrature point p and
+// the tying points p, p + 4, p + 8, and they exchange normals, tying strains
+// and their adjoints through LDS.  The element gradients go to a buffer and a
+// second kernel adds them up per node, in element order, so all elements run
+// in one launch whatever the colouring (a colour of a 20,000-element mesh has
+// too few wavefronts to fill the GPU).
+//
+// Bound by the registers: the strains of two vectors and two pairs with their
+// adjoints hold all 512 of a lane, one wavefront per SIMD.  Against one lane
+// per (element, coordinate) in forward-mode dual numbers, which evaluated
+// every strain 12 times: s_G + s_K of 19,691 elements 6 x 246 us -> 45 us,
+// s_R 34, s_K 25, and 4.5 us for the sums per node; a lane per element would
+// need four times the registers and leave three quarters of the GPU idle.
 #include "elem_common.h"
 #include "shellgpu_internal.h"
 
 namespace shellgpu {
 namespace {
 
-constexpr int kThreads = 192;  // 16 elements x 12 coordinates
+constexpr int kElems = 32;  // per workgroup of 128 threads
 
-template <typename S>
-__device__ __forceinline__ void apply_cs(const Section &c, const S &w, const S b[9], S y[9]) {
-  y[0] = w * (c.A[0] * b[0] + c.A[1] * b[1] + c.A[2] * b[2]);
-  y[1] = w * (c.A[1] * b[0] + c.A[3] * b[1] + c.A[4] * b[2]);
-  y[2] = w * (c.A[2] * b[0] + c.A[4] * b[1] + c.A[5] * b[2]);
-  y[3] = w * (c.D[0] * b[3] + c.D[1] * b[4] + c.D[2] * b[5]);
-  y[4] = w * (c.D[1] * b[3] + c.D[3] * b[4] + c.D[4] * b[5]);
-  y[5] = w * (c.D[2] * b[3] + c.D[4] * b[4] + c.D[5] * b[5]);
-  y[6] = w * (c.As[0] * b[6] + c.As[1] * b[7]);
-  y[7] = w * (c.As[1] * b[6] + c.As[2] * b[7]);
-  y[8] = w * (c.drill * b[8]);
+struct V3 {
+  double x, y, z;
+};
+__device__ __forceinline__ V3 operator+(V3 a, V3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
+__device__ __forceinline__ V3 operator-(V3 a, V3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
+__device__ __forceinline__ V3 operator*(double s, V3 a) { return {s * a.x, s * a.y, s * a.z}; }
+__device__ __forceinline__ V3 &operator+=(V3 &a, V3 b) { return a = a + b; }
+__device__ __forceinline__ double dot(V3 a, V3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+__device__ __forceinline__ V3 cross(V3 a, V3 b) {
+  return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
+__device__ __forceinline__ V3 load3(const double *p) { return {p[0], p[1], p[2]}; }
+__device__ __forceinline__ V3 zero3() { return {0.0, 0.0, 0.0}; }
+// a x_0 + b x_1 + c x_2 of a triple of vectors
+__device__ __forceinline__ V3 comb(V3 x, V3 a, V3 b, V3 c) { return x.x * a + x.y * b + x.z * c; }
 
-template <typename S>
-__device__ __forceinline__ S dot9(const S a[9], const S b[9]) {
-  S s = a[0] * b[0];
+// natural transform (elem_common.h) of the surface direction a and the normal
+// n0: T = [t1 t2 n], and its adjoint
+struct Frame {
+  V3 T[3];
+  double iv, in, d;
+  __device__ __forceinline__ void set(V3 a, V3 n0) {
+    in = 1.0 / sqrt(dot(n0, n0));
+    const V3 n = in * n0;
+    d = dot(n, a);
+    V3 v = a;
+    v.x = a.x - d * n.x;
+    v.x = v.x - d * n.x;
+    v.x = v.x - d * n.x;
+    iv = 1.0 / sqrt(dot(v, v));
+    T[0] = iv * v;
+    T[1] = cross(n, T[0]);
+    T[2] = n;
+  }
+  __device__ __forceinline__ void adjoint(V3 a, const V3 Tb[3], V3 &ab, V3 &n0b) const {
+    const V3 n = T[2], t1 = T[0];
+    V3 nb = Tb[2] + cross(t1, Tb[1]);
+    const V3 t1b = Tb[0] + cross(Tb[1], n);
+    const V3 vb = iv * (t1b - dot(t1, t1b) * t1);
+    const double db = -3.0 * n.x * vb.x;
+    nb.x -= 3.0 * d * vb.x;
+    nb += db * a;
+    ab += vb + db * n;
+    n0b += in * (nb - dot(n, nb) * n);
+  }
+};
+
+// inverse of [a b c]: rows r, determinant; and the adjoint: Gi[i] is the
+// adjoint of row i
+struct Inverse {
+  V3 r[3];
+  double det;
+  __device__ __forceinline__ void set(V3 a, V3 b, V3 c) {
+    const V3 bc = cross(b, c);
+    det = dot(a, bc);
+    const double i = 1.0 / det;
+    r[0] = i * bc;
+    r[1] = i * cross(c, a);
+    r[2] = i * cross(a, b);
+  }
+  __device__ __forceinline__ V3 mul(V3 v) const { return {dot(r[0], v), dot(r[1], v), dot(r[2], v)}; }
+  __device__ __forceinline__ V3 mul_t(V3 v) const { return comb(v, r[0], r[1], r[2]); }
+  __device__ __forceinline__ V3 column(int l, const V3 Gi[3], double detb) const {
+    return (detb * det) * r[l] - comb({dot(Gi[0], r[l]), dot(Gi[1], r[l]), dot(Gi[2], r[l])}, r[0], r[1], r[2]);
+  }
+};
+
+__device__ __forceinline__ void apply_c(const Section &c, const double b[9], double y[9]) {
+  y[0] = c.A[0] * b[0] + c.A[1] * b[1] + c.A[2] * b[2];
+  y[1] = c.A[1] * b[0] + c.A[3] * b[1] + c.A[4] * b[2];
+  y[2] = c.A[2] * b[0] + c.A[4] * b[1] + c.A[5] * b[2];
+  y[3] = c.D[0] * b[3] + c.D[1] * b[4] + c.D[2] * b[5];
+  y[4] = c.D[1] * b[3] + c.D[3] * b[4] + c.D[4] * b[5];
+  y[5] = c.D[2] * b[3] + c.D[4] * b[4] + c.D[5] * b[5];
+  y[6] = c.As[0] * b[6] + c.As[1] * b[7];
+  y[7] = c.As[1] * b[6] + c.As[2] * b[7];
+  y[8] = c.drill * b[8];
+}
+__device__ __forceinline__ double dot9(const double a[9], const double b[9]) {
+  double s = a[0] * b[0];
 #pragma unroll
-  for (int i = 1; i < 9; i++) s = s + a[i] * b[i];
+  for (int i = 1; i < 9; i++) s += a[i] * b[i];
   return s;
-}
-
-// linear tying strain of a field: U = interleaved xi/eta displacement
-// gradient, d0 = director, X = interleaved xi/eta coordinate gradient,
-// n0 = interpolated normal (TACSShellElementModel.h:32-77)
-template <typename S>
-__device__ __forceinline__ S tying_lin(int f, const S U[6], const S d0[3], const S X[6], const S n0[3]) {
-  if (f == kG11) return U[0] * X[0] + U[2] * X[2] + U[4] * X[4];
-  if (f == kG22) return U[1] * X[1] + U[3] * X[3] + U[5] * X[5];
-  if (f == kG12)
-    return 0.5 * (U[0] * X[1] + U[2] * X[3] + U[4] * X[5] + U[1] * X[0] + U[3] * X[2] + U[5] * X[4]);
-  if (f == kG23) return 0.5 * (X[1] * d0[0] + X[3] * d0[1] + X[5] * d0[2] + n0[0] * U[1] + n0[1] * U[3] + n0[2] * U[5]);
-  return 0.5 * (X[0] * d0[0] + X[2] * d0[1] + X[4] * d0[2] + n0[0] * U[0] + n0[1] * U[2] + n0[2] * U[4]);
-}
-
-// symmetric bilinear form of the quadratic tying terms
-// (TACSShellElementModel.h:643-697): the nonlinear tying strain is
-// lin(q) + Q(q, q) / 2
-template <typename S>
-__device__ __forceinline__ S tying_quad(int f, const S Ua[6], const S da[3], const S Ub[6], const S db[3]) {
-  if (f == kG11) return Ua[0] * Ub[0] + Ua[2] * Ub[2] + Ua[4] * Ub[4];
-  if (f == kG22) return Ua[1] * Ub[1] + Ua[3] * Ub[3] + Ua[5] * Ub[5];
-  if (f == kG12)
-    return 0.5 * (Ua[0] * Ub[1] + Ua[2] * Ub[3] + Ua[4] * Ub[5] + Ub[0] * Ua[1] + Ub[2] * Ua[3] + Ub[4] * Ua[5]);
-  if (f == kG23)
-    return 0.5 * (da[0] * Ub[1] + da[1] * Ub[3] + da[2] * Ub[5] + db[0] * Ua[1] + db[1] * Ua[3] + db[2] * Ua[5]);
-  return 0.5 * (da[0] * Ub[0] + da[1] * Ub[2] + da[2] * Ub[4] + db[0] * Ua[0] + db[1] * Ua[2] + db[2] * Ua[4]);
 }
 
 // vectors: 0 phi, 1 u, 2 psi; bilinear pairs (u,phi), (phi,phi), (u,psi), (u,u)
 constexpr int kPairA[4] = {1, 0, 1, 1};
 constexpr int kPairB[4] = {0, 0, 2, 1};
+constexpr int bits(int m) { return (m & 1) + ((m >> 1) & 1) + ((m >> 2) & 1) + ((m >> 3) & 1); }
 
-// tying strains of the needed vectors and pairs at tying point t
-// (TACSShellElementModel.h:32-77 linear, :643-697 quadratic)
-template <typename S, int WM, int PM>
-__device__ __forceinline__ void tying_at(int t, const S X[12], const S fn[12], const double q[3][24], S tl[3],
-                                         S tq[4]) {
-  double u, v, N[4], Na[4], Nb[4];
-  tying_point(t, u, v);
-  shape4(u, v, N, Na, Nb);
-  S Xxi[6], n0[3] = {0.0, 0.0, 0.0};
-  for (int i = 0; i < 6; i++) Xxi[i] = 0.0;
-  for (int m = 0; m < 4; m++)
-    for (int d = 0; d < 3; d++) {
-      Xxi[2 * d] = Xxi[2 * d] + Na[m] * X[3 * m + d];
-      Xxi[2 * d + 1] = Xxi[2 * d + 1] + Nb[m] * X[3 * m + d];
-      n0[d] = n0[d] + N[m] * fn[3 * m + d];
-    }
-  S U[3][6], d0[3][3];
-  for (int w = 0; w < 3; w++) {
-    if (!((WM >> w) & 1)) continue;
-    for (int i = 0; i < 6; i++) U[w][i] = 0.0;
-    for (int i = 0; i < 3; i++) d0[w][i] = 0.0;
-    for (int m = 0; m < 4; m++) {
-      const S qr[3] = {q[w][6 * m + 3], q[w][6 * m + 4], q[w][6 * m + 5]};
-      S dm[3];
-      cross3(qr, &fn[3 * m], dm);
-      for (int d = 0; d < 3; d++) {
-        d0[w][d] = d0[w][d] + N[m] * dm[d];
-        U[w][2 * d] = U[w][2 * d] + Na[m] * q[w][6 * m + d];
-        U[w][2 * d + 1] = U[w][2 * d + 1] + Nb[m] * q[w][6 * m + d];
-      }
-    }
-  }
-  const int f = tying_field(t);
-  for (int w = 0; w < 3; w++)
-    if ((WM >> w) & 1) tl[w] = tying_lin(f, U[w], d0[w], Xxi, n0);
-  for (int p = 0; p < 4; p++)
-    if ((PM >> p) & 1) tq[p] = tying_quad(f, U[kPairA[p]], d0[kPairA[p]], U[kPairB[p]], d0[kPairB[p]]);
-}
+// LDS of one element.  The sources of tying strains are the vectors of WM,
+// then the pairs of PM.
+template <int WM, int PM>
+struct XptSmem {
+  static constexpr int kNw = bits(WM), kNs = kNw + bits(PM);
+  double q[kNw][24];
+  double fn[12];
+  union {
+    struct {
+      double et[kNw][4];   // drilling strains at the nodes
+      double ty[kNs][9];   // tying strains
+    } f;
+    struct {
+      double g[4][kNs][5];  // per quadrature point, adjoints of the tying fields
+      double e8[4][kNw];    // and of the drilling strain
+    } b;
+    double part[4][12];     // per lane, adjoints of the normals, then of the coordinates
+  };
+};
 
 // WM: the vectors a variant evaluates (bit w), PM: the pairs (bit p).  Each
 // scalar needs: s_K and s_M phi; s_G phi, u and the pairs (u,phi),
 // (phi,phi); s_R u, psi and, for the nonlinear model, (u,psi), (u,u).
-// Vectors and pairs outside the masks are never formed, which keeps the
-// dual-number strains of a variant in registers.
-template <typename S, int WM, int PM>
-__device__ void element_scalars(const S X[12], const double q[3][24], const Section &sec, double eth, bool nonlin,
-                                const double c[4], double m0, double m2, S &out) {
+// Vectors and pairs outside the masks are never formed.
+template <int WM, int PM>
+__global__ __launch_bounds__(4 * kElems) void xpt_kernel(XptArgs a, double *out) {
+  using SM = XptSmem<WM, PM>;
+  constexpr int NW = SM::kNw, NS = SM::kNs;
   constexpr bool kPhi = WM & 1, kU = (WM >> 1) & 1, kPsi = (WM >> 2) & 1;
   constexpr bool kGeo = kPhi && kU && (PM & 3) == 3;
   constexpr bool kRes = kU && kPsi;
   constexpr bool kResNl = kRes && (PM & 12) == 12;
-  // ---- node normals ----
-  S fn[12];
-  for (int n = 0; n < 4; n++) {
-    double u, v, N[4], Na[4], Nb[4];
-    node_point(n, u, v);
-    shape4(u, v, N, Na, Nb);
-    S a3[3] = {0.0, 0.0, 0.0}, b3[3] = {0.0, 0.0, 0.0};
-    for (int m = 0; m < 4; m++)
-      for (int d = 0; d < 3; d++) {
-        a3[d] = a3[d] + Na[m] * X[3 * m + d];
-        b3[d] = b3[d] + Nb[m] * X[3 * m + d];
-      }
-    S f[3];
-    cross3(a3, b3, f);
-    const S nrm = sqrt(dot3(f, f));
-    if (value(nrm) != 0.0) {
-      const S inv = 1.0 / nrm;
-      f[0] = f[0] * inv;
-      f[1] = f[1] * inv;
-      f[2] = f[2] * inv;
-    }
-    fn[3 * n] = f[0];
-    fn[3 * n + 1] = f[1];
-    fn[3 * n + 2] = f[2];
-  }
-  // ---- drilling strain at the nodes (TacsShellComputeDrillStrain with
-  // TACSLinearizedRotation: et = 0.5 (Ct[3] + u0x[3] - Ct[1] - u0x[1])) ----
-  S etn[3][4];
-  for (int n = 0; n < 4; n++) {
-    double u, v, N[4], Na[4], Nb[4];
-    node_point(n, u, v);
-    shape4(u, v, N, Na, Nb);
-    S Xxi[6];
-    for (int i = 0; i < 6; i++) Xxi[i] = 0.0;
-    for (int m = 0; m < 4; m++)
-      for (int d = 0; d < 3; d++) {
-        Xxi[2 * d] = Xxi[2 * d] + Na[m] * X[3 * m + d];
-        Xxi[2 * d + 1] = Xxi[2 * d + 1] + Nb[m] * X[3 * m + d];
-      }
-    S Tn[9], Xd[9], Xdi[9], XTn[9];
-    natural_transform(Xxi, &fn[3 * n], Tn);
-    frame3(Xxi, &fn[3 * n], Xd);
-    inv3(Xd, Xdi);
-    mm3(Xdi, Tn, XTn);
-    // dC = Tn dA Tn^T, du0d = Tn dA XTn^T with dA = d et / d(Ct or u0x)
-    const double dA[9] = {0, -0.5, 0, 0.5, 0, 0, 0, 0, 0};
-    S tmp[9], dC[9], du0d[9];
-    for (int i = 0; i < 3; i++)
-      for (int j = 0; j < 3; j++)
-        tmp[3 * i + j] = dA[3 * i] * Tn[3 * j] + dA[3 * i + 1] * Tn[3 * j + 1] + dA[3 * i + 2] * Tn[3 * j + 2];
-    mm3(Tn, tmp, dC);
-    for (int i = 0; i < 3; i++)
-      for (int j = 0; j < 3; j++)
-        tmp[3 * i + j] = dA[3 * i] * XTn[3 * j] + dA[3 * i + 1] * XTn[3 * j + 1] + dA[3 * i + 2] * XTn[3 * j + 2];
-    mm3(Tn, tmp, du0d);
-    const S rot[3] = {dC[5] - dC[7], dC[6] - dC[2], dC[1] - dC[3]};
-    const S g[6] = {du0d[0], du0d[1], du0d[3], du0d[4], du0d[6], du0d[7]};
-    for (int w = 0; w < 3; w++) {
-      if (!((WM >> w) & 1)) continue;
-      S et = rot[0] * q[w][6 * n + 3] + rot[1] * q[w][6 * n + 4] + rot[2] * q[w][6 * n + 5];
-      for (int m = 0; m < 4; m++)
-        for (int d = 0; d < 3; d++) et = et + (Na[m] * g[2 * d] + Nb[m] * g[2 * d + 1]) * q[w][6 * m + d];
-      etn[w][n] = et;
-    }
-  }
-  // ---- tying strains: linear parts of the vectors and the bilinear
-  // quadratic terms of the pairs.  Variants with pairs evaluate them again at
-  // every quadrature point instead of holding 9 points' worth of dual
-  // numbers through the quadrature loop (which spilled to scratch memory) ----
-  constexpr bool kLate = PM != 0;
-  S tyl[3][kLate ? 1 : 9];
-  if constexpr (!kLate) {
-    for (int t = 0; t < 9; t++) {
-      S tl[3], tq[4];
-      tying_at<S, WM, PM>(t, X, fn, q, tl, tq);
-      for (int w = 0; w < 3; w++)
-        if ((WM >> w) & 1) tyl[w][t] = tl[w];
-    }
-  }
-  // ---- quadrature points ----
-  S acc = 0.0;
-  // rolled: an unrolled loop keeps four points' dual numbers live at once
-#pragma unroll 1
-  for (int iq = 0; iq < 4; iq++) {
-    double u, v, N[4], Na[4], Nb[4];
-    quad_point(iq, u, v);
-    shape4(u, v, N, Na, Nb);
-    S Xxi[6], nxi[6], n0[3] = {0.0, 0.0, 0.0};
-    for (int i = 0; i < 6; i++) Xxi[i] = nxi[i] = 0.0;
-    for (int m = 0; m < 4; m++)
-      for (int d = 0; d < 3; d++) {
-        Xxi[2 * d] = Xxi[2 * d] + Na[m] * X[3 * m + d];
-        Xxi[2 * d + 1] = Xxi[2 * d + 1] + Nb[m] * X[3 * m + d];
-        nxi[2 * d] = nxi[2 * d] + Na[m] * fn[3 * m + d];
-        nxi[2 * d + 1] = nxi[2 * d + 1] + Nb[m] * fn[3 * m + d];
-        n0[d] = n0[d] + N[m] * fn[3 * m + d];
-      }
-    S T[9], Xd[9], Xdz[9], Xdi[9], XT[9], nXdz[9], XzT[9];
-    natural_transform(Xxi, n0, T);
-    frame3(Xxi, n0, Xd);
-    frame3z(nxi, Xdz);
-    const S det = inv3(Xd, Xdi);
-    mm3(Xdi, Xdz, nXdz);
-    for (int i = 0; i < 9; i++) nXdz[i] = -nXdz[i];
-    mm3(Xdi, T, XT);
-    mm3(nXdz, XT, XzT);
-    // displacement gradients u0x, u1x of the three vectors
-    S U0[3][9], U1[3][9];
-    for (int w = 0; w < 3; w++) {
-      if (!((WM >> w) & 1)) continue;
-      S d0[3] = {0.0, 0.0, 0.0}, d0xi[6], u0xi[6];
-      for (int i = 0; i < 6; i++) d0xi[i] = u0xi[i] = 0.0;
-      for (int m = 0; m < 4; m++) {
-        const S qr[3] = {q[w][6 * m + 3], q[w][6 * m + 4], q[w][6 * m + 5]};
-        S dm[3];
-        cross3(qr, &fn[3 * m], dm);
-        for (int d = 0; d < 3; d++) {
-          d0[d] = d0[d] + N[m] * dm[d];
-          d0xi[2 * d] = d0xi[2 * d] + Na[m] * dm[d];
-          d0xi[2 * d + 1] = d0xi[2 * d + 1] + Nb[m] * dm[d];
-          u0xi[2 * d] = u0xi[2 * d] + Na[m] * q[w][6 * m + d];
-          u0xi[2 * d + 1] = u0xi[2 * d + 1] + Nb[m] * q[w][6 * m + d];
-        }
-      }
-      S u0d[9], u1d[9], tmp[9], tmp2[9];
-      frame3(u0xi, d0, u0d);
-      frame3z(d0xi, u1d);
-      mm3(u1d, XT, tmp);
-      mm3(u0d, XzT, tmp2);
-      for (int i = 0; i < 9; i++) tmp[i] = tmp[i] + tmp2[i];
-      mtm3(T, tmp, U1[w]);
-      mm3(u0d, XT, tmp);
-      mtm3(T, tmp, U0[w]);
-    }
-    // strains: e1 of the vectors, Q of the pairs
-    S e1[3][9], eq[4][9];
-    double Nt[9];
-    tying_interp(u, v, Nt);
-    const int kk[5] = {0, 3, 1, 4, 2};
-    const double ff[5] = {1.0, 1.0, 2.0, 2.0, 2.0};
-    const int pa[5] = {0, 0, 0, 1, 1}, pb[5] = {0, 1, 2, 1, 2};
-    S al[5][3], aq[5][4];
-    for (int r = 0; r < 5; r++) {
-      for (int w = 0; w < 3; w++) al[r][w] = 0.0;
-      for (int p = 0; p < 4; p++) aq[r][p] = 0.0;
-    }
-    for (int t = 0; t < 9; t++) {
-      S tl[3], tq[4];
-      if constexpr (kLate) {
-        tying_at<S, WM, PM>(t, X, fn, q, tl, tq);
-      } else {
-        for (int w = 0; w < 3; w++)
-          if ((WM >> w) & 1) tl[w] = tyl[w][t];
-      }
-      const int sl = field_slot(tying_field(t));
-      const int cc = pa[sl], dd = pb[sl];
-      for (int r = 0; r < 5; r++) {
-        const int ka = pa[kk[r]], kb = pb[kk[r]];
-        const S M = (cc == dd) ? XT[3 * cc + ka] * XT[3 * cc + kb]
-                               : XT[3 * cc + ka] * XT[3 * dd + kb] + XT[3 * dd + ka] * XT[3 * cc + kb];
-        const S W = (ff[r] * Nt[t]) * M;
-        for (int w = 0; w < 3; w++)
-          if ((WM >> w) & 1) al[r][w] = al[r][w] + W * tl[w];
-        for (int p = 0; p < 4; p++)
-          if ((PM >> p) & 1) aq[r][p] = aq[r][p] + W * tq[p];
-      }
-    }
-    for (int r = 0; r < 5; r++) {
-      const int row = r < 3 ? r : (r == 3 ? 6 : 7);
-      for (int w = 0; w < 3; w++)
-        if ((WM >> w) & 1) e1[w][row] = al[r][w];
-      for (int p = 0; p < 4; p++)
-        if ((PM >> p) & 1) eq[p][row] = aq[r][p];
-    }
-    for (int w = 0; w < 3; w++) {
-      if (!((WM >> w) & 1)) continue;
-      e1[w][3] = U1[w][0];
-      e1[w][4] = U1[w][4];
-      e1[w][5] = U1[w][1] + U1[w][3];
-      e1[w][8] = N[0] * etn[w][0] + N[1] * etn[w][1] + N[2] * etn[w][2] + N[3] * etn[w][3];
-    }
-    for (int p = 0; p < 4; p++) {
-      if (!((PM >> p) & 1)) continue;
-      const S *A0 = U0[kPairA[p]], *A1 = U1[kPairA[p]], *B0 = U0[kPairB[p]], *B1 = U1[kPairB[p]];
-      eq[p][3] = A0[0] * B1[0] + A0[3] * B1[3] + A0[6] * B1[6] + B0[0] * A1[0] + B0[3] * A1[3] + B0[6] * A1[6];
-      eq[p][4] = A0[1] * B1[1] + A0[4] * B1[4] + A0[7] * B1[7] + B0[1] * A1[1] + B0[4] * A1[4] + B0[7] * A1[7];
-      eq[p][5] = A0[0] * B1[1] + A0[3] * B1[4] + A0[6] * B1[7] + A1[0] * B0[1] + A1[3] * B0[4] + A1[6] * B0[7] +
-                 B0[0] * A1[1] + B0[3] * A1[4] + B0[6] * A1[7] + B1[0] * A0[1] + B1[3] * A0[4] + B1[6] * A0[7];
-      eq[p][8] = 0.0;
-    }
-    // mechanical strain of the path (u = 0 where u is not evaluated)
-    S eu[9];
-    for (int i = 0; i < 9; i++) {
-      if constexpr (kU)
-        eu[i] = e1[1][i];
-      else
-        eu[i] = 0.0;
-    }
-    eu[0] = eu[0] - eth;
-    eu[1] = eu[1] - eth;
-    S y[9];
-    if (kPhi && (c[0] != 0.0 || c[1] != 0.0)) {
-      apply_cs(sec, det, e1[0], y);  // det C e1(phi)
-      if (c[0] != 0.0) acc = acc + c[0] * dot9(e1[0], y);
-      if constexpr (kGeo) {
-        if (c[1] != 0.0) {
-          S z[9];
-          apply_cs(sec, det, eq[1], z);  // det C Q(phi, phi)
-          acc = acc + c[1] * (2.0 * dot9(eq[0], y) + dot9(eu, z));
-        }
-      }
-    }
-    if (kPhi && c[3] != 0.0) {
-      S u0[3] = {0.0, 0.0, 0.0}, d0[3] = {0.0, 0.0, 0.0};
-      for (int m = 0; m < 4; m++) {
-        const S qr[3] = {q[0][6 * m + 3], q[0][6 * m + 4], q[0][6 * m + 5]};
-        S dm[3];
-        cross3(qr, &fn[3 * m], dm);
-        for (int d = 0; d < 3; d++) {
-          u0[d] = u0[d] + N[m] * q[0][6 * m + d];
-          d0[d] = d0[d] + N[m] * dm[d];
-        }
-      }
-      acc = acc + c[3] * det * (m0 * dot3(u0, u0) + m2 * dot3(d0, d0));
-    }
-    if constexpr (kRes) {
-      if (c[2] != 0.0) {
-        S ep[9];
-        for (int i = 0; i < 9; i++) ep[i] = e1[2][i];
-        if constexpr (kResNl) {
-          if (nonlin) {
-            for (int i = 0; i < 9; i++) {
-              ep[i] = ep[i] + eq[2][i];
-              eu[i] = eu[i] + 0.5 * eq[3][i];
-            }
-          }
-        }
-        apply_cs(sec, det, eu, y);
-        acc = acc + c[2] * dot9(ep, y);
-      }
-    }
-  }
-  out = acc;
-}
-
-template <int WM, int PM>
-__global__ __launch_bounds__(kThreads) void xpt_kernel(XptArgs a, int nel) {
-  // the element's three vectors, shared by its 12 threads (read-only)
-  __shared__ double qs[kThreads / 12][3][24];
-  const int tid = blockIdx.x * kThreads + threadIdx.x;
-  const int le = tid / 12, dir = tid % 12, ll = threadIdx.x / 12;
-  const bool active = le < nel;
-  const int e = a.elems[active ? le : nel - 1];
+  // places of the vectors and pairs among the sources
+  constexpr int wi[3] = {0, bits(WM & 1), bits(WM & 3)};
+  constexpr int pi[4] = {NW, NW + bits(PM & 1), NW + bits(PM & 3), NW + bits(PM & 7)};
+  __shared__ SM smem[kElems];
+  SM &sm = smem[threadIdx.x >> 2];
+  const int p = threadIdx.x & 3;
+  const long le = (long)blockIdx.x * kElems + (threadIdx.x >> 2);
+  const bool active = le < a.nelems;
+  const int e = active ? (int)le : a.nelems - 1;
   const long design = blockIdx.y;
   const int *cn = a.conn + 4 * e;
-  const double *src[3] = {a.phi, a.u, a.psi};
-  for (int k = dir; k < 72; k += 12) {
-    const int w = k / 24, i = k % 24;
-    qs[ll][w][i] = ((WM >> w) & 1) && src[w] ? src[w][design * a.stride + 6 * cn[i / 6] + i % 6] : 0.0;
+  const double c[4] = {a.coef[4 * design], a.coef[4 * design + 1], a.coef[4 * design + 2], a.coef[4 * design + 3]};
+  {
+    // a vector whose coefficients are zero does not enter
+    const bool has[3] = {c[0] != 0.0 || c[1] != 0.0 || c[3] != 0.0, c[1] != 0.0 || c[2] != 0.0, c[2] != 0.0};
+    const double *src[3] = {a.phi, a.u, a.psi};
+    const long o = design * a.stride + 6 * cn[p];
+#pragma unroll
+    for (int w = 0; w < 3; w++)
+      if ((WM >> w) & 1) {
+#pragma unroll
+        for (int i = 0; i < 6; i++) sm.q[wi[w]][6 * p + i] = src[w] && has[w] ? src[w][o + i] : 0.0;
+      }
+  }
+  V3 X[4];
+#pragma unroll
+  for (int m = 0; m < 4; m++) X[m] = load3(a.Xpts + 3 * cn[m]);
+  auto sum = [](const double N[4], const V3 v[4]) { return N[0] * v[0] + N[1] * v[1] + N[2] * v[2] + N[3] * v[3]; };
+  double u_, v_, nN[4], nNa[4], nNb[4];
+  // ---- node p: normal, frame, drilling strains (et = 0.5 (Ct[3] + u0x[3] -
+  // Ct[1] - u0x[1]), TacsShellComputeDrillStrain) ----
+  node_point(p, u_, v_);
+  shape4(u_, v_, nN, nNa, nNb);
+  const V3 an = sum(nNa, X), bn = sum(nNb, X);
+  V3 fnp = cross(an, bn);
+  const double fl = sqrt(dot(fnp, fnp)), fi = fl != 0.0 ? 1.0 / fl : 1.0;
+  fnp = fi * fnp;
+  sm.fn[3 * p] = fnp.x;
+  sm.fn[3 * p + 1] = fnp.y;
+  sm.fn[3 * p + 2] = fnp.z;
+  __syncthreads();
+  // gradient of a vector's displacements, and its nodal directors d = q x n
+  auto grad_u = [&](int s, const double Na[4], const double Nb[4], V3 &ux, V3 &ue) {
+    ux = zero3();
+    ue = zero3();
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      const V3 q = load3(&sm.q[s][6 * m]);
+      ux += Na[m] * q;
+      ue += Nb[m] * q;
+    }
+  };
+  auto director = [&](int s, int m) { return cross(load3(&sm.q[s][6 * m + 3]), load3(&sm.fn[3 * m])); };
+  Frame nf;
+  Inverse ni;
+  nf.set(an, fnp);
+  ni.set(an, bn, fnp);
+  const V3 nx1 = ni.mul(nf.T[0]), nx2 = ni.mul(nf.T[1]);
+#pragma unroll
+  for (int s = 0; s < NW; s++) {
+    V3 ux, ue;
+    grad_u(s, nNa, nNb, ux, ue);
+    const V3 rot = load3(&sm.q[s][6 * p + 3]);
+    sm.f.et[s][p] = -dot(rot, cross(nf.T[0], nf.T[1])) +
+                    0.5 * (dot(nf.T[1], nx1.x * ux + nx1.y * ue) - dot(nf.T[0], nx2.x * ux + nx2.y * ue));
+  }
+  // ---- tying strains at points p, p + 4, p + 8 ----
+#pragma unroll 1
+  for (int t = p; t < 9; t += 4) {
+    double u, v, N[4], Na[4], Nb[4];
+    tying_point(t, u, v);
+    shape4(u, v, N, Na, Nb);
+    const V3 at = sum(Na, X), bt = sum(Nb, X);
+    V3 n0 = zero3(), ux[NW], ue[NW], d0[NW];
+#pragma unroll
+    for (int m = 0; m < 4; m++) n0 += N[m] * load3(&sm.fn[3 * m]);
+    const int f = tying_field(t);
+#pragma unroll
+    for (int s = 0; s < NW; s++) {
+      grad_u(s, Na, Nb, ux[s], ue[s]);
+      d0[s] = zero3();
+#pragma unroll
+      for (int m = 0; m < 4; m++) d0[s] += N[m] * director(s, m);
+      sm.f.ty[s][t] = f == kG11   ? dot(ux[s], at)
+                      : f == kG22 ? dot(ue[s], bt)
+                      : f == kG12 ? 0.5 * (dot(ux[s], bt) + dot(ue[s], at))
+                      : f == kG23 ? 0.5 * (dot(bt, d0[s]) + dot(n0, ue[s]))
+                                  : 0.5 * (dot(at, d0[s]) + dot(n0, ux[s]));
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if ((PM >> k) & 1) {
+        const int A = wi[kPairA[k]], B = wi[kPairB[k]];
+        sm.f.ty[pi[k]][t] = f == kG11   ? dot(ux[A], ux[B])
+                            : f == kG22 ? dot(ue[A], ue[B])
+                            : f == kG12 ? 0.5 * (dot(ux[A], ue[B]) + dot(ux[B], ue[A]))
+                            : f == kG23 ? 0.5 * (dot(d0[A], ue[B]) + dot(d0[B], ue[A]))
+                                        : 0.5 * (dot(d0[A], ux[B]) + dot(d0[B], ux[A]));
+      }
+  }
+  __syncthreads();
+  // ---- quadrature point p ----
+  double N[4], Na[4], Nb[4], Nt[9];
+  quad_point(p, u_, v_);
+  shape4(u_, v_, N, Na, Nb);
+  tying_interp(u_, v_, Nt);
+  const V3 aq = sum(Na, X), bq = sum(Nb, X);
+  V3 n0 = zero3(), na = zero3(), nb = zero3();
+#pragma unroll
+  for (int m = 0; m < 4; m++) {
+    const V3 f = load3(&sm.fn[3 * m]);
+    n0 += N[m] * f;
+    na += Na[m] * f;
+    nb += Nb[m] * f;
+  }
+  Frame F;
+  Inverse I;
+  F.set(aq, n0);
+  I.set(aq, bq, n0);
+  V3 x[3], z[2], h[2];  // columns of X_d^{-1} T and of the normal-gradient part
+#pragma unroll
+  for (int k = 0; k < 3; k++) x[k] = I.mul(F.T[k]);
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    h[k] = x[k].x * na + x[k].y * nb;
+    z[k] = -1.0 * I.mul(h[k]);
+  }
+  // tying fields of a source, interpolated here
+  auto fields = [&](int s, double g[5]) {
+    const double *t = sm.f.ty[s];
+    g[kG11] = Nt[0] * t[0] + Nt[1] * t[1];
+    g[kG22] = Nt[2] * t[2] + Nt[3] * t[3];
+    g[kG12] = Nt[4] * t[4];
+    g[kG23] = Nt[5] * t[5] + Nt[6] * t[6];
+    g[kG13] = Nt[7] * t[7] + Nt[8] * t[8];
+  };
+  auto sym_mul = [](const double g[5], V3 v) -> V3 {
+    return {g[kG11] * v.x + g[kG12] * v.y + g[kG13] * v.z, g[kG12] * v.x + g[kG22] * v.y + g[kG23] * v.z,
+            g[kG13] * v.x + g[kG23] * v.y};
+  };
+  // displacement fields of the vectors at the point
+  V3 ux[NW], ue[NW], d0[NW], dx[NW], de[NW], U0[NW][2], U1[NW][2];
+#pragma unroll
+  for (int s = 0; s < NW; s++) {
+    grad_u(s, Na, Nb, ux[s], ue[s]);
+    d0[s] = dx[s] = de[s] = zero3();
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      const V3 d = director(s, m);
+      d0[s] += N[m] * d;
+      dx[s] += Na[m] * d;
+      de[s] += Nb[m] * d;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const V3 P = comb(x[k], ux[s], ue[s], d0[s]);
+      const V3 S = x[k].x * dx[s] + x[k].y * de[s] + comb(z[k], ux[s], ue[s], d0[s]);
+      U0[s][k] = {dot(F.T[0], P), dot(F.T[1], P), dot(F.T[2], P)};
+      U1[s][k] = {dot(F.T[0], S), dot(F.T[1], S), dot(F.T[2], S)};
+    }
+  }
+  auto tensor_strains = [&](int s, double e9[9]) {
+    double g[5];
+    fields(s, g);
+    const V3 y0 = sym_mul(g, x[0]), y1 = sym_mul(g, x[1]);
+    e9[0] = dot(x[0], y0);
+    e9[1] = dot(x[1], y1);
+    e9[2] = 2.0 * dot(x[0], y1);
+    e9[6] = 2.0 * dot(x[2], y1);
+    e9[7] = 2.0 * dot(x[2], y0);
+  };
+  auto linear_strain = [&](int s, double e9[9]) {
+    tensor_strains(s, e9);
+    e9[3] = U1[s][0].x;
+    e9[4] = U1[s][1].y;
+    e9[5] = U1[s][1].x + U1[s][0].y;
+    e9[8] = N[0] * sm.f.et[s][0] + N[1] * sm.f.et[s][1] + N[2] * sm.f.et[s][2] + N[3] * sm.f.et[s][3];
+  };
+  auto pair_strain = [&](int k, double e9[9]) {
+    const int A = wi[kPairA[k]], B = wi[kPairB[k]];
+    tensor_strains(pi[k], e9);
+    e9[3] = dot(U0[A][0], U1[B][0]) + dot(U0[B][0], U1[A][0]);
+    e9[4] = dot(U0[A][1], U1[B][1]) + dot(U0[B][1], U1[A][1]);
+    e9[5] = dot(U0[A][0], U1[B][1]) + dot(U1[A][0], U0[B][1]) + dot(U0[B][0], U1[A][1]) + dot(U1[B][0], U0[A][1]);
+    e9[8] = 0.0;
+  };
+  // ---- the scalar's terms and the adjoints of its strains ----
+  const double thick = a.thick[design * a.nelems + e];
+  const Section sec = make_section(a.mat, thick);
+  const double eth = a.temp ? a.mat.cte * a.temp[design * a.nelems + e] : 0.0;
+  const double det = I.det;
+  double value = 0.0;  // of the integrand: the adjoint of the determinant
+  double sb[NS][9];    // adjoints of the sources' strains
+#pragma unroll
+  for (int s = 0; s < NS; s++)
+#pragma unroll
+    for (int i = 0; i < 9; i++) sb[s][i] = 0.0;
+  double eu[9], Ceu[9];
+  if constexpr (kU) {
+    linear_strain(wi[1], eu);
+    eu[0] -= eth;
+    eu[1] -= eth;
+  }
+  if constexpr (kPhi) {
+    double ep[9], Cep[9];
+    linear_strain(wi[0], ep);
+    apply_c(sec, ep, Cep);
+    value += c[0] * dot9(ep, Cep);
+#pragma unroll
+    for (int i = 0; i < 9; i++) sb[wi[0]][i] += 2.0 * c[0] * det * Cep[i];
+    if constexpr (kGeo) {
+      double q0[9], q1[9], Cq[9];
+      pair_strain(0, q0);
+      pair_strain(1, q1);
+      apply_c(sec, eu, Ceu);
+      value += c[1] * (2.0 * dot9(q0, Cep) + dot9(q1, Ceu));
+      const double w = c[1] * det;
+      apply_c(sec, q0, Cq);
+#pragma unroll
+      for (int i = 0; i < 9; i++) {
+        sb[wi[0]][i] += 2.0 * w * Cq[i];
+        sb[pi[0]][i] += 2.0 * w * Cep[i];
+        sb[pi[1]][i] += w * Ceu[i];
+      }
+      apply_c(sec, q1, Cq);
+#pragma unroll
+      for (int i = 0; i < 9; i++) sb[wi[1]][i] += w * Cq[i];
+    }
+  }
+  if constexpr (kRes) {
+    double es[9], Ces[9];
+    linear_strain(wi[2], es);
+    double et[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) et[i] = eu[i];
+    if constexpr (kResNl) {
+      if (a.nonlin) {
+        double q[9];
+        pair_strain(2, q);
+#pragma unroll
+        for (int i = 0; i < 9; i++) es[i] += q[i];
+        pair_strain(3, q);
+#pragma unroll
+        for (int i = 0; i < 9; i++) et[i] += 0.5 * q[i];
+      }
+    }
+    apply_c(sec, et, Ceu);
+    apply_c(sec, es, Ces);
+    value += c[2] * dot9(es, Ceu);
+    const double w = c[2] * det;
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+      sb[wi[1]][i] += w * Ces[i];
+      sb[wi[2]][i] += w * Ceu[i];
+    }
+    if constexpr (kResNl) {
+      if (a.nonlin) {
+#pragma unroll
+        for (int i = 0; i < 9; i++) {
+          sb[pi[2]][i] += w * Ceu[i];
+          sb[pi[3]][i] += 0.5 * w * Ces[i];
+        }
+      }
+    }
+  }
+  // adjoints of the directors at the point (values and gradients)
+  V3 d0b[NW], dxb[NW], deb[NW];
+#pragma unroll
+  for (int s = 0; s < NW; s++) d0b[s] = dxb[s] = deb[s] = zero3();
+  if constexpr (kPhi) {
+    if (c[3] != 0.0) {
+      // mass moments of TACSIsoShellConstitutive with tOffset = 0
+      const double m0 = a.mat.rho * thick, m2 = a.mat.rho * thick * thick * thick / 12.0;
+      V3 u0 = zero3();
+#pragma unroll
+      for (int m = 0; m < 4; m++) u0 += N[m] * load3(&sm.q[wi[0]][6 * m]);
+      value += c[3] * (m0 * dot(u0, u0) + m2 * dot(d0[wi[0]], d0[wi[0]]));
+      d0b[wi[0]] += (2.0 * c[3] * det * m2) * d0[wi[0]];
+    }
+  }
+  // ---- back through the strains ----
+  V3 xb[3] = {zero3(), zero3(), zero3()}, zb[2] = {zero3(), zero3()};
+  double gb[NS][5], e8b[NW];
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    // E = x^T G x with E's adjoint symmetric: rows 0, 1, 2, 6, 7
+    double g[5];
+    fields(s, g);
+    const double *b = sb[s];
+    const V3 y0 = sym_mul(g, x[0]), y1 = sym_mul(g, x[1]), y2 = sym_mul(g, x[2]);
+    xb[0] += 2.0 * (b[0] * y0 + b[2] * y1 + b[7] * y2);
+    xb[1] += 2.0 * (b[2] * y0 + b[1] * y1 + b[6] * y2);
+    xb[2] += 2.0 * (b[7] * y0 + b[6] * y1);
+    const V3 m0 = b[0] * x[0] + b[2] * x[1] + b[7] * x[2], m1 = b[2] * x[0] + b[1] * x[1] + b[6] * x[2],
+             m2 = b[7] * x[0] + b[6] * x[1];
+    gb[s][kG11] = x[0].x * m0.x + x[1].x * m1.x + x[2].x * m2.x;
+    gb[s][kG22] = x[0].y * m0.y + x[1].y * m1.y + x[2].y * m2.y;
+    gb[s][kG12] = 2.0 * (x[0].x * m0.y + x[1].x * m1.y + x[2].x * m2.y);
+    gb[s][kG23] = 2.0 * (x[0].y * m0.z + x[1].y * m1.z + x[2].y * m2.z);
+    gb[s][kG13] = 2.0 * (x[0].x * m0.z + x[1].x * m1.z + x[2].x * m2.z);
+  }
+  V3 Tb[3] = {zero3(), zero3(), zero3()};
+#pragma unroll
+  for (int s = 0; s < NW; s++) {
+    e8b[s] = sb[s][8];
+    // adjoints of the columns of U0, U1: bending strains, then the pairs
+    V3 U0b[2] = {zero3(), zero3()}, U1b[2];
+    U1b[0] = {sb[s][3], sb[s][5], 0.0};
+    U1b[1] = {sb[s][5], sb[s][4], 0.0};
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if ((PM >> k) & 1) {
+        const double *b = sb[pi[k]];
+        const int A = wi[kPairA[k]], B = wi[kPairB[k]];
+        if (s == A) {
+          U0b[0] += b[3] * U1[B][0] + b[5] * U1[B][1];
+          U0b[1] += b[5] * U1[B][0] + b[4] * U1[B][1];
+          U1b[0] += b[3] * U0[B][0] + b[5] * U0[B][1];
+          U1b[1] += b[5] * U0[B][0] + b[4] * U0[B][1];
+        }
+        if (s == B) {
+          U0b[0] += b[3] * U1[A][0] + b[5] * U1[A][1];
+          U0b[1] += b[5] * U1[A][0] + b[4] * U1[A][1];
+          U1b[0] += b[3] * U0[A][0] + b[5] * U0[A][1];
+          U1b[1] += b[5] * U0[A][0] + b[4] * U0[A][1];
+        }
+      }
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const V3 P = comb(x[k], ux[s], ue[s], d0[s]);
+      const V3 S = x[k].x * dx[s] + x[k].y * de[s] + comb(z[k], ux[s], ue[s], d0[s]);
+      const V3 P0 = comb(U0b[k], F.T[0], F.T[1], F.T[2]), P1 = comb(U1b[k], F.T[0], F.T[1], F.T[2]);
+      Tb[0] += U0b[k].x * P + U1b[k].x * S;
+      Tb[1] += U0b[k].y * P + U1b[k].y * S;
+      Tb[2] += U0b[k].z * P + U1b[k].z * S;
+      xb[k] += V3{dot(ux[s], P0) + dot(dx[s], P1), dot(ue[s], P0) + dot(de[s], P1), dot(d0[s], P0)};
+      zb[k] += V3{dot(ux[s], P1), dot(ue[s], P1), dot(d0[s], P1)};
+      d0b[s] += x[k].z * P0 + z[k].z * P1;
+      dxb[s] += x[k].x * P1;
+      deb[s] += x[k].y * P1;
+    }
+  }
+  // ---- back through the frame of the point ----
+  V3 Gi[3] = {zero3(), zero3(), zero3()}, nab = zero3(), nbb = zero3();
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const V3 hb = -1.0 * I.mul_t(zb[k]);
+    Gi[0] += -zb[k].x * h[k];
+    Gi[1] += -zb[k].y * h[k];
+    Gi[2] += -zb[k].z * h[k];
+    nab += x[k].x * hb;
+    nbb += x[k].y * hb;
+    xb[k].x += dot(na, hb);
+    xb[k].y += dot(nb, hb);
+  }
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    Tb[k] += I.mul_t(xb[k]);
+    Gi[0] += xb[k].x * F.T[k];
+    Gi[1] += xb[k].y * F.T[k];
+    Gi[2] += xb[k].z * F.T[k];
+  }
+  V3 ab = I.column(0, Gi, value), bb = I.column(1, Gi, value), n0b = I.column(2, Gi, value);
+  F.adjoint(aq, Tb, ab, n0b);
+  V3 Xb[4], fb[4];
+#pragma unroll
+  for (int m = 0; m < 4; m++) {
+    Xb[m] = Na[m] * ab + Nb[m] * bb;
+    fb[m] = N[m] * n0b + Na[m] * nab + Nb[m] * nbb;
+#pragma unroll
+    for (int s = 0; s < NW; s++)
+      fb[m] += cross(N[m] * d0b[s] + Na[m] * dxb[s] + Nb[m] * deb[s], load3(&sm.q[s][6 * m + 3]));
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < NS; s++)
+#pragma unroll
+    for (int i = 0; i < 5; i++) sm.b.g[p][s][i] = gb[s][i];
+#pragma unroll
+  for (int s = 0; s < NW; s++) sm.b.e8[p][s] = e8b[s];
+  __syncthreads();
+  // ---- back through the tying points ----
+#pragma unroll 1
+  for (int t = p; t < 9; t += 4) {
+    double u, v, tN[4], tNa[4], tNb[4], w[NS];
+    const int f = tying_field(t);
+#pragma unroll
+    for (int s = 0; s < NS; s++) w[s] = 0.0;
+#pragma unroll
+    for (int iq = 0; iq < 4; iq++) {
+      double Nq[9];
+      quad_point(iq, u, v);
+      tying_interp(u, v, Nq);
+      double Nqt = Nq[0];
+#pragma unroll
+      for (int k = 1; k < 9; k++) Nqt = t == k ? Nq[k] : Nqt;
+#pragma unroll
+      for (int s = 0; s < NS; s++) w[s] += Nqt * sm.b.g[iq][s][f];
+    }
+    tying_point(t, u, v);
+    shape4(u, v, tN, tNa, tNb);
+    const V3 at = sum(tNa, X), bt = sum(tNb, X);
+    V3 tux[NW], tue[NW], td[NW];
+#pragma unroll
+    for (int s = 0; s < NW; s++) grad_u(s, tNa, tNb, tux[s], tue[s]);
+    V3 atb = zero3(), btb = zero3(), tnb = zero3();
+#pragma unroll
+    for (int s = 0; s < NW; s++) {
+      V3 d = zero3();
+      td[s] = zero3();
+#pragma unroll
+      for (int m = 0; m < 4; m++) d += tN[m] * director(s, m);
+      if (f == kG11) {
+        atb += w[s] * tux[s];
+      } else if (f == kG22) {
+        btb += w[s] * tue[s];
+      } else if (f == kG12) {
+        atb += (0.5 * w[s]) * tue[s];
+        btb += (0.5 * w[s]) * tux[s];
+      } else if (f == kG23) {
+        btb += (0.5 * w[s]) * d;
+        td[s] += (0.5 * w[s]) * bt;
+        tnb += (0.5 * w[s]) * tue[s];
+      } else {
+        atb += (0.5 * w[s]) * d;
+        td[s] += (0.5 * w[s]) * at;
+        tnb += (0.5 * w[s]) * tux[s];
+      }
+    }
+    if (f == kG23 || f == kG13) {
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if ((PM >> k) & 1) {
+          const int A = wi[kPairA[k]], B = wi[kPairB[k]];
+          const double hw = 0.5 * w[pi[k]];
+          td[A] += hw * (f == kG23 ? tue[B] : tux[B]);
+          td[B] += hw * (f == kG23 ? tue[A] : tux[A]);
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      Xb[m] += tNa[m] * atb + tNb[m] * btb;
+      V3 s3 = tnb;
+#pragma unroll
+      for (int s = 0; s < NW; s++) s3 += cross(td[s], load3(&sm.q[s][6 * m + 3]));
+      fb[m] += tN[m] * s3;
+    }
+  }
+  // ---- back through the drilling strains of node p ----
+  V3 Tnb[3] = {zero3(), zero3(), zero3()}, x1b = zero3(), x2b = zero3(), cb = zero3();
+#pragma unroll
+  for (int s = 0; s < NW; s++) {
+    double w = 0.0;
+#pragma unroll
+    for (int iq = 0; iq < 4; iq++) {
+      double u, v, qN[4], qa[4], qb[4];
+      quad_point(iq, u, v);
+      shape4(u, v, qN, qa, qb);
+      const double Nn = p == 0 ? qN[0] : p == 1 ? qN[1] : p == 2 ? qN[2] : qN[3];
+      w += Nn * sm.b.e8[iq][s];
+    }
+    V3 sx, se;
+    grad_u(s, nNa, nNb, sx, se);
+    cb += -w * load3(&sm.q[s][6 * p + 3]);
+    const double hw = 0.5 * w;
+    Tnb[1] += hw * (nx1.x * sx + nx1.y * se);
+    Tnb[0] += -hw * (nx2.x * sx + nx2.y * se);
+    x1b.x += hw * dot(nf.T[1], sx);
+    x1b.y += hw * dot(nf.T[1], se);
+    x2b.x -= hw * dot(nf.T[0], sx);
+    x2b.y -= hw * dot(nf.T[0], se);
+  }
+  Tnb[0] += cross(nf.T[1], cb) + ni.mul_t(x1b);
+  Tnb[1] += cross(cb, nf.T[0]) + ni.mul_t(x2b);
+  V3 nGi[3];
+  nGi[0] = x1b.x * nf.T[0] + x2b.x * nf.T[1];
+  nGi[1] = x1b.y * nf.T[0] + x2b.y * nf.T[1];
+  nGi[2] = zero3();
+  V3 anb = ni.column(0, nGi, 0.0), bnb = ni.column(1, nGi, 0.0), fnb = ni.column(2, nGi, 0.0);
+  nf.adjoint(an, Tnb, anb, fnb);
+  // ---- the normals' adjoints, summed over the lanes, through node p's normal ----
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < 4; m++) {
+    sm.part[p][3 * m] = fb[m].x;
+    sm.part[p][3 * m + 1] = fb[m].y;
+    sm.part[p][3 * m + 2] = fb[m].z;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int l = 0; l < 4; l++) fnb += load3(&sm.part[l][3 * p]);
+  const V3 cb3 = fi * (fnb - dot(fnp, fnb) * fnp);
+  anb += cross(bn, cb3);
+  bnb += cross(cb3, an);
+#pragma unroll
+  for (int m = 0; m < 4; m++) Xb[m] += nNa[m] * anb + nNb[m] * bnb;
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < 4; m++) {
+    sm.part[p][3 * m] = Xb[m].x;
+    sm.part[p][3 * m + 1] = Xb[m].y;
+    sm.part[p][3 * m + 2] = Xb[m].z;
   }
   __syncthreads();
   if (!active) return;
-  const double(*q)[24] = qs[ll];
-  Dual X[12];
-  for (int i = 0; i < 12; i++) X[i] = Dual(a.Xpts[3 * cn[i / 3] + i % 3], i == dir ? 1.0 : 0.0);
-  const double thick = a.thick[design * a.nelems + e];
-  const double temp = a.temp ? a.temp[design * a.nelems + e] : 0.0;
-  const Section sec = make_section(a.mat, thick);
-  const double c[4] = {a.coef[4 * design], a.coef[4 * design + 1], a.coef[4 * design + 2], a.coef[4 * design + 3]};
-  // mass moments of TACSIsoShellConstitutive with tOffset = 0
-  const double m0 = a.mat.rho * thick, m2 = a.mat.rho * thick * thick * thick / 12.0;
-  Dual s;
-  element_scalars<Dual, WM, PM>(X, q, sec, a.mat.cte * temp, a.nonlin != 0, c, m0, m2, s);
-  a.dfdX[design * a.dX_stride + 3 * cn[dir / 3] + dir % 3] += s.d;
+  const V3 o = ((load3(&sm.part[0][3 * p]) + load3(&sm.part[1][3 * p])) + load3(&sm.part[2][3 * p])) +
+               load3(&sm.part[3][3 * p]);
+  double *dst = out + (design * a.nelems + e) * 12 + 3 * p;
+  dst[0] = o.x;
+  dst[1] = o.y;
+  dst[2] = o.z;
+}
+
+// dfdX[node] += the node's parts of its elements' gradients, in element order
+__global__ __launch_bounds__(256) void xpt_gather_kernel(XptArgs a, int nnodes, const int *__restrict__ ptr,
+                                                         const int *__restrict__ corner, const double *__restrict__ g) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= 3 * nnodes) return;
+  const int n = i / 3, d = i - 3 * n;
+  const long o = blockIdx.y * (long)a.nelems * 12 + d;
+  double s = 0.0;
+  for (int k = ptr[n]; k < ptr[n + 1]; k++) s += g[o + 3L * corner[k]];
+  a.dfdX[blockIdx.y * a.dX_stride + i] += s;
 }
 
 }  // namespace
 
-hipError_t launch_xpt_kernel(const XptArgs &args, int nel, int nbatch, hipStream_t stream) {
-  if (nel <= 0) return hipSuccess;
-  const unsigned blocks = (unsigned)((12L * nel + kThreads - 1) / kThreads);
-  const dim3 grid(blocks, nbatch);
+hipError_t launch_xpt_kernel(const XptArgs &args, int nnodes, int nbatch, const int *node_ptr, const int *node_corner,
+                             double *work, hipStream_t stream) {
+  if (args.nelems <= 0) return hipSuccess;
+  const dim3 grid((args.nelems + kElems - 1) / kElems, nbatch), block(4 * kElems);
   const int t = args.terms;
   if ((t & kXptR) && (t & (kXptK | kXptG | kXptM)))  // every vector and pair
-    hipLaunchKernelGGL((xpt_kernel<7, 15>), grid, dim3(kThreads), 0, stream, args, nel);
+    hipLaunchKernelGGL((xpt_kernel<7, 15>), grid, block, 0, stream, args, work);
   else if (t & kXptR)  // u, psi; (u, psi) and (u, u) for the nonlinear model
     if (args.nonlin)
-      hipLaunchKernelGGL((xpt_kernel<6, 12>), grid, dim3(kThreads), 0, stream, args, nel);
+      hipLaunchKernelGGL((xpt_kernel<6, 12>), grid, block, 0, stream, args, work);
     else
-      hipLaunchKernelGGL((xpt_kernel<6, 0>), grid, dim3(kThreads), 0, stream, args, nel);
+      hipLaunchKernelGGL((xpt_kernel<6, 0>), grid, block, 0, stream, args, work);
   else if (t & kXptG)  // phi, u; (u, phi) and (phi, phi)
-    hipLaunchKernelGGL((xpt_kernel<3, 3>), grid, dim3(kThreads), 0, stream, args, nel);
+    hipLaunchKernelGGL((xpt_kernel<3, 3>), grid, block, 0, stream, args, work);
   else  // phi alone: s_K, s_M
-    hipLaunchKernelGGL((xpt_kernel<1, 0>), grid, dim3(kThreads), 0, stream, args, nel);
+    hipLaunchKernelGGL((xpt_kernel<1, 0>), grid, block, 0, stream, args, work);
+  hipLaunchKernelGGL(xpt_gather_kernel, dim3((3 * nnodes + 255) / 256, nbatch), dim3(256), 0, stream, args, nnodes,
+                     node_ptr, node_corner, work);
   return hipGetLastError();
 }
 
