@@ -49,19 +49,16 @@ struct ModeTraits {
   static constexpr bool kMassTerms = kJac || kJvp;
   static constexpr bool kMat = (MODE == kModeKLin || MODE == kModeKNl || MODE == kModeG || kJac || kJvp);
   static constexpr bool kState = (MODE != kModeKLin);
-  static constexpr bool kNonlin = (MODE == kModeKNl || MODE == kModeRNl || MODE == kModeAdjResNl ||
-                                   MODE == kModeOutNl || MODE == kModeJacNl || MODE == kModeJvpNl);
+  static constexpr bool kNonlin = (MODE == kModeKNl || MODE == kModeRNl || MODE == kModeOutNl || MODE == kModeJacNl ||
+                                   MODE == kModeJvpNl);
   // strains, stresses and failure values at the element nodes instead of
   // the quadrature points (getOutputData)
   static constexpr bool kOut = (MODE == kModeOutLin || MODE == kModeOutNl);
-  static constexpr bool kRes = (MODE == kModeRLin || MODE == kModeRNl || MODE == kModeAdjResLin ||
-                                MODE == kModeAdjResNl || kJac);
+  static constexpr bool kRes = (MODE == kModeRLin || MODE == kModeRNl || kJac);
   static constexpr bool kGeo = (MODE == kModeKNl || MODE == kModeG || MODE == kModeJacNl || MODE == kModeJvpNl);
-  // B1 = dB/dq along the state is formed too (geometric stiffness and the
-  // thickness adjoint), which doubles the tying Jacobian and B storage
-  static constexpr bool kTwo = (MODE == kModeG || MODE == kModeAdjDV);
-  static constexpr bool kAdj =
-      (MODE == kModeAdjDV || MODE == kModeAdjResLin || MODE == kModeAdjResNl);
+  // B1 = dB/dq along the state is formed too (geometric stiffness), which
+  // doubles the tying Jacobian and B storage
+  static constexpr bool kTwo = (MODE == kModeG);
   static constexpr bool kStrain = kRes || kGeo;  // stresses at the quadrature points
 };
 
@@ -74,7 +71,6 @@ struct ElemSmem {
   static constexpr int kNB = MT::kTwo ? 2 : 1;
   double X[12];
   double s[24];
-  double v2[MT::kAdj ? 24 : 1];  // second state of the adjoint modes: path u or psi
   double dd[MT::kJac ? 24 : 1];  // second time derivative of the state (addJacobian)
   double fn[12];
   double T[36], XT[36], XzT[36], wdet[4];
@@ -392,10 +388,6 @@ __device__ __forceinline__ void elem_body(const ElemArgs &a) {
     sm.s[lane] = (kState && a.state)
                      ? a.state[design * a.state_stride + 6 * cn[lane / 6] + lane % 6]
                      : 0.0;
-    if (MODE == kModeAdjDV)
-      sm.v2[lane] = a.u2 ? a.u2[design * a.u2_stride + 6 * cn[lane / 6] + lane % 6] : 0.0;
-    if (MODE == kModeAdjResLin || MODE == kModeAdjResNl)
-      sm.v2[lane] = a.psi[design * a.psi_stride + 6 * cn[lane / 6] + lane % 6];
     if (MT::kJac) sm.dd[lane] = a.ddu ? a.ddu[design * a.ddu_stride + 6 * cn[lane / 6] + lane % 6] : 0.0;
   }
   __syncthreads();
@@ -566,7 +558,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs &a) {
     if (kState) sm.ety[t] = kNonlin ? lin + quad : lin;
     // derivative coefficients with a = xfac X + ufac U, nd = xfac n0 + ufac d0
     for (int pass = 0; pass < 2; pass++) {
-      if (pass == 1 && MODE != kModeG && MODE != kModeAdjDV) break;
+      if (pass == 1 && MODE != kModeG) break;
       const double xf = (pass == 0) ? 1.0 : 0.0;
       const double uf = (pass == 0) ? (kNonlin ? 1.0 : 0.0) : 1.0;
       double av[6], nd[3], dU[6] = {0, 0, 0, 0, 0, 0}, dd[3] = {0, 0, 0};
@@ -841,12 +833,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs &a) {
         e[0] -= a.mat.cte * temp;
         e[1] -= a.mat.cte * temp;
         double s9[9];
-        if (MODE == kModeAdjResLin || MODE == kModeAdjResNl) {
-#pragma unroll
-          for (int i = 0; i < 9; i++) s9[i] = e[i];  // mechanical strain
-        } else {
-          apply_c(sec, sm.wdet[iq], e, s9);
-        }
+        apply_c(sec, sm.wdet[iq], e, s9);
 #pragma unroll
         for (int i = 0; i < 9; i++) sm.sig[9 * iq + i] = s9[i];
       }
@@ -871,116 +858,6 @@ __device__ __forceinline__ void elem_body(const ElemArgs &a) {
       acc += Nt[t] * w;
     }
     sm.dety[t] = acc;
-  }
-
-  // ---- thickness derivative of phi^T K phi and phi^T G(u) phi, and the
-  // path-adjoint right-hand side d(phi^T G(u) phi)/du ----
-  // With e(q) = B0 q + Q(q, q)/2 (Q symmetric bilinear, Bq(a) b = Q(a, b)):
-  //   phi^T K phi    = sum w e1(phi)^T C e1(phi),            e1 = B0 .
-  //   phi^T G(u) phi = sum w [2 Q(u, phi)^T C e1(phi) + (e1(u) - e_th)^T C Q(phi, phi)]
-  if constexpr (MODE == kModeAdjDV) {
-    const IsoSection dsec = iso_section(make_section_dt(a.mat, thick));
-    const double *su = sm.v2;
-    double *E = &sm.c.Y[0][0], *cv = &sm.c.Y[0][45];
-    const double ca = a.coef[2 * design], cb = a.coef[2 * design + 1];
-    double gdv = 0.0, gu = 0.0;
-    for (int iq = 0; iq < 4; iq++) {
-      if (lane < 24) {
-        double b[9];
-        build_bcol<kBLin>(sm, iq, lane, Jr[0], b);
-#pragma unroll
-        for (int i = 0; i < 9; i++) sm.c.B[0][24 * i + lane] = b[i];
-        build_bcol<kBQuad>(sm, iq, lane, Jr[kNB - 1], b);
-#pragma unroll
-        for (int i = 0; i < 9; i++) sm.c.B[1][24 * i + lane] = b[i];
-      }
-      elem_sync<EPW>();
-      // E = [e1(phi), e1(u), Q(phi, u), Q(phi, phi)]
-      for (int it = lane; it < 36; it += 32) {
-        const int v = it / 9, i = it % 9;
-        const double *M = (v < 2) ? &sm.c.B[0][24 * i] : &sm.c.B[1][24 * i];
-        const double *x = (v == 0 || v == 3) ? sm.s : su;
-        double acc = 0.0;
-#pragma unroll
-        for (int k = 0; k < 24; k++) acc += M[k] * x[k];
-        E[it] = acc;
-      }
-      elem_sync<EPW>();
-      if (lane == 0) {
-        const double w = sm.wdet[iq];
-        const double *e1p = &E[0], *e1u = &E[9], *e2up = &E[18], *e2pp = &E[27];
-        double eu[9], t1[9], t2[9], c1[9], c2[9];
-#pragma unroll
-        for (int i = 0; i < 9; i++) eu[i] = e1u[i];
-        eu[0] -= a.mat.cte * temp;
-        eu[1] -= a.mat.cte * temp;
-        apply_c(dsec, w, e1p, t1);  // w C' e1(phi)
-        apply_c(dsec, w, eu, t2);   // w C' (e1(u) - e_th)
-        double da = 0.0, db = 0.0;
-#pragma unroll
-        for (int i = 0; i < 9; i++) {
-          da += e1p[i] * t1[i];
-          db += 2.0 * e2up[i] * t1[i] + e2pp[i] * t2[i];
-        }
-        gdv += ca * da + cb * db;
-        apply_c(sec, w, e1p, c1);
-        apply_c(sec, w, e2pp, c2);
-#pragma unroll
-        for (int i = 0; i < 9; i++) {
-          cv[i] = 2.0 * cb * c1[i];
-          cv[9 + i] = cb * c2[i];
-        }
-      }
-      elem_sync<EPW>();
-      // d/du: Bq(phi)^T (2 w C e1(phi)) + B0^T (w C Q(phi, phi))
-      if (lane < 24) {
-#pragma unroll
-        for (int i = 0; i < 9; i++) gu += sm.c.B[1][24 * i + lane] * cv[i] + sm.c.B[0][24 * i + lane] * cv[9 + i];
-      }
-      elem_sync<EPW>();
-    }
-    if (valid && lane == 0 && a.dv) a.dv[design * a.nelems + e] += gdv;
-    if (valid && lane < 24 && a.res) a.res[design * a.res_stride + 6 * cn[lane / 6] + lane % 6] += gu;
-    return;
-  }
-
-  // ---- psi^T dR_e/dt (TACSShellElement::addAdjResProduct, SE.h:774-868,
-  // with TACSIsoShellConstitutive::addStressDVSens) ----
-  if constexpr (MODE == kModeAdjResLin || MODE == kModeAdjResNl) {
-    const IsoSection dsec = iso_section(make_section_dt(a.mat, thick));
-    const double *sp = sm.v2;
-    double *E = &sm.c.Y[0][0];
-    double g = 0.0;
-    for (int iq = 0; iq < 4; iq++) {
-      if (lane < 24) {
-        double b[9];
-        if (kNonlin)
-          build_bcol<kBFull>(sm, iq, lane, Jr[0], b);
-        else
-          build_bcol<kBLin>(sm, iq, lane, Jr[0], b);
-#pragma unroll
-        for (int i = 0; i < 9; i++) sm.c.B[0][24 * i + lane] = b[i];
-      }
-      elem_sync<EPW>();
-      if (lane < 9) {  // dR/dq^T psi strain: B(u) psi
-        double acc = 0.0;
-#pragma unroll
-        for (int k = 0; k < 24; k++) acc += sm.c.B[0][24 * lane + k] * sp[k];
-        E[lane] = acc;
-      }
-      elem_sync<EPW>();
-      if (lane == 0) {
-        double t2[9];
-        apply_c(dsec, sm.wdet[iq], &sm.sig[9 * iq], t2);  // sig holds e(u) - e_th
-        double d = 0.0;
-#pragma unroll
-        for (int i = 0; i < 9; i++) d += E[i] * t2[i];
-        g += d;
-      }
-      elem_sync<EPW>();
-    }
-    if (valid && lane == 0) a.dv[design * a.nelems + e] += a.coef[design] * g;
-    return;
   }
 
   // ---- P5: quadrature loop: B columns, residual, B^T C B tile ----
@@ -1413,12 +1290,6 @@ hipError_t launch_elem_kernel(int mode, int variant, const ElemArgs &args, int c
       return launch_mode<kModeRLin>(args, count, nbatch, stream);
     case kModeRNl:
       return launch_mode<kModeRNl>(args, count, nbatch, stream);
-    case kModeAdjDV:
-      return launch_mode<kModeAdjDV>(args, count, nbatch, stream);
-    case kModeAdjResLin:
-      return launch_mode<kModeAdjResLin>(args, count, nbatch, stream);
-    case kModeAdjResNl:
-      return launch_mode<kModeAdjResNl>(args, count, nbatch, stream);
     case kModeOutLin:
       return launch_mode<kModeOutLin>(args, count, nbatch, stream);
     case kModeOutNl:

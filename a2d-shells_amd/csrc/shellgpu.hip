@@ -453,18 +453,18 @@ int run_colored(shellgpu_ctx *ctx, int mode, ElemArgs a) {
   return record_end(ctx, ctx->elem_ev);
 }
 
-// designs of one coordinate-derivative launch: as many as keep the element
-// gradients within 64 MiB (700,000 elements, many times what fills the GPU),
-// at least one
+// designs of one launch of the scalars' derivatives: as many as keep the
+// element gradients within 64 MiB (350,000 elements, many times what fills
+// the GPU), at least one
 static int xpt_designs(const shellgpu_ctx *ctx) {
-  const long n = (8L << 20) / (12L * ctx->nelems);
+  const long n = (8L << 20) / (24L * ctx->nelems);
   return (int)std::max(1L, std::min(n, (long)ctx->nbatch));
 }
 
 // the element gradients' buffer; sized with the designs, so that a
 // derivative call allocates nothing
 int reserve_xpt(shellgpu_ctx *ctx) {
-  const size_t need = 12L * ctx->nelems * xpt_designs(ctx);
+  const size_t need = 24L * ctx->nelems * xpt_designs(ctx);
   if (need <= ctx->xg_doubles) return 0;
   HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
   if (ctx->d_xg) (void)hipFree(ctx->d_xg);
@@ -475,40 +475,63 @@ int reserve_xpt(shellgpu_ctx *ctx) {
   return 0;
 }
 
-int run_xpt(shellgpu_ctx *ctx, const double *phi, const double *u, const double *psi, const double *coef,
-            int nonlin, int terms, double *dfdX) {
-  XptArgs a{};
+using XptLaunch = hipError_t(const XptArgs &, int, int, const int *, const int *, double *, hipStream_t);
+
+static int run_scalars(shellgpu_ctx *ctx, XptLaunch launch, XptArgs a) {
   a.conn = ctx->d_conn;
   a.Xpts = ctx->d_X;
-  a.thick = ctx->d_thick;
-  a.temp = ctx->d_temp;
   a.nelems = ctx->nelems;
   a.mat = ctx->mat;
-  a.phi = phi;
-  a.u = u;
-  a.psi = psi;
   a.stride = 6L * ctx->nnodes;
-  a.coef = coef;
-  a.nonlin = nonlin;
-  a.dfdX = dfdX;
   a.dX_stride = 3L * ctx->nnodes;
-  a.terms = terms;
   int rc = reserve_xpt(ctx);
   if (rc) return rc;
   const int nd = xpt_designs(ctx);
   for (int d = 0; d < ctx->nbatch; d += nd) {
     XptArgs b = a;
-    b.thick += (long)d * a.nelems;
-    if (b.temp) b.temp += (long)d * a.nelems;
+    b.thick = ctx->d_thick + (long)d * a.nelems;
+    b.temp = ctx->d_temp ? ctx->d_temp + (long)d * a.nelems : nullptr;
     if (b.phi) b.phi += d * a.stride;
     if (b.u) b.u += d * a.stride;
     if (b.psi) b.psi += d * a.stride;
     b.coef += 4L * d;
-    b.dfdX += d * a.dX_stride;
-    HIPCALL(ctx, launch_xpt_kernel(b, ctx->nnodes, std::min(nd, ctx->nbatch - d), ctx->d_nptr, ctx->d_corner, ctx->d_xg,
-                                   ctx->stream));
+    if (b.dfdX) b.dfdX += d * a.dX_stride;
+    if (b.dv) b.dv += (long)d * a.nelems;
+    if (b.res) b.res += d * a.stride;
+    HIPCALL(ctx, launch(b, ctx->nnodes, std::min(nd, ctx->nbatch - d), ctx->d_nptr, ctx->d_corner, ctx->d_xg,
+                        ctx->stream));
   }
   return 0;
+}
+
+int run_xpt(shellgpu_ctx *ctx, const double *phi, const double *u, const double *psi, const double *coef,
+            int nonlin, int terms, double *dfdX) {
+  XptArgs a{};
+  a.phi = phi;
+  a.u = u;
+  a.psi = psi;
+  a.coef = coef;
+  a.nonlin = nonlin;
+  a.terms = terms;
+  a.dfdX = dfdX;
+  return run_scalars(ctx, launch_xpt_kernel, a);
+}
+
+int run_dv(shellgpu_ctx *ctx, const double *phi, const double *u, const double *psi, const double *coef, int nonlin,
+           int terms, double *dfdt, double *dfdu) {
+  XptArgs a{};
+  a.phi = phi;
+  a.u = u;
+  a.psi = psi;
+  a.coef = coef;
+  a.nonlin = nonlin;
+  a.terms = terms;
+  a.dv = dfdt;
+  a.res = dfdu;
+  int rc = record_begin(ctx, ctx->elem_ev);
+  if (rc || (rc = run_scalars(ctx, launch_dv_kernel, a))) return rc;
+  if (ctx->timing) ctx->elem_launches += (ctx->nbatch + xpt_designs(ctx) - 1) / xpt_designs(ctx);
+  return record_end(ctx, ctx->elem_ev);
 }
 
 }  // namespace shellgpu
@@ -1098,15 +1121,16 @@ int shellgpu_assemble_jacobian(shellgpu_ctx *ctx, int model, double alpha, doubl
   return shellgpu_mat_apply_bcs(A, 1.0);
 }
 
-// per-design coefficients (c0, c1) into ctx->d_coef
-static int set_coef(shellgpu_ctx *ctx, double c0, double c1) {
-  std::vector<double> h(2 * ctx->nbatch);
+// per-design coefficient quadruples (c0, c1, c2, 0) into ctx->d_coef
+static int set_coef4(shellgpu_ctx *ctx, double c0, double c1, double c2, double c3 = 0.0) {
+  std::vector<double> h(4 * ctx->nbatch, 0.0);
   for (int d = 0; d < ctx->nbatch; d++) {
-    h[2 * d] = c0;
-    h[2 * d + 1] = c1;
+    h[4 * d] = c0;
+    h[4 * d + 1] = c1;
+    h[4 * d + 2] = c2;
+    h[4 * d + 3] = c3;
   }
   HIPCALL(ctx, hipMemcpyAsync(ctx->d_coef, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice, ctx->stream));
-  // h is released on return: the copy must have consumed it
   HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
   return 0;
 }
@@ -1116,15 +1140,8 @@ int shellgpu_add_adj_res_product(shellgpu_ctx *ctx, int model, double scale, con
   int rc = check_batch(ctx, nullptr);
   if (rc) return rc;
   if (!psi || !dfdt) return set_err(ctx, 1, "psi and dfdt are required");
-  std::vector<double> h(ctx->nbatch, scale);
-  HIPCALL(ctx, hipMemcpyAsync(ctx->d_coef, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice, ctx->stream));
-  HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
-  ElemArgs a = base_args(ctx, u);
-  a.psi = psi;
-  a.psi_stride = 6L * ctx->nnodes;
-  a.coef = ctx->d_coef;
-  a.dv = dfdt;
-  return run_colored(ctx, model == SHELLGPU_NONLINEAR ? kModeAdjResNl : kModeAdjResLin, a);
+  if ((rc = set_coef4(ctx, 0.0, 0.0, scale))) return rc;
+  return run_dv(ctx, nullptr, u, psi, ctx->d_coef, model == SHELLGPU_NONLINEAR, kXptR, dfdt, nullptr);
 }
 
 // psi^T A phi for a symmetric A (K, G(u), M and their derivatives) by
@@ -1165,13 +1182,8 @@ static int mat_dv_sym(shellgpu_ctx *ctx, int mattype, double scale, const double
     return run_colored(ctx, kModeMassDV, a);
   }
   const bool geo = mattype == SHELLGPU_GEOMETRIC;
-  if ((rc = set_coef(ctx, geo ? 0.0 : scale, geo ? scale : 0.0))) return rc;
-  ElemArgs a = base_args(ctx, phi);
-  a.u2 = u;
-  a.u2_stride = 6L * ctx->nnodes;
-  a.coef = ctx->d_coef;
-  a.dv = dfdt;
-  return run_colored(ctx, kModeAdjDV, a);
+  if ((rc = set_coef4(ctx, geo ? 0.0 : scale, geo ? scale : 0.0, 0.0))) return rc;
+  return run_dv(ctx, phi, geo ? u : nullptr, nullptr, ctx->d_coef, 0, geo ? kXptG : kXptK, dfdt, nullptr);
 }
 
 int shellgpu_add_mat_dv_sens_inner_product(shellgpu_ctx *ctx, int mattype, double scale, const double *psi,
@@ -1192,27 +1204,9 @@ int shellgpu_eval_mat_sv_sens_inner_product(shellgpu_ctx *ctx, const double *psi
   if (!phi || !dfdu) return set_err(ctx, 1, "phi and dfdu are required");
   HIPCALL(ctx, hipMemsetAsync(dfdu, 0, sizeof(double) * 6L * ctx->nnodes * ctx->nbatch, ctx->stream));
   return polarized(ctx, psi, phi, [&](const double *w, double c) {
-    int r = set_coef(ctx, 0.0, c);
-    if (r) return r;
-    ElemArgs a = base_args(ctx, w);
-    a.coef = ctx->d_coef;
-    a.res = dfdu;
-    return run_colored(ctx, kModeAdjDV, a);
+    const int r = set_coef4(ctx, 0.0, c, 0.0);
+    return r ? r : run_dv(ctx, w, nullptr, nullptr, ctx->d_coef, 0, kXptG, nullptr, dfdu);
   });
-}
-
-// per-design coefficient quadruples (c0, c1, c2, 0) into ctx->d_coef
-static int set_coef4(shellgpu_ctx *ctx, double c0, double c1, double c2, double c3 = 0.0) {
-  std::vector<double> h(4 * ctx->nbatch, 0.0);
-  for (int d = 0; d < ctx->nbatch; d++) {
-    h[4 * d] = c0;
-    h[4 * d + 1] = c1;
-    h[4 * d + 2] = c2;
-    h[4 * d + 3] = c3;
-  }
-  HIPCALL(ctx, hipMemcpyAsync(ctx->d_coef, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice, ctx->stream));
-  HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
-  return 0;
 }
 
 int shellgpu_add_mat_xpt_sens_inner_product(shellgpu_ctx *ctx, int mattype, double scale, const double *psi,

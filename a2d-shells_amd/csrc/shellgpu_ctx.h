@@ -51,8 +51,8 @@ struct shellgpu_ctx {
   double *d_thick = nullptr, *d_temp = nullptr;
   bool same_designs = false;  // every design has the same thickness and temperature
   double *d_coef = nullptr;  // 4 * nbatch per-design kernel coefficients
-  // element gradients of run_xpt, 12 doubles per element for as many designs
-  // as xpt_designs() allows at a time
+  // element gradients of run_xpt and run_dv, 24 doubles per element for as
+  // many designs as xpt_designs() allows at a time
   double *d_xg = nullptr;
   size_t xg_doubles = 0;
   // timing
@@ -92,4 +92,8 @@ int run_colored(shellgpu_ctx *ctx, int mode, ElemArgs a);
 // design), vectors with stride 6*nnodes, dfdX with stride 3*nnodes
 int run_xpt(shellgpu_ctx *ctx, const double *phi, const double *u, const double *psi, const double *coef,
             int nonlin, int terms, double *dfdX);
+// the thickness derivatives of the same scalars, and d(phi^T G(u) phi)/du
+// (dfdt, stride nelems, and dfdu, stride 6*nnodes, may be null)
+int run_dv(shellgpu_ctx *ctx, const double *phi, const double *u, const double *psi, const double *coef, int nonlin,
+           int terms, double *dfdt, double *dfdu);
 }  // namespace shellgpu

@@ -46,9 +46,6 @@ enum ElemMode {
   kModeG = 2,     // geometric stiffness, exact directional derivative
   kModeRLin = 3,  // linear-model residual
   kModeRNl = 4,   // nonlinear-model residual
-  kModeAdjDV = 5,     // thickness terms of a buckling eigenpair (state = phi)
-  kModeAdjResLin = 6, // psi^T dR/dt, linear model (state = u)
-  kModeAdjResNl = 7,  // psi^T dR/dt, nonlinear model (state = u)
   kModeMass = 8,      // mass matrix (getMatType MASS)
   kModeMassDV = 9,    // dv[e] += coef[d] phi^T dM_e/dt phi (state = phi)
   kModeOutLin = 10,   // output data at the element nodes, linear model (getOutputData)
@@ -86,14 +83,7 @@ struct ElemArgs {
   const int *first;
   double *res;
   long res_stride;
-  // thickness-derivative modes (' = d/dt_e, all outputs accumulate):
-  //  kModeAdjDV (state = phi, u2 = path u):
-  //    dv[e] += coef[2d] phi^T K' phi + coef[2d+1] phi^T G'(u) phi
-  //    res   += coef[2d+1] d(phi^T G(u) phi)/du
-  //  kModeAdjRes* (state = u): dv[e] += coef[d] psi^T dR_e/dt
-  const double *u2;
-  const double *psi;
-  long u2_stride, psi_stride;
+  // kModeMassDV (state = phi): dv[e] += coef[d] phi^T dM_e/dt phi
   const double *coef;
   double *dv;
   // output modes: out[((d nelems + e) 4 + node) 31 + k], ys = yield stress
@@ -146,11 +136,17 @@ struct XptArgs {
   double *dfdX;
   long dX_stride;
   int terms;
+  // launch_dv_kernel: dv[e] += the scalars' thickness derivatives (coef[4d],
+  // coef[4d+1], coef[4d+2]; may be null); res (6 per node, stride as phi; may
+  // be null) += coef[4d+1] d(phi^T G_e(u) phi)/du
+  double *dv, *res;
 };
-// work: 12 doubles per element and design; node_corner[node_ptr[n]..] lists
+// work: 24 doubles per element and design; node_corner[node_ptr[n]..] lists
 // the places 4 element + corner of node n
 hipError_t launch_xpt_kernel(const XptArgs &args, int nnodes, int nbatch, const int *node_ptr, const int *node_corner,
                              double *work, hipStream_t stream);
+hipError_t launch_dv_kernel(const XptArgs &args, int nnodes, int nbatch, const int *node_ptr, const int *node_corner,
+                            double *work, hipStream_t stream);
 
 // variant: the compiled schedule of the matrix modes (kModeKLin, kModeKNl,
 // kModeG, kModeJac*): bit 0 reads the BSR blocks at the scatter (default:

@@ -3344,7 +3344,7 @@ struct shellgpu_buckling {
   shellgpu_factor *F = nullptr;
   // device: path u, work vectors, Lanczos basis Q and K Q, coefficients
   double *u = nullptr, *res = nullptr, *f0 = nullptr, *Q = nullptr, *KQ = nullptr, *hv = nullptr, *dsig = nullptr;
-  double *ph = nullptr, *gv = nullptr, *psi = nullptr, *dcoef = nullptr;  // dcoef: 6 per design
+  double *ph = nullptr, *gv = nullptr, *psi = nullptr, *dcoef = nullptr;  // dcoef: 4 per design
   std::vector<double> sig;
   bool solved = false;
   int steps = 0;
@@ -3453,7 +3453,7 @@ int shellgpu_buckling_create(shellgpu_ctx *ctx, int model, double sigma, int nev
         hipMalloc((void **)&B->KQ, v * (m + 1)) != hipSuccess ||
         hipMalloc((void **)&B->hv, sizeof(double) * lz_doubles(n, nb, m)) != hipSuccess ||
         hipMalloc((void **)&B->dsig, sizeof(double) * nb) != hipSuccess ||
-        hipMalloc((void **)&B->dcoef, sizeof(double) * 6 * nb) != hipSuccess) {
+        hipMalloc((void **)&B->dcoef, sizeof(double) * 4 * nb) != hipSuccess) {
       rc = ferr(ctx, 2, "out of device memory (Lanczos basis)");
       goto fail;
     }
@@ -3729,11 +3729,8 @@ int shellgpu_buckling_add_eigen_sens(shellgpu_buckling *B, const double *coef, d
   int rc = 0;
   VecOps vo;
   if ((rc = vo.init(ctx, n, nb))) return rc;
-  // coefficient layout: [0, 2 nb) pairs for the thickness kernels, [2 nb,
-  // 6 nb) quadruples for the coordinate kernel
-  double *c2 = B->dcoef, *c4 = B->dcoef + 2 * nb;
   HIPCALL(ctx, hipMemsetAsync(B->gv, 0, sizeof(double) * (size_t)n * nb, ctx->stream));
-  std::vector<double> hc(6 * nb, 0.0);
+  std::vector<double> hc(4 * nb, 0.0);
   for (int j = 0; j < nev; j++) {
     bool any = false;
     for (int d = 0; d < nb; d++) any = any || coef[(size_t)d * nev + j] != 0.0;
@@ -3746,21 +3743,13 @@ int shellgpu_buckling_add_eigen_sens(shellgpu_buckling *B, const double *coef, d
     for (int d = 0; d < nb; d++) {
       // d lambda = -(phi^T K' phi + lambda phi^T G' phi - lambda psi^T R') / (phi^T G phi)
       const double f = -coef[(size_t)d * nev + j] / pgp[d];
-      hc[2 * d] = f;
-      hc[2 * d + 1] = f * B->lam[d][j];
-      hc[2 * nb + 4 * d] = f;
-      hc[2 * nb + 4 * d + 1] = f * B->lam[d][j];
-      hc[2 * nb + 4 * d + 2] = 0.0;
+      hc[4 * d] = f;
+      hc[4 * d + 1] = f * B->lam[d][j];
+      hc[4 * d + 2] = 0.0;
     }
-    HIPCALL(ctx, hipMemcpyAsync(B->dcoef, hc.data(), sizeof(double) * 6 * nb, hipMemcpyHostToDevice, ctx->stream));
-    ElemArgs a = base_args(ctx, B->ph);
-    a.u2 = B->u;
-    a.u2_stride = n;
-    a.coef = c2;
-    a.dv = dfdt;
-    a.res = B->gv;
-    if ((rc = run_colored(ctx, kModeAdjDV, a))) return rc;
-    if (dfdX && (rc = run_xpt(ctx, B->ph, B->u, nullptr, c4, 0, kXptK | kXptG, dfdX))) return rc;
+    HIPCALL(ctx, hipMemcpyAsync(B->dcoef, hc.data(), sizeof(double) * 4 * nb, hipMemcpyHostToDevice, ctx->stream));
+    if ((rc = run_dv(ctx, B->ph, B->u, nullptr, B->dcoef, 0, kXptK | kXptG, dfdt, B->gv))) return rc;
+    if (dfdX && (rc = run_xpt(ctx, B->ph, B->u, nullptr, B->dcoef, 0, kXptK | kXptG, dfdX))) return rc;
     HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
   }
   // path adjoint: dR/du psi = sum_j f_j lambda_j d(phi_j^T G phi_j)/du, with
@@ -3793,22 +3782,14 @@ int shellgpu_buckling_add_eigen_sens(shellgpu_buckling *B, const double *coef, d
     }
   }
   for (int d = 0; d < nb; d++) {
-    hc[d] = -1.0;
-    hc[2 * nb + 4 * d] = 0.0;
-    hc[2 * nb + 4 * d + 1] = 0.0;
-    hc[2 * nb + 4 * d + 2] = -1.0;
+    hc[4 * d] = 0.0;
+    hc[4 * d + 1] = 0.0;
+    hc[4 * d + 2] = -1.0;
   }
-  HIPCALL(ctx, hipMemcpyAsync(B->dcoef, hc.data(), sizeof(double) * 6 * nb, hipMemcpyHostToDevice, ctx->stream));
+  HIPCALL(ctx, hipMemcpyAsync(B->dcoef, hc.data(), sizeof(double) * 4 * nb, hipMemcpyHostToDevice, ctx->stream));
   const int nonlin = B->model == SHELLGPU_NONLINEAR;
-  if (dfdt) {
-    ElemArgs a = base_args(ctx, B->u);
-    a.psi = B->psi;
-    a.psi_stride = n;
-    a.coef = c2;
-    a.dv = dfdt;
-    if ((rc = run_colored(ctx, nonlin ? kModeAdjResNl : kModeAdjResLin, a))) return rc;
-  }
-  if (dfdX && (rc = run_xpt(ctx, nullptr, B->u, B->psi, c4, nonlin, kXptR, dfdX))) return rc;
+  if (dfdt && (rc = run_dv(ctx, nullptr, B->u, B->psi, B->dcoef, nonlin, kXptR, dfdt, nullptr))) return rc;
+  if (dfdX && (rc = run_xpt(ctx, nullptr, B->u, B->psi, B->dcoef, nonlin, kXptR, dfdX))) return rc;
   HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
   return 0;
 }
@@ -4047,20 +4028,13 @@ int shellgpu_frequency_add_eigen_sens(shellgpu_frequency *F, const double *coef,
       HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
     }
     if (!dfdt) continue;
-    // stiffness term: (c, 0) pairs of the thickness-adjoint kernel
+    // stiffness term
     for (int d = 0; d < nb; d++) {
-      hc[2 * d] = coef[(size_t)d * nev + j] / pmp[d];
-      hc[2 * d + 1] = 0.0;
+      hc[4 * d] = coef[(size_t)d * nev + j] / pmp[d];
+      hc[4 * d + 1] = hc[4 * d + 2] = hc[4 * d + 3] = 0.0;
     }
-    HIPCALL(ctx, hipMemcpyAsync(ctx->d_coef, hc.data(), sizeof(double) * 2 * nb, hipMemcpyHostToDevice, ctx->stream));
-    {
-      ElemArgs a = base_args(ctx, F->ph);
-      a.u2 = nullptr;
-      a.res = nullptr;
-      a.coef = ctx->d_coef;
-      a.dv = dfdt;
-      if ((rc = run_colored(ctx, kModeAdjDV, a))) return rc;
-    }
+    HIPCALL(ctx, hipMemcpyAsync(ctx->d_coef, hc.data(), sizeof(double) * 4 * nb, hipMemcpyHostToDevice, ctx->stream));
+    if ((rc = run_dv(ctx, F->ph, nullptr, nullptr, ctx->d_coef, 0, kXptK, dfdt, nullptr))) return rc;
     HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
     // mass term: one coefficient per design
     for (int d = 0; d < nb; d++) hc[d] = -coef[(size_t)d * nev + j] * F->lam[d][j] / pmp[d];

@@ -1,5 +1,5 @@
-// xpt_kernels.hip -- nodal-coordinate derivatives of the element scalars of
-// the buckling sensitivities:
+// xpt_kernels.hip -- coordinate, thickness and path derivatives of the
+// element scalars of the buckling sensitivities:
 //
 //   s_K = phi^T K_e phi,   s_G = phi^T G_e(u) phi,   s_R = psi^T R_e(u)
 //
@@ -44,6 +44,9 @@
 // every strain 12 times: s_G + s_K of 19,691 elements 6 x 246 us -> 45 us,
 // s_R 34, s_K 25, and 4.5 us for the sums per node; a lane per element would
 // need four times the registers and leave three quarters of the GPU idle.
+// The thickness derivatives need the forward half only (two wavefronts per
+// SIMD): against half a wavefront per element with the 24 columns of B in LDS,
+// s_G of 19,691 elements 6 x 58 us -> 15 us, s_R 6 x 24 -> 13, s_K 6 x 26 -> 12.
 #include "elem_common.h"
 #include "shellgpu_internal.h"
 
@@ -51,6 +54,7 @@ namespace shellgpu {
 namespace {
 
 constexpr int kElems = 32;  // per workgroup of 128 threads
+enum { kCoord, kThick, kThickPath };
 
 struct V3 {
   double x, y, z;
@@ -144,7 +148,7 @@ constexpr int bits(int m) { return (m & 1) + ((m >> 1) & 1) + ((m >> 2) & 1) + (
 
 // LDS of one element.  The sources of tying strains are the vectors of WM,
 // then the pairs of PM.
-template <int WM, int PM>
+template <int WM, int PM, int W>
 struct XptSmem {
   static constexpr int kNw = bits(WM), kNs = kNw + bits(PM);
   double q[kNw][24];
@@ -158,7 +162,7 @@ struct XptSmem {
       double g[4][kNs][5];  // per quadrature point, adjoints of the tying fields
       double e8[4][kNw];    // and of the drilling strain
     } b;
-    double part[4][12];     // per lane, adjoints of the normals, then of the coordinates
+    double part[4][W];      // per lane, adjoints of the normals, then of the result
   };
 };
 
@@ -166,9 +170,13 @@ struct XptSmem {
 // scalar needs: s_K and s_M phi; s_G phi, u and the pairs (u,phi),
 // (phi,phi); s_R u, psi and, for the nonlinear model, (u,psi), (u,u).
 // Vectors and pairs outside the masks are never formed.
-template <int WM, int PM>
+//
+// OUT: kCoord, the gradient in the coordinates; kThick, the scalars with the
+// section's thickness derivative, into a.dv; kThickPath, those and
+// d s_G / du (s_G is affine in u: the adjoint of Q(u, phi) and e1(u) alone)
+template <int WM, int PM, int OUT>
 __global__ __launch_bounds__(4 * kElems) void xpt_kernel(XptArgs a, double *out) {
-  using SM = XptSmem<WM, PM>;
+  using SM = XptSmem<WM, PM, OUT == kThickPath ? 24 : 12>;
   constexpr int NW = SM::kNw, NS = SM::kNs;
   constexpr bool kPhi = WM & 1, kU = (WM >> 1) & 1, kPsi = (WM >> 2) & 1;
   constexpr bool kGeo = kPhi && kU && (PM & 3) == 3;
@@ -363,6 +371,7 @@ __global__ __launch_bounds__(4 * kElems) void xpt_kernel(XptArgs a, double *out)
   // ---- the scalar's terms and the adjoints of its strains ----
   const double thick = a.thick[design * a.nelems + e];
   const Section sec = make_section(a.mat, thick);
+  const Section vsec = OUT == kCoord ? sec : make_section_dt(a.mat, thick);  // of the value
   const double eth = a.temp ? a.mat.cte * a.temp[design * a.nelems + e] : 0.0;
   const double det = I.det;
   double value = 0.0;  // of the integrand: the adjoint of the determinant
@@ -380,27 +389,36 @@ __global__ __launch_bounds__(4 * kElems) void xpt_kernel(XptArgs a, double *out)
   if constexpr (kPhi) {
     double ep[9], Cep[9];
     linear_strain(wi[0], ep);
-    apply_c(sec, ep, Cep);
+    apply_c(vsec, ep, Cep);
     value += c[0] * dot9(ep, Cep);
+    if constexpr (OUT == kCoord) {
 #pragma unroll
-    for (int i = 0; i < 9; i++) sb[wi[0]][i] += 2.0 * c[0] * det * Cep[i];
+      for (int i = 0; i < 9; i++) sb[wi[0]][i] += 2.0 * c[0] * det * Cep[i];
+    }
     if constexpr (kGeo) {
       double q0[9], q1[9], Cq[9];
       pair_strain(0, q0);
       pair_strain(1, q1);
-      apply_c(sec, eu, Ceu);
+      apply_c(vsec, eu, Ceu);
       value += c[1] * (2.0 * dot9(q0, Cep) + dot9(q1, Ceu));
       const double w = c[1] * det;
-      apply_c(sec, q0, Cq);
+      if constexpr (OUT == kCoord) {
+        apply_c(sec, q0, Cq);
 #pragma unroll
-      for (int i = 0; i < 9; i++) {
-        sb[wi[0]][i] += 2.0 * w * Cq[i];
-        sb[pi[0]][i] += 2.0 * w * Cep[i];
-        sb[pi[1]][i] += w * Ceu[i];
+        for (int i = 0; i < 9; i++) {
+          sb[wi[0]][i] += 2.0 * w * Cq[i];
+          sb[pi[1]][i] += w * Ceu[i];
+        }
       }
-      apply_c(sec, q1, Cq);
+      if constexpr (OUT == kThickPath) apply_c(sec, ep, Cep);
+      if constexpr (OUT != kThick) {
+        apply_c(sec, q1, Cq);
 #pragma unroll
-      for (int i = 0; i < 9; i++) sb[wi[1]][i] += w * Cq[i];
+        for (int i = 0; i < 9; i++) {
+          sb[pi[0]][i] += 2.0 * w * Cep[i];
+          sb[wi[1]][i] += w * Cq[i];
+        }
+      }
     }
   }
   if constexpr (kRes) {
@@ -420,10 +438,10 @@ __global__ __launch_bounds__(4 * kElems) void xpt_kernel(XptArgs a, double *out)
         for (int i = 0; i < 9; i++) et[i] += 0.5 * q[i];
       }
     }
-    apply_c(sec, et, Ceu);
-    apply_c(sec, es, Ces);
+    apply_c(vsec, et, Ceu);
     value += c[2] * dot9(es, Ceu);
     const double w = c[2] * det;
+    apply_c(sec, es, Ces);
 #pragma unroll
     for (int i = 0; i < 9; i++) {
       sb[wi[1]][i] += w * Ces[i];
@@ -439,11 +457,149 @@ __global__ __launch_bounds__(4 * kElems) void xpt_kernel(XptArgs a, double *out)
       }
     }
   }
+  if constexpr (OUT != kCoord) {
+    double dv = value * det;
+    dv += __shfl_xor(dv, 1);
+    dv += __shfl_xor(dv, 2);
+    if (active && p == 0 && a.dv) a.dv[design * a.nelems + e] += dv;
+    if constexpr (OUT == kThick) return;
+  }
+  // adjoint of a source's tying fields here
+  auto fields_adjoint = [&](const double b[9], double g[5]) {
+    const V3 m0 = b[0] * x[0] + b[2] * x[1] + b[7] * x[2], m1 = b[2] * x[0] + b[1] * x[1] + b[6] * x[2],
+             m2 = b[7] * x[0] + b[6] * x[1];
+    g[kG11] = x[0].x * m0.x + x[1].x * m1.x + x[2].x * m2.x;
+    g[kG22] = x[0].y * m0.y + x[1].y * m1.y + x[2].y * m2.y;
+    g[kG12] = 2.0 * (x[0].x * m0.y + x[1].x * m1.y + x[2].x * m2.y);
+    g[kG23] = 2.0 * (x[0].y * m0.z + x[1].y * m1.z + x[2].y * m2.z);
+    g[kG13] = 2.0 * (x[0].x * m0.z + x[1].x * m1.z + x[2].x * m2.z);
+  };
+  // weight of the source s at tying point t: its field's adjoints of the four
+  // quadrature points
+  auto tying_weight = [&](int t, int s) {
+    double w = 0.0;
+#pragma unroll
+    for (int iq = 0; iq < 4; iq++) {
+      double u, v, Nq[9];
+      quad_point(iq, u, v);
+      tying_interp(u, v, Nq);
+      double Nqt = Nq[0];
+#pragma unroll
+      for (int k = 1; k < 9; k++) Nqt = t == k ? Nq[k] : Nqt;
+      w += Nqt * sm.b.g[iq][s][tying_field(t)];
+    }
+    return w;
+  };
+  // adjoint of the drilling strain of node p
+  auto drill_weight = [&](int s) {
+    double w = 0.0;
+#pragma unroll
+    for (int iq = 0; iq < 4; iq++) {
+      double u, v, qN[4], qa[4], qb[4];
+      quad_point(iq, u, v);
+      shape4(u, v, qN, qa, qb);
+      w += (p == 0 ? qN[0] : p == 1 ? qN[1] : p == 2 ? qN[2] : qN[3]) * sm.b.e8[iq][s];
+    }
+    return w;
+  };
+  if constexpr (OUT == kThickPath) {
+    constexpr int A = wi[1], B = wi[0], P = pi[0];
+    const double *b = sb[P], *l = sb[A];
+    const V3 U0b[2] = {b[3] * U1[B][0] + b[5] * U1[B][1], b[5] * U1[B][0] + b[4] * U1[B][1]};
+    const V3 U1b[2] = {V3{l[3], l[5], 0.0} + b[3] * U0[B][0] + b[5] * U0[B][1],
+                       V3{l[5], l[4], 0.0} + b[5] * U0[B][0] + b[4] * U0[B][1]};
+    V3 uxb = zero3(), ueb = zero3(), d0b = zero3(), dxb = zero3(), deb = zero3();
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const V3 P0 = comb(U0b[k], F.T[0], F.T[1], F.T[2]), P1 = comb(U1b[k], F.T[0], F.T[1], F.T[2]);
+      uxb += x[k].x * P0 + z[k].x * P1;
+      ueb += x[k].y * P0 + z[k].y * P1;
+      d0b += x[k].z * P0 + z[k].z * P1;
+      dxb += x[k].x * P1;
+      deb += x[k].y * P1;
+    }
+    double gl[5], gp[5];
+    fields_adjoint(l, gl);
+    fields_adjoint(b, gp);
+    V3 qb[4], db[4];  // displacements and directors of the nodes
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      qb[m] = Na[m] * uxb + Nb[m] * ueb;
+      db[m] = N[m] * d0b + Na[m] * dxb + Nb[m] * deb;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+      sm.b.g[p][A][i] = gl[i];
+      sm.b.g[p][P][i] = gp[i];
+    }
+    sm.b.e8[p][A] = l[8];
+    __syncthreads();
+#pragma unroll 1
+    for (int t = p; t < 9; t += 4) {
+      double u, v, tN[4], tNa[4], tNb[4];
+      const int f = tying_field(t);
+      const double wl = tying_weight(t, A), wp = tying_weight(t, P);
+      tying_point(t, u, v);
+      shape4(u, v, tN, tNa, tNb);
+      V3 fx, fe, d = zero3(), tn = zero3(), tux = zero3(), tue = zero3(), td = zero3();
+      const V3 at = sum(tNa, X), bt = sum(tNb, X);
+      grad_u(B, tNa, tNb, fx, fe);
+#pragma unroll
+      for (int m = 0; m < 4; m++) {
+        d += tN[m] * director(B, m);
+        tn += tN[m] * load3(&sm.fn[3 * m]);
+      }
+      if (f == kG11) {
+        tux = wl * at + wp * fx;
+      } else if (f == kG22) {
+        tue = wl * bt + wp * fe;
+      } else if (f == kG12) {
+        tux = 0.5 * (wl * bt + wp * fe);
+        tue = 0.5 * (wl * at + wp * fx);
+      } else if (f == kG23) {
+        td = 0.5 * (wl * bt + wp * fe);
+        tue = 0.5 * (wl * tn + wp * d);
+      } else {
+        td = 0.5 * (wl * at + wp * fx);
+        tux = 0.5 * (wl * tn + wp * d);
+      }
+#pragma unroll
+      for (int m = 0; m < 4; m++) {
+        qb[m] += tNa[m] * tux + tNb[m] * tue;
+        db[m] += tN[m] * td;
+      }
+    }
+    const double w = drill_weight(A), hw = 0.5 * w;
+    const V3 sxb = hw * (nx1.x * nf.T[1] - nx2.x * nf.T[0]), seb = hw * (nx1.y * nf.T[1] - nx2.y * nf.T[0]);
+    const V3 rotb = -w * cross(nf.T[0], nf.T[1]);
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      const V3 qm = qb[m] + nNa[m] * sxb + nNb[m] * seb;
+      V3 rm = cross(load3(&sm.fn[3 * m]), db[m]);
+      if (m == p) rm += rotb;
+      double *o = &sm.part[p][6 * m];
+      o[0] = qm.x;
+      o[1] = qm.y;
+      o[2] = qm.z;
+      o[3] = rm.x;
+      o[4] = rm.y;
+      o[5] = rm.z;
+    }
+    __syncthreads();
+    if (!active) return;
+    double *dst = out + (design * a.nelems + e) * 24 + 6 * p;
+#pragma unroll
+    for (int i = 0; i < 6; i++)
+      dst[i] = ((sm.part[0][6 * p + i] + sm.part[1][6 * p + i]) + sm.part[2][6 * p + i]) + sm.part[3][6 * p + i];
+    return;
+  }
   // adjoints of the directors at the point (values and gradients)
   V3 d0b[NW], dxb[NW], deb[NW];
 #pragma unroll
   for (int s = 0; s < NW; s++) d0b[s] = dxb[s] = deb[s] = zero3();
-  if constexpr (kPhi) {
+  if constexpr (kPhi && OUT == kCoord) {
     if (c[3] != 0.0) {
       // mass moments of TACSIsoShellConstitutive with tOffset = 0
       const double m0 = a.mat.rho * thick, m2 = a.mat.rho * thick * thick * thick / 12.0;
@@ -467,13 +623,7 @@ __global__ __launch_bounds__(4 * kElems) void xpt_kernel(XptArgs a, double *out)
     xb[0] += 2.0 * (b[0] * y0 + b[2] * y1 + b[7] * y2);
     xb[1] += 2.0 * (b[2] * y0 + b[1] * y1 + b[6] * y2);
     xb[2] += 2.0 * (b[7] * y0 + b[6] * y1);
-    const V3 m0 = b[0] * x[0] + b[2] * x[1] + b[7] * x[2], m1 = b[2] * x[0] + b[1] * x[1] + b[6] * x[2],
-             m2 = b[7] * x[0] + b[6] * x[1];
-    gb[s][kG11] = x[0].x * m0.x + x[1].x * m1.x + x[2].x * m2.x;
-    gb[s][kG22] = x[0].y * m0.y + x[1].y * m1.y + x[2].y * m2.y;
-    gb[s][kG12] = 2.0 * (x[0].x * m0.y + x[1].x * m1.y + x[2].x * m2.y);
-    gb[s][kG23] = 2.0 * (x[0].y * m0.z + x[1].y * m1.z + x[2].y * m2.z);
-    gb[s][kG13] = 2.0 * (x[0].x * m0.z + x[1].x * m1.z + x[2].x * m2.z);
+    fields_adjoint(b, gb[s]);
   }
   V3 Tb[3] = {zero3(), zero3(), zero3()};
 #pragma unroll
@@ -561,18 +711,7 @@ __global__ __launch_bounds__(4 * kElems) void xpt_kernel(XptArgs a, double *out)
     double u, v, tN[4], tNa[4], tNb[4], w[NS];
     const int f = tying_field(t);
 #pragma unroll
-    for (int s = 0; s < NS; s++) w[s] = 0.0;
-#pragma unroll
-    for (int iq = 0; iq < 4; iq++) {
-      double Nq[9];
-      quad_point(iq, u, v);
-      tying_interp(u, v, Nq);
-      double Nqt = Nq[0];
-#pragma unroll
-      for (int k = 1; k < 9; k++) Nqt = t == k ? Nq[k] : Nqt;
-#pragma unroll
-      for (int s = 0; s < NS; s++) w[s] += Nqt * sm.b.g[iq][s][f];
-    }
+    for (int s = 0; s < NS; s++) w[s] = tying_weight(t, s);
     tying_point(t, u, v);
     shape4(u, v, tN, tNa, tNb);
     const V3 at = sum(tNa, X), bt = sum(tNb, X);
@@ -626,15 +765,7 @@ __global__ __launch_bounds__(4 * kElems) void xpt_kernel(XptArgs a, double *out)
   V3 Tnb[3] = {zero3(), zero3(), zero3()}, x1b = zero3(), x2b = zero3(), cb = zero3();
 #pragma unroll
   for (int s = 0; s < NW; s++) {
-    double w = 0.0;
-#pragma unroll
-    for (int iq = 0; iq < 4; iq++) {
-      double u, v, qN[4], qa[4], qb[4];
-      quad_point(iq, u, v);
-      shape4(u, v, qN, qa, qb);
-      const double Nn = p == 0 ? qN[0] : p == 1 ? qN[1] : p == 2 ? qN[2] : qN[3];
-      w += Nn * sm.b.e8[iq][s];
-    }
+    const double w = drill_weight(s);
     V3 sx, se;
     grad_u(s, nNa, nNb, sx, se);
     cb += -w * load3(&sm.q[s][6 * p + 3]);
@@ -687,16 +818,25 @@ __global__ __launch_bounds__(4 * kElems) void xpt_kernel(XptArgs a, double *out)
   dst[2] = o.z;
 }
 
-// dfdX[node] += the node's parts of its elements' gradients, in element order
-__global__ __launch_bounds__(256) void xpt_gather_kernel(XptArgs a, int nnodes, const int *__restrict__ ptr,
-                                                         const int *__restrict__ corner, const double *__restrict__ g) {
+// dst[node] += the node's W values of its elements' gradients, in element order
+template <int W>
+__global__ __launch_bounds__(256) void xpt_gather_kernel(int n, int nelems, const int *__restrict__ ptr,
+                                                         const int *__restrict__ corner, const double *__restrict__ g,
+                                                         double *dst, long stride) {
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= 3 * nnodes) return;
-  const int n = i / 3, d = i - 3 * n;
-  const long o = blockIdx.y * (long)a.nelems * 12 + d;
+  if (i >= W * n) return;
+  const int node = i / W, d = i - W * node;
+  const long o = blockIdx.y * (long)nelems * (4 * W) + d;
   double s = 0.0;
-  for (int k = ptr[n]; k < ptr[n + 1]; k++) s += g[o + 3L * corner[k]];
-  a.dfdX[blockIdx.y * a.dX_stride + i] += s;
+  for (int k = ptr[node]; k < ptr[node + 1]; k++) s += g[o + (long)W * corner[k]];
+  dst[blockIdx.y * stride + i] += s;
+}
+
+template <int W>
+void gather(const XptArgs &a, int nnodes, int nbatch, const int *node_ptr, const int *node_corner, const double *work,
+            double *dst, long stride, hipStream_t stream) {
+  hipLaunchKernelGGL(xpt_gather_kernel<W>, dim3((W * nnodes + 255) / 256, nbatch), dim3(256), 0, stream, nnodes,
+                     a.nelems, node_ptr, node_corner, work, dst, stride);
 }
 
 }  // namespace
@@ -706,19 +846,35 @@ hipError_t launch_xpt_kernel(const XptArgs &args, int nnodes, int nbatch, const 
   if (args.nelems <= 0) return hipSuccess;
   const dim3 grid((args.nelems + kElems - 1) / kElems, nbatch), block(4 * kElems);
   const int t = args.terms;
-  if ((t & kXptR) && (t & (kXptK | kXptG | kXptM)))  // every vector and pair
-    hipLaunchKernelGGL((xpt_kernel<7, 15>), grid, block, 0, stream, args, work);
-  else if (t & kXptR)  // u, psi; (u, psi) and (u, u) for the nonlinear model
+  if (t & kXptR)  // u, psi; (u, psi) and (u, u) for the nonlinear model
     if (args.nonlin)
-      hipLaunchKernelGGL((xpt_kernel<6, 12>), grid, block, 0, stream, args, work);
+      hipLaunchKernelGGL((xpt_kernel<6, 12, kCoord>), grid, block, 0, stream, args, work);
     else
-      hipLaunchKernelGGL((xpt_kernel<6, 0>), grid, block, 0, stream, args, work);
+      hipLaunchKernelGGL((xpt_kernel<6, 0, kCoord>), grid, block, 0, stream, args, work);
   else if (t & kXptG)  // phi, u; (u, phi) and (phi, phi)
-    hipLaunchKernelGGL((xpt_kernel<3, 3>), grid, block, 0, stream, args, work);
+    hipLaunchKernelGGL((xpt_kernel<3, 3, kCoord>), grid, block, 0, stream, args, work);
   else  // phi alone: s_K, s_M
-    hipLaunchKernelGGL((xpt_kernel<1, 0>), grid, block, 0, stream, args, work);
-  hipLaunchKernelGGL(xpt_gather_kernel, dim3((3 * nnodes + 255) / 256, nbatch), dim3(256), 0, stream, args, nnodes,
-                     node_ptr, node_corner, work);
+    hipLaunchKernelGGL((xpt_kernel<1, 0, kCoord>), grid, block, 0, stream, args, work);
+  gather<3>(args, nnodes, nbatch, node_ptr, node_corner, work, args.dfdX, args.dX_stride, stream);
+  return hipGetLastError();
+}
+
+hipError_t launch_dv_kernel(const XptArgs &args, int nnodes, int nbatch, const int *node_ptr, const int *node_corner,
+                            double *work, hipStream_t stream) {
+  if (args.nelems <= 0) return hipSuccess;
+  const dim3 grid((args.nelems + kElems - 1) / kElems, nbatch), block(4 * kElems);
+  if (args.terms & kXptR)
+    if (args.nonlin)
+      hipLaunchKernelGGL((xpt_kernel<6, 12, kThick>), grid, block, 0, stream, args, work);
+    else
+      hipLaunchKernelGGL((xpt_kernel<6, 0, kThick>), grid, block, 0, stream, args, work);
+  else if (args.res) {
+    hipLaunchKernelGGL((xpt_kernel<3, 3, kThickPath>), grid, block, 0, stream, args, work);
+    gather<6>(args, nnodes, nbatch, node_ptr, node_corner, work, args.res, args.stride, stream);
+  } else if (args.terms & kXptG)
+    hipLaunchKernelGGL((xpt_kernel<3, 3, kThick>), grid, block, 0, stream, args, work);
+  else
+    hipLaunchKernelGGL((xpt_kernel<1, 0, kThick>), grid, block, 0, stream, args, work);
   return hipGetLastError();
 }
 

@@ -87,3 +87,53 @@ def test_more_designs_than_one_launch():
         g = g.download().reshape(nb, -1)
     assert np.abs(g[0]).max() > 0
     assert np.array_equal(g[0], g[-1]) and np.array_equal(g[0], g[nb // 2])
+
+
+@pytest.mark.parametrize("nx,ny", [(1, 1), (31, 1), (8, 4), (11, 3)])
+def test_thickness_and_path_products_around_a_workgroup(nx, ny):
+    # the scalars are cubic in the thickness and s_G is affine in the path, so
+    # five-point and two-point differences are exact: 1e-10 is their round-off
+    conn, X = random_mesh(nx, ny, seed=5 * nx + ny)
+    nn, ne = X.shape[0], conn.shape[0]
+    rng = np.random.default_rng(nx + 1)
+    thick = rng.uniform(0.002, 0.02, (2, ne))
+    phi, psi, w = rng.standard_normal((3, 2, 6 * nn))
+    u = 1e-3 * rng.standard_normal((2, 6 * nn))
+    m = O.material()
+    with mesh_ctx(conn, X, thick) as ctx:
+        dphi, dpsi, du = ctx.vector(phi), ctx.vector(psi), ctx.vector(u)
+        out = []
+        for k in range(4):
+            g = ctx.design_vector()
+            if k == 0:
+                ctx.add_mat_dv_sens_inner_product(g, sg.STIFFNESS, dphi)
+            elif k == 1:
+                ctx.add_mat_dv_sens_inner_product(g, sg.GEOMETRIC, dphi, du)
+            else:
+                ctx.add_adj_res_product(g, dpsi, du, model=(sg.LINEAR, sg.NONLINEAR)[k - 2])
+            out.append(g.download().reshape(2, ne))
+        gu = ctx.vector()
+        ctx.eval_mat_sv_sens_inner_product(dphi, gu)
+        gu = gu.download().reshape(2, -1)
+    ref, sens, mag = np.zeros((4, 2, ne)), np.zeros(2), np.zeros(2)
+    for d in range(2):
+        for e in range(ne):
+            idx = (6 * conn[e][:, None] + np.arange(6)).ravel()
+            Xe, p, t = X[conn[e]].ravel(), phi[d, idx], thick[d, e]
+            h = 0.05 * t
+            ref[0, d, e] = five_point(
+                lambda s: p @ O.elem_stiffness(0, m, s, 0.0, Xe, np.zeros(24)) @ p, t, h)
+            ref[1, d, e] = five_point(
+                lambda s: p @ O.elem_geometric_step(m, s, 0.0, Xe, u[d, idx], 1.0) @ p, t, h)
+            for k in range(2):
+                ref[2 + k, d, e] = O.elem_adj_res_dv(k, m, t, 0.0, psi[d, idx], Xe, u[d, idx])
+            c = p @ O.elem_geometric_step(m, t, 0.0, Xe, w[d, idx], 1.0) @ p
+            sens[d] += c
+            mag[d] += abs(c)
+    for k in range(4):
+        err = np.abs(out[k] - ref[k]).max() / np.abs(ref[k]).max()
+        print(k, err)
+        assert err <= 1e-10, k
+    err = np.abs((gu * w).sum(axis=1) - sens) / mag
+    print("path", err)
+    assert err.max() <= 1e-10
