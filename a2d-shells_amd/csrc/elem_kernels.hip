@@ -26,7 +26,8 @@
 //
 // Work split: each half-wavefront (32 lanes) owns one element and its LDS.
 // Strain-Jacobian columns run on lanes 0-23 (B1 after B) and the 24 x 24
-// product as one 3 x 6 register tile per lane.  The geometry per node /
+// product as one 3 x 6 register tile per lane, over the tying, drilling and
+// bending strains apart (their products with C are separate).  The geometry per node /
 // quadrature point / tying point (4 to 9 tasks per element) is spread over
 // the workgroup by (element, point): with two elements per workgroup (one
 // wavefront) it fills lanes the per-element phases would leave idle; the
@@ -82,16 +83,22 @@ struct ElemSmem {
   double drot[96];  // [node][24] d(drill strain at node)/dq
   double etn[4];
   double sig[MT::kStrain ? 36 : 1];  // [qp][9]
-  double dety[MT::kGeo ? 9 : 1];
+  double dety[MT::kStrain ? 9 : 1];
+  // [qp][15]: upper triangle of W^T (w C) W over the 5 tying fields
+  double Mq[MT::kMat ? 60 : 1];
   struct Frames {
     double Tn[36], XTn[36], tXxi[54];
     double tcU[kNB][54], tcd[kNB][27];  // tying derivative coefficients
   };
-  // [strain][24] for one qp.  The adjoint modes, which form no C B
-  // products, keep in Y[0]: five strain vectors [0,45) and two weighted
-  // stress vectors [45,63)
+  // rows of 24 dof columns.  First the tying rows [J | Y] and, but for G, the
+  // drilling Y; then per quadrature point the bending rows [B | Y] and, with
+  // geometric terms, [alpha (3) | beta (2) | S gamma (2)]
+  static constexpr int kTyRows = MT::kTwo ? 36 : 22;
+  static constexpr int kQpRows = (MT::kTwo ? 12 : 6) + (MT::kGeo ? 7 : 0);
+  static constexpr int kQp = 2;  // quadrature points at a time
+  static constexpr int kRows = !MT::kMat ? 0 : (kQp * kQpRows > kTyRows ? kQp * kQpRows : kTyRows);
   struct Cols {
-    double B[kNB][216], Y[kNB][216];
+    double R[kRows > 0 ? 24 * kRows : 1];
   };
   union {
     Frames f;
@@ -156,32 +163,15 @@ __device__ __forceinline__ void dof_abg(const SM &sm, int iq, int k,
 
 enum BVariant { kBLin = 0, kBFull = 1, kBQuad = 2 };
 
-// one column of B_qp (9 strains) for dof k
-// (J: this dof's column of the tying-strain Jacobian, one value per tying point)
+// the bending strains of one column of B_qp from the dof's alpha, beta, gamma
 template <int VAR, class SM>
-__device__ __forceinline__ void build_bcol(const SM &sm, int iq, int k,
-                                           const double J[9], double out[9]) {
-  double u, v, N[4], Na[4], Nb[4];
-  quad_point(iq, u, v);
-  shape4(u, v, N, Na, Nb);
-  double Nt[9], g[5];
-  tying_interp(u, v, Nt);
-  tying_fields(Nt, J, g);
-  const double *Wq = &sm.Wf[25 * iq];
-#pragma unroll
-  for (int r = 0; r < 5; r++) {
-    double acc = 0.0;
-#pragma unroll
-    for (int f = 0; f < 5; f++) acc += Wq[5 * r + f] * g[f];
-    out[tying_row(r)] = acc;
-  }
-  double al[3], be[3], ga[3];
-  dof_abg(sm, iq, k, N, Na, Nb, al, be, ga);
-  double e3 = 0.0, e4 = 0.0, e5 = 0.0;
+__device__ __forceinline__ void bending_col(const SM &sm, int iq, const double al[3], const double be[3],
+                                            const double ga[3], double e[3]) {
+  e[0] = e[1] = e[2] = 0.0;
   if (VAR != kBQuad) {
-    e3 = al[0] * ga[0];
-    e4 = al[1] * ga[1];
-    e5 = al[0] * ga[1] + al[1] * ga[0];
+    e[0] = al[0] * ga[0];
+    e[1] = al[1] * ga[1];
+    e[2] = al[0] * ga[1] + al[1] * ga[0];
   }
   if (VAR != kBLin) {
     const double *U0 = &sm.u0x[9 * iq], *U1 = &sm.u1x[9 * iq];
@@ -189,19 +179,40 @@ __device__ __forceinline__ void build_bcol(const SM &sm, int iq, int k,
     const double p01 = al[0] * U0[1] + al[1] * U0[4] + al[2] * U0[7];
     const double p10 = al[0] * U1[0] + al[1] * U1[3] + al[2] * U1[6];
     const double p11 = al[0] * U1[1] + al[1] * U1[4] + al[2] * U1[7];
-    e3 += be[0] * p10 + ga[0] * p00;
-    e4 += be[1] * p11 + ga[1] * p01;
-    e5 += be[0] * p11 + ga[1] * p00 + ga[0] * p01 + be[1] * p10;
+    e[0] += be[0] * p10 + ga[0] * p00;
+    e[1] += be[1] * p11 + ga[1] * p01;
+    e[2] += be[0] * p11 + ga[1] * p00 + ga[0] * p01 + be[1] * p10;
   }
-  out[3] = e3;
-  out[4] = e4;
-  out[5] = e5;
-  double e8 = 0.0;
-  if (VAR != kBQuad) {
+}
+
+// pair p < 15 of the upper triangle of a 5 x 5 matrix, row by row
+__device__ __forceinline__ int pair_row(int p) { return (int)(0x433222111100000ull >> (4 * p)) & 7; }
+__device__ __forceinline__ int pair_col(int p) { return (int)(0x443432432143210ull >> (4 * p)) & 7; }
+
+// y = D J for one column J of the tying-strain Jacobian, D (9 x 9) = sum_qp
+// Nt^T W^T (w C) W Nt the section stiffness seen by the tying strains
+template <class SM>
+__device__ __forceinline__ void tying_stress(const SM &sm, const double J[9], double y[9]) {
 #pragma unroll
-    for (int m = 0; m < 4; m++) e8 += N[m] * sm.drot[24 * m + k];
+  for (int t = 0; t < 9; t++) y[t] = 0.0;
+#pragma unroll
+  for (int iq = 0; iq < 4; iq++) {
+    double u, v, Nt[9], g[5], m[5];
+    quad_point(iq, u, v);
+    tying_interp(u, v, Nt);
+    tying_fields(Nt, J, g);
+#pragma unroll
+    for (int f = 0; f < 5; f++) {
+      m[f] = 0.0;
+#pragma unroll
+      for (int h = 0; h < 5; h++) {
+        constexpr int off[5] = {0, 5, 9, 12, 14};
+        m[f] += sm.Mq[15 * iq + (f < h ? off[f] + h - f : off[h] + f - h)] * g[h];
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 9; t++) y[t] += Nt[t] * m[tying_field(t)];
   }
-  out[8] = e8;
 }
 
 // Isotropic section stiffness with the entries that are zero by construction
@@ -232,47 +243,44 @@ __device__ __forceinline__ void apply_c(const IsoSection &c, double w,
 
 // second derivative of the tying strains summed with weights dety
 // (the dety * d2(ety)/dq2 terms of addComputeTyingStrainHessian,
-// TACSShellElementModel.h:782-1031)
+// TACSShellElementModel.h:782-1031), added to the tile of rows rr..rr+2 of
+// node n (rr = 0 or 3) and the 6 dofs of node m: displacements couple by one
+// factor of the node pair, a displacement of node nd and a rotation of node nr
+// by another times (e_cr x n_nr)_cd
 template <class SM>
-__device__ __forceinline__ double tying_geo(const SM &sm, int k, int l) {
-  const int n = k / 6, r = k % 6, m = l / 6, rp = l % 6;
-  if (r >= 3 && rp >= 3) return 0.0;
-  if (r < 3 && rp < 3) {
-    if (r != rp) return 0.0;
-    double h = 0.0;
+__device__ __forceinline__ void tying_geo(const SM &sm, int n, int rr, int m, double acc[18]) {
+  const int nd = rr == 0 ? n : m, nr = rr == 0 ? m : n;
+  double h = 0.0, g = 0.0;
 #pragma unroll
-    for (int t = 0; t < 5; t++) {
-      double u, v, N[4], Na[4], Nb[4];
-      tying_point(t, u, v);
-      shape4(u, v, N, Na, Nb);
-      if (t < 2) {
-        h += sm.dety[t] * (Na[n] * Na[m]);
-      } else if (t < 4) {
-        h += sm.dety[t] * (Nb[n] * Nb[m]);
-      } else {
-        h += sm.dety[t] * (0.5 * (Na[n] * Nb[m] + Nb[n] * Na[m]));
-      }
-    }
-    return h;
-  }
-  // one displacement dof (node nd, comp cd) and one rotation dof (node nr, comp cr)
-  const int nd = r < 3 ? n : m, cd = r < 3 ? r : rp;
-  const int nr = r < 3 ? m : n, cr = (r < 3 ? rp : r) - 3;
-  const double *f = &sm.fn[3 * nr];
-  double c[3];
-  c[0] = cr == 0 ? 0.0 : (cr == 1 ? f[2] : -f[1]);
-  c[1] = cr == 0 ? -f[2] : (cr == 1 ? 0.0 : f[0]);
-  c[2] = cr == 0 ? f[1] : (cr == 1 ? -f[0] : 0.0);
-  double h = 0.0;
-#pragma unroll
-  for (int t = 5; t < 9; t++) {
-    double u, v, N[4], Na[4], Nb[4];
+  for (int t = 0; t < 9; t++) {
+    double u, v;
     tying_point(t, u, v);
-    shape4(u, v, N, Na, Nb);
-    const double g = (t < 7) ? Nb[nd] : Na[nd];
-    h += sm.dety[t] * (0.5 * N[nr] * c[cd] * g);
+    // shape values of the two nodes at the tying point, as in shape4
+    const double da = (nd & 1) ? 0.5 : -0.5, db = (nd & 2) ? 0.5 : -0.5;
+    const double ra = (nr & 1) ? 0.5 : -0.5, rb = (nr & 2) ? 0.5 : -0.5;
+    const double dNa = da * (0.5 + db * v), dNb = (0.5 + da * u) * db;
+    const double rNa = ra * (0.5 + rb * v), rNb = (0.5 + ra * u) * rb;
+    if (t < 2)
+      h += sm.dety[t] * (dNa * rNa);
+    else if (t < 4)
+      h += sm.dety[t] * (dNb * rNb);
+    else if (t == 4)
+      h += sm.dety[t] * (0.5 * (dNa * rNb + dNb * rNa));
+    else
+      g += sm.dety[t] * (0.5 * ((0.5 + ra * u) * (0.5 + rb * v)) * (t < 7 ? dNb : dNa));
   }
-  return h;
+  const double f0 = g * sm.fn[3 * nr], f1 = g * sm.fn[3 * nr + 1], f2 = g * sm.fn[3 * nr + 2];
+  const double c[3][3] = {{0.0, -f2, f1}, {f2, 0.0, -f0}, {-f1, f0, 0.0}};  // g (e_cr x n)_cd
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+      if (rr == 0) {
+        if (i == j) acc[6 * i + j] += h;
+        acc[6 * i + 3 + j] += c[j][i];
+      } else {
+        acc[6 * i + j] += c[i][j];
+      }
 }
 
 // Consistent mass of the linearized-rotation shell between nodes ni and nj
@@ -729,7 +737,15 @@ __device__ __forceinline__ void elem_body(const ElemArgs &a) {
   __syncthreads();
 
   // ---- P3: tying-strain Jacobian rows; strains and stresses at the
-  // quadrature points ----
+  // quadrature points; section stiffness over the tying fields ----
+  if constexpr (kMat) {
+    for (int it = lane; it < 60; it += 32) {
+      const int iq = it / 15, p = it - 15 * iq;
+      const double *x = &sm.Wf[25 * iq + pair_row(p)], *y = &sm.Wf[25 * iq + pair_col(p)];
+      sm.Mq[it] = sm.wdet[iq] * (sec.a11 * (x[0] * y[0] + x[5] * y[5]) + sec.a12 * (x[0] * y[5] + x[5] * y[0]) +
+                                 sec.a66 * (x[10] * y[10]) + sec.as * (x[15] * y[15] + x[20] * y[20]));
+    }
+  }
   // lane k < 24 keeps column k of the tying-strain Jacobian (one value per
   // tying point) in registers: only it reads that column when building B
   double Jr[kNB][9];
@@ -844,7 +860,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs &a) {
   if (MT::kOut) return;
 
   // ---- P4: stress resultants at the tying points ----
-  if (kGeo && lane >= 8 && lane < 17) {
+  if ((kGeo || kRes) && lane >= 8 && lane < 17) {
     const int t = lane - 8, f = tying_field(t);
     double acc = 0.0;
 #pragma unroll
@@ -860,16 +876,26 @@ __device__ __forceinline__ void elem_body(const ElemArgs &a) {
     sm.dety[t] = acc;
   }
 
-  // ---- P5: quadrature loop: B columns, residual, B^T C B tile ----
+  if (kRes) elem_sync<EPW>();
+
+  // ---- P5: residual, B^T C B tile ----
+  // Bound by the LDS reads of the tile product (9 doubles for 18 multiply-adds
+  // and a wavefront's two elements), so the rows are as few as the strains
+  // allow: the tying strains enter as J^T D J, D summed over the quadrature
+  // points (9 rows instead of 4 x 5), the drilling strains by their 4 nodal
+  // values, bending by 4 x 3: 25 rows instead of 36 (G 21 + 21 of 36 + 36).
+  // The 36-row form, one quadrature point at a time, held 256 registers and
+  // more; this one 148 (K) to 240 (G), two or three wavefronts per SIMD.
+  // Assemblies before and after: K of 200 x 400 338 -> 243 us, tangent with
+  // residual of 150 x 301 442 -> 261, G of 7 designs of 53 x 107 503 -> 313.
   // lane tile: rows row0..row0+2 (one node's translations or rotations),
   // columns col0..col0+5 (all dofs of node col0 / 6)
   const int row0 = 3 * (lane >> 2), col0 = 6 * (lane & 3);
   // the lane's 18 entries of its BSR block, read now so that the read
-  // completes during the quadrature loop (no other element of this launch
-  // writes the block): 6 % faster than reading them at the scatter for the
-  // linear stiffness of the 200 x 400 cylinder, more for the nonlinear modes
-  // (schedule bit 0 reads them at the scatter instead: fewer live registers
-  // through the loop)
+  // completes during the products (no other element of this launch writes the
+  // block): 12 % faster than reading them at the scatter for the linear
+  // stiffness of the 200 x 400 cylinder, 2 to 3 % for the nonlinear modes
+  // (schedule bit 0 reads them at the scatter instead)
   constexpr bool kEarly = kMat && !MT::kJvp && !(VAR & 1);
   double prev[18];
   double *dst = nullptr;
@@ -893,100 +919,150 @@ __device__ __forceinline__ void elem_body(const ElemArgs &a) {
   for (int i = 0; i < 18; i++) acc[i] = 0.0;
   double racc = 0.0;
 
-  for (int iq = 0; iq < 4; iq++) {
-    if (lane < 24) {
-      double b[9], y[9];
-      if (kNonlin) {
-        build_bcol<kBFull>(sm, iq, lane, Jr[0], b);
-      } else {
-        build_bcol<kBLin>(sm, iq, lane, Jr[0], b);
-      }
-      if (kRes) {
+  // acc += rows of B (at b) times rows of Y (at y), n rows each
+  auto tile_product = [&](const double *b, const double *y, int n) {
 #pragma unroll
-        for (int i = 0; i < 9; i++) racc += b[i] * sm.sig[9 * iq + i];
-      }
-      if (kMat) {
-        apply_c(sec, sm.wdet[iq], b, y);
+    for (int s = 0; s < n; s++)
 #pragma unroll
-        for (int i = 0; i < 9; i++) {
-          sm.c.B[0][24 * i + lane] = b[i];
-          sm.c.Y[0][24 * i + lane] = y[i];
+      for (int i = 0; i < 3; i++) {
+        const double x = b[24 * s + row0 + i];
+#pragma unroll
+        for (int j = 0; j < 6; j++) acc[6 * i + j] += x * y[24 * s + col0 + j];
+      }
+  };
+  double *R = sm.c.R;
+  if (lane < 24) {
+    if (kRes) {
+#pragma unroll
+      for (int t = 0; t < 9; t++) racc += Jr[0][t] * sm.dety[t];
+    }
+    if (kMat) {
+#pragma unroll
+      for (int w = 0; w < kNB; w++) {
+        double y[9];
+        tying_stress(sm, Jr[w], y);
+#pragma unroll
+        for (int t = 0; t < 9; t++) {
+          R[24 * (9 * w + t) + lane] = Jr[w][t];
+          R[24 * (9 * kNB + 9 * w + t) + lane] = y[t];
         }
       }
-      if constexpr (MODE == kModeG) {
-        build_bcol<kBQuad>(sm, iq, lane, Jr[kNB - 1], b);
-        apply_c(sec, sm.wdet[iq], b, y);
+    }
+    if (!kTwo) {  // the drilling strain is linear: no part of B1
+      double dr[4], yd[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int i = 0; i < 9; i++) {
-          sm.c.B[kTwo ? 1 : 0][24 * i + lane] = b[i];
-          sm.c.Y[kTwo ? 1 : 0][24 * i + lane] = y[i];
+      for (int m = 0; m < 4; m++) dr[m] = sm.drot[24 * m + lane];
+#pragma unroll
+      for (int iq = 0; iq < 4; iq++) {
+        double u, v, N[4], Na[4], Nb[4];
+        quad_point(iq, u, v);
+        shape4(u, v, N, Na, Nb);
+        const double e8 = N[0] * dr[0] + N[1] * dr[1] + N[2] * dr[2] + N[3] * dr[3];
+        if (kRes) racc += e8 * sm.sig[9 * iq + 8];
+        const double y8 = sm.wdet[iq] * (sec.drill * e8);
+#pragma unroll
+        for (int m = 0; m < 4; m++) yd[m] += N[m] * y8;
+      }
+      if (kMat) {
+#pragma unroll
+        for (int m = 0; m < 4; m++) R[24 * (18 + m) + lane] = yd[m];
+      }
+    }
+  }
+  if (kMat) {
+    elem_sync<EPW>();
+    if constexpr (kTwo) {  // J0^T D J1 + J1^T D J0
+      tile_product(R, R + 24 * 27, 9);
+      tile_product(R + 24 * 9, R + 24 * 18, 9);
+    } else {
+      tile_product(R, R + 24 * 9, 9);
+      tile_product(sm.drot, R + 24 * 18, 4);
+    }
+    elem_sync<EPW>();
+  }
+  constexpr int kQp = ElemSmem<MODE>::kQp, kQpRows = ElemSmem<MODE>::kQpRows;
+  constexpr int kBend = kTwo ? 12 : 6;  // then alpha, beta, S gamma
+  // rolled: unrolled, the loads of all points are hoisted and spill
+#pragma unroll 1
+  for (int q0 = 0; q0 < 4; q0 += kQp) {
+    if (lane < 24) {
+#pragma unroll 2
+      for (int iq = q0; iq < q0 + kQp; iq++) {
+        double *row = R + 24 * kQpRows * (iq - q0) + lane;
+        double u, v, N[4], Na[4], Nb[4], al[3], be[3], ga[3];
+        quad_point(iq, u, v);
+        shape4(u, v, N, Na, Nb);
+        dof_abg(sm, iq, lane, N, Na, Nb, al, be, ga);
+        // B, C B of the bending strains: [B0 | C B0], for G [B0 | B1 | C B0 | C B1]
+#pragma unroll
+        for (int w = 0; w < kNB; w++) {
+          double b[3];
+          if (w == 1)
+            bending_col<kBQuad>(sm, iq, al, be, ga, b);
+          else if (kNonlin)
+            bending_col<kBFull>(sm, iq, al, be, ga, b);
+          else
+            bending_col<kBLin>(sm, iq, al, be, ga, b);
+          if (kRes) racc += b[0] * sm.sig[9 * iq + 3] + b[1] * sm.sig[9 * iq + 4] + b[2] * sm.sig[9 * iq + 5];
+          if (kMat) {
+            const double det = sm.wdet[iq];
+#pragma unroll
+            for (int i = 0; i < 3; i++) row[24 * (3 * w + i)] = b[i];
+            double *y = row + 24 * (3 * kNB + 3 * w);
+            y[0] = det * (sec.d11 * b[0] + sec.d12 * b[1]);
+            y[24] = det * (sec.d12 * b[0] + sec.d11 * b[1]);
+            y[48] = det * (sec.d66 * b[2]);
+          }
+        }
+        if (kGeo) {
+          const double S00 = sm.sig[9 * iq + 3], S11 = sm.sig[9 * iq + 4], S01 = sm.sig[9 * iq + 5];
+          double *o = row + 24 * kBend;
+          o[0] = al[0];
+          o[24] = al[1];
+          o[48] = al[2];
+          o[72] = be[0];
+          o[96] = be[1];
+          o[120] = S00 * ga[0] + S01 * ga[1];
+          o[144] = S11 * ga[1] + S01 * ga[0];
         }
       }
     }
     if (kMat) {
       elem_sync<EPW>();
+#pragma unroll 1
+      for (int ql = 0; ql < kQp; ql++) {
+        const double *q = R + 24 * kQpRows * ql;
+        if constexpr (kTwo) {
+          tile_product(q, q + 24 * 9, 3);
+          tile_product(q + 24 * 3, q + 24 * 6, 3);
+        } else {
+          tile_product(q, q + 24 * 3, 3);
+        }
+        if (kGeo) {
+          // (alpha_i . alpha_j) (beta_i . S gamma_j + S gamma_i . beta_j)
+          const double *o = q + 24 * kBend;
+          double r[3][7];
 #pragma unroll
-      for (int s = 0; s < 9; s++) {
-        double b[3], y[6];
+          for (int i = 0; i < 3; i++)
 #pragma unroll
-        for (int i = 0; i < 3; i++) b[i] = sm.c.B[0][24 * s + row0 + i];
-        if constexpr (MODE == kModeG) {
-          // B0^T C B1 + B1^T C B0
-          double c[3], z[6];
-#pragma unroll
-          for (int i = 0; i < 3; i++) c[i] = sm.c.B[kTwo ? 1 : 0][24 * s + row0 + i];
+            for (int d = 0; d < 7; d++) r[i][d] = o[24 * d + row0 + i];
 #pragma unroll
           for (int j = 0; j < 6; j++) {
-            y[j] = sm.c.Y[kTwo ? 1 : 0][24 * s + col0 + j];
-            z[j] = sm.c.Y[0][24 * s + col0 + j];
+            double c[7];
+#pragma unroll
+            for (int d = 0; d < 7; d++) c[d] = o[24 * d + col0 + j];
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+              const double aa = r[i][0] * c[0] + r[i][1] * c[1] + r[i][2] * c[2];
+              acc[6 * i + j] += aa * (r[i][3] * c[5] + r[i][4] * c[6] + r[i][5] * c[3] + r[i][6] * c[4]);
+            }
           }
-#pragma unroll
-          for (int i = 0; i < 3; i++)
-#pragma unroll
-            for (int j = 0; j < 6; j++) acc[6 * i + j] += b[i] * y[j] + c[i] * z[j];
-        } else {
-#pragma unroll
-          for (int j = 0; j < 6; j++) y[j] = sm.c.Y[0][24 * s + col0 + j];
-#pragma unroll
-          for (int i = 0; i < 3; i++)
-#pragma unroll
-            for (int j = 0; j < 6; j++) acc[6 * i + j] += b[i] * y[j];
         }
       }
-      elem_sync<EPW>();
+      if (q0 + kQp < 4) elem_sync<EPW>();
     }
   }
-
-  // ---- P6: geometric (stress) terms ----
-  if (kGeo) {
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-      for (int j = 0; j < 6; j++) acc[6 * i + j] += tying_geo(sm, row0 + i, col0 + j);
-    for (int iq = 0; iq < 4; iq++) {
-      double u, v, N[4], Na[4], Nb[4];
-      quad_point(iq, u, v);
-      shape4(u, v, N, Na, Nb);
-      const double S00 = sm.sig[9 * iq + 3], S11 = sm.sig[9 * iq + 4], S01 = sm.sig[9 * iq + 5];
-      double ar[3][3], br[3][3], gr[3][3];
-#pragma unroll
-      for (int i = 0; i < 3; i++) dof_abg(sm, iq, row0 + i, N, Na, Nb, ar[i], br[i], gr[i]);
-#pragma unroll
-      for (int j = 0; j < 6; j++) {
-        double ac[3], bc[3], gc[3];
-        dof_abg(sm, iq, col0 + j, N, Na, Nb, ac, bc, gc);
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-          const double aa = ar[i][0] * ac[0] + ar[i][1] * ac[1] + ar[i][2] * ac[2];
-          const double h = S00 * (br[i][0] * gc[0] + bc[0] * gr[i][0]) +
-                           S11 * (br[i][1] * gc[1] + bc[1] * gr[i][1]) +
-                           S01 * (br[i][0] * gc[1] + bc[0] * gr[i][1] + br[i][1] * gc[0] +
-                                  bc[1] * gr[i][0]);
-          acc[6 * i + j] += aa * h;
-        }
-      }
-    }
-  }
+  if (kGeo) tying_geo(sm, row0 / 6, row0 % 6, col0 / 6, acc);
 
   // ---- inertial terms of addJacobian (TACSShellElement.h:613-648 and the
   // gamma d2Tdotd part of TACSLinearizedRotation::addDirectorJacobian,
@@ -1088,14 +1164,6 @@ __device__ __forceinline__ void elem_body(const ElemArgs &a) {
 
 template <int MODE, int VAR, int EPW>
 __global__ __launch_bounds__(32 * EPW) void elem_kernel(ElemArgs a) {
-  elem_body<MODE, VAR, EPW>(a);
-}
-
-// the same body within the register budget of two wavefronts per SIMD (the
-// compiler spills to scratch memory instead of holding one wavefront with
-// accumulation registers)
-template <int MODE, int VAR, int EPW>
-__global__ __launch_bounds__(32 * EPW) __attribute__((amdgpu_waves_per_eu(2))) void elem_kernel_w2(ElemArgs a) {
   elem_body<MODE, VAR, EPW>(a);
 }
 
@@ -1231,11 +1299,10 @@ static hipError_t launch_mode(const ElemArgs &args, int count, int nbatch, hipSt
   return hipGetLastError();
 }
 
-// elements per workgroup of the wide schedules: 4 (two wavefronts).  On the
-// 200x400 cylinder the stiffness took 90.2 us per colour launch with 4
-// against 91.9 with 8 (four wavefronts, 51 KB of LDS); the tangent, G and
-// the Jacobians, whose LDS for 8 would not fit twice per CU, take 4 either
-// way.
+// elements per workgroup of the wide schedules: 4 (two wavefronts).  With 8
+// (four wavefronts, 60 to 93 KB of LDS) K of the 200 x 400 cylinder takes 295
+// us against 257, the tangent with residual of 150 x 301 348 against 336, and
+// G of 7 designs of 53 x 107 the same.
 template <int MODE>
 constexpr int wide_epw() {
   return 4;
@@ -1244,24 +1311,15 @@ constexpr int wide_epw() {
 template <int MODE, int EPW>
 static void launch_var(int variant, const dim3 &grid, hipStream_t stream, const ElemArgs &a) {
   const dim3 block(32 * EPW);
-  switch (variant & 3) {
-    case 1:
-      hipLaunchKernelGGL((elem_kernel<MODE, 1, EPW>), grid, block, 0, stream, a);
-      break;
-    case 2:
-      hipLaunchKernelGGL((elem_kernel_w2<MODE, 0, EPW>), grid, block, 0, stream, a);
-      break;
-    case 3:
-      hipLaunchKernelGGL((elem_kernel_w2<MODE, 1, EPW>), grid, block, 0, stream, a);
-      break;
-    default:
-      hipLaunchKernelGGL((elem_kernel<MODE, 0, EPW>), grid, block, 0, stream, a);
-  }
+  if (variant & 1)
+    hipLaunchKernelGGL((elem_kernel<MODE, 1, EPW>), grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL((elem_kernel<MODE, 0, EPW>), grid, block, 0, stream, a);
 }
 
 // the matrix modes in every schedule: variant bit 0 = VAR bit 0 (BSR block
-// reads at the scatter instead of before the quadrature loop), bit 1 = the
-// two-wavefront register budget, bit 2 = wide workgroups (wide_epw elements,
+// reads at the scatter instead of before the tile product), bit 1 = nothing,
+// bit 2 = wide workgroups (wide_epw elements,
 // the geometry tasks spread over the workgroup) instead of two elements
 template <int MODE>
 static hipError_t launch_tuned(const ElemArgs &args, int count, int nbatch, int variant, hipStream_t stream) {

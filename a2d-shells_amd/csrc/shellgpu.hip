@@ -412,42 +412,13 @@ ElemArgs base_args(shellgpu_ctx *ctx, const double *u) {
 // one launch per colour, back to back on the stream; with timing enabled one
 // event pair brackets the colour sequence (events between the launches
 // would add about 3 us each to the pass)
-// Schedule of a matrix mode for a launch of n elements (all designs) where
-// neither shellgpu_tune nor shellgpu_set_elem_schedule chose one.  Whole
-// assemblies, us, schedules 0 / 2 (two-wavefront budget) / 4 (wide) / 6 (both):
-//   K        200 x 400           391 / 391 / 564 / 363, 20 x 40  57 /  58 /  55 /  55
-//            8 designs 50 x 100  216 / 216 / 297 / 203, 60 x 120 76 /  76 /  69 /  70
-//   tangent  150 x 301           570 / 571 / 531 / 533, 20 x 40 127 / 129 / 124 / 124
-//   G        200 x 400          1598 /1132 /1516 /1235, 20 x 40 154 / 155 / 151 / 153
-//            7 designs 53 x 107  888 / 690 / 844 / 734
-//   tangent with residual
-//            150 x 301           616 / 615 / 866 / 575, 20 x 40 139 / 139 / 134 / 135
-//            60 x 120            161 / 161 / 148 / 166
-// The wide schedules spread the geometry over 4 elements; the two-wavefront
-// budget pays once a SIMD has two wavefronts (1,024 SIMDs, half a wavefront per
-// element), and for the tangent its spills cost what it gains.
-int auto_schedule(int mode, long n) {
-  switch (mode) {
-    case kModeKNl:
-      return 4;
-    case kModeG:
-      return 2;
-    case kModeJacNl:
-      return n <= 2048 ? 4 : 6;
-    default:
-      return 6;
-  }
-}
-
 int run_colored(shellgpu_ctx *ctx, int mode, ElemArgs a) {
   int rc = 0;
   if ((rc = record_begin(ctx, ctx->elem_ev))) return rc;
   for (int c = 0; c < ctx->ncolors; c++) {
     a.elems = ctx->d_color_elems + ctx->h_color_ptr[c];
     const int nb = ctx->h_color_ptr[c + 1] - ctx->h_color_ptr[c];
-    const int set = ctx->elem_variant[mode & 31];
-    const int v = set >= 0 ? set : auto_schedule(mode, (long)nb * ctx->nbatch);
-    HIPCALL(ctx, launch_elem_kernel(mode, v, a, nb, ctx->nbatch, ctx->stream));
+    HIPCALL(ctx, launch_elem_kernel(mode, ctx->elem_variant[mode & 31], a, nb, ctx->nbatch, ctx->stream));
   }
   if (ctx->timing) ctx->elem_launches += ctx->ncolors;
   return record_end(ctx, ctx->elem_ev);

@@ -35,10 +35,16 @@ struct shellgpu_ctx {
   // fit with the elements of most neighbours first (shellgpu_tune chooses)
   int coloring = 0;
   // compiled schedule of each element-kernel mode (launch_elem_kernel's
-  // variant) chosen by shellgpu_tune or shellgpu_set_elem_schedule, -1: by the
-  // launch's size; and the tuner's report
+  // variant); shellgpu_tune and shellgpu_set_elem_schedule choose another, and
+  // the tuner's report.  The default, four elements per workgroup, is the
+  // fastest for every size measured (us, schedules 0 / 1 / 4 / 5):
+  //   K        200 x 400 285 / 308 / 257 / 292, 20 x 40 48 / 50 / 46 / 48
+  //   tangent  150 x 301 378 / 390 / 341 / 352, 20 x 40 77 / 79 / 73 / 75
+  //   G        200 x 400 743 / 755 / 690 / 703, 20 x 40 88 / 90 / 85 / 87
+  //   tangent with residual
+  //            150 x 301 369 / 382 / 335 / 343, 20 x 40 81 / 82 / 78 / 78
   int elem_variant[32];
-  shellgpu_ctx() { std::fill(elem_variant, elem_variant + 32, -1); }
+  shellgpu_ctx() { std::fill(elem_variant, elem_variant + 32, 4); }
   std::string schedule;
 
   shellgpu::Material mat = shellgpu::make_material(70e9, 0.3, 2700.0, 0.0, 10.0);

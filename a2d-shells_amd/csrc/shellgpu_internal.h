@@ -150,9 +150,9 @@ hipError_t launch_dv_kernel(const XptArgs &args, int nnodes, int nbatch, const i
 
 // variant: the compiled schedule of the matrix modes (kModeKLin, kModeKNl,
 // kModeG, kModeJac*): bit 0 reads the BSR blocks at the scatter (default:
-// before the quadrature loop), bit 1 two-wavefront register budget, bit 2
-// wide workgroups (4 elements, the geometry spread over them, instead of
-// 2); other modes ignore it
+// before the tile product), bit 1 nothing (every schedule keeps the
+// two-wavefront register budget), bit 2 wide workgroups (4 elements, the
+// geometry spread over them, instead of 2); other modes ignore it
 constexpr int kElemVariants = 8;
 hipError_t launch_elem_kernel(int mode, int variant, const ElemArgs &args, int count, int nbatch,
                               hipStream_t stream);
