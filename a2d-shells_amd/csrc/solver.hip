@@ -47,9 +47,9 @@
 // Lanczos.  Shift-invert Lanczos on (K + sigma G)^{-1} K in the K inner
 // product with full re-orthogonalisation (SEP::solve + EPBucklingShiftInvert,
 // src/bpmat/GSEP.cpp:202-244, 485-599), run in lock-step for every design of
-// the batch.  Re-orthogonalisation is classical Gram-Schmidt applied twice
-// (two GEMV pairs per step against the stored K q_j), the cached K q_j
-// removing the reference's one K-SpMV per inner product.  Ritz values are
+// the batch.  Re-orthogonalisation is one classical Gram-Schmidt pass
+// over the basis after the three-term recurrence, against the stored K q_j,
+// which saves the reference's one K-SpMV per inner product.  Ritz values are
 // converted by lambda = -theta sigma / (1 - theta) and sorted by magnitude
 // (SMALLEST_MAGNITUDE), with a residual-based stopping test (the reference's
 // test is disabled, GSEP.cpp:754-789).
@@ -2684,14 +2684,20 @@ __global__ void shifted_kernel(long n, const double *K, const double *G, const d
 
 // ---- the Lanczos recurrence on the device --------------------------------
 //
-// One step orthogonalises w against the basis (twice: h = KQ^T w, w -= Q h)
-// and normalises it.  The kernels read each basis vector once per product, at
-// the rate of a copy; the coefficients, norms and projection entries stay on
-// the device, so the host waits only where it tests convergence.  Sums run in
-// a fixed order: a workgroup's rows, then the workgroups.  Against library
-// GEMVs with a host wait after each and a start vector made on the host, 16
-// load cases of a 32,000-quad box beam 206 -> 161 ms (one step reads the 16
-// bases four times, 5.5 TB/s), a 20 x 40 cylinder 13.5 -> 10.5 ms.
+// One step takes from w its parts along the last two basis vectors (the
+// three-term recurrence: in exact arithmetic w has no others), orthogonalises
+// the rest against the whole basis (h = KQ^T w, w -= Q h) and normalises it.
+// The second pass starts from a w without cancellation ahead, so it leaves
+// round-off of |w| along the basis, as a second full pass would: two full
+// passes read the bases four times a step and gave the same loads (error
+// against 64-bit references 2.1e-10, 2.0e-10 now, of a 20 x 40 cylinder).
+// The kernels read each basis vector once per product, at the rate of a copy;
+// the coefficients, norms and projection entries stay on the device, so the
+// host waits only where it tests convergence.  Sums run in a fixed order: a
+// workgroup's rows, then the workgroups.  16 load cases of a 32,000-quad box
+// beam: 206 ms with library GEMVs, a host wait after each and a start vector
+// made on the host, 161 with these kernels and two full passes; 132 -> 116 ms
+// (after other steps) by the single full pass, a 20 x 40 cylinder 10.5 -> 9.8.
 constexpr int kLzThreads = 256;
 constexpr int kLzPairs = 4;                             // row pairs per thread
 constexpr int kLzRows = 2 * kLzThreads * kLzPairs;      // rows per workgroup
@@ -2883,8 +2889,8 @@ struct LanczosOut {
   std::vector<std::vector<double>> T, R;
 };
 
-// Lanczos in the K inner product, designs in lock-step, full CGS2
-// re-orthogonalisation.  mode 0: w = A^{-1} K q (shift-invert, A = K +
+// Lanczos in the K inner product, designs in lock-step, full
+// re-orthogonalisation after the three-term recurrence.  mode 0: w = A^{-1} K q (shift-invert, A = K +
 // sigma G factored in F); mode 1: w = K^{-1} (-G q) (buckling mode, F
 // factors K); mode 2: w = A^{-1} K q with the argument K holding the mass
 // matrix M and A = K - sigma M (generalised shift-invert, M inner product).
@@ -2944,14 +2950,17 @@ int lanczos(shellgpu_ctx *ctx, shellgpu_factor *F, shellgpu_mat *K, shellgpu_mat
     }
     if ((rc = shellgpu_vec_zero_bcs(ctx, qn))) return rc;
     for (int pass = 0; pass < 2; pass++) {
+      // the operator is self-adjoint in the basis' inner product: the first
+      // pass takes the two vectors with a part beyond round-off
+      const int j0 = pass == 0 ? std::max(0, k - 1) : 0, k1 = k + 1 - j0;
       const double sg = pass == 0 ? sgn : 1.0;
-      hipLaunchKernelGGL(lz_dots_kernel, grid, dim3(kLzThreads), 0, ctx->stream, n, k + 1, KQ, stride, qn, sg, part,
-                         ldp);
+      hipLaunchKernelGGL(lz_dots_kernel, grid, dim3(kLzThreads), 0, ctx->stream, n, k1, KQ + j0 * stride, stride, qn,
+                         sg, part, ldp);
       // few chunks: every workgroup of the update adds them up itself
       const bool few = chunks <= 16;
       if (!few)
-        hipLaunchKernelGGL(lz_finish_kernel, dim3(k + 1, nb), dim3(64), 0, ctx->stream, chunks, part, ldp, h);
-      hipLaunchKernelGGL(lz_update_kernel, grid, dim3(kLzThreads), 0, ctx->stream, n, k + 1, Q, stride,
+        hipLaunchKernelGGL(lz_finish_kernel, dim3(k1, nb), dim3(64), 0, ctx->stream, chunks, part, ldp, h);
+      hipLaunchKernelGGL(lz_update_kernel, grid, dim3(kLzThreads), 0, ctx->stream, n, k1, Q + j0 * stride, stride,
                          few ? part : h, few ? chunks : 1, ldp, sg, qn, ab + k, 2 * ldp, pass == 0);
     }
     if ((rc = normalise(qn, Kqn, ab + ldp + k))) return rc;
