@@ -53,6 +53,8 @@ struct shellgpu_ctx {
   std::vector<int> h_bc_nodes, h_bc_mask;
   int *d_bc_nodes = nullptr, *d_bc_mask = nullptr;
   double *d_bc_vals = nullptr;
+  int *d_bc_rows = nullptr;  // the masks per node, for a mesh of bc_rows nodes
+  int bc_rows = 0;
 
   double *d_thick = nullptr, *d_temp = nullptr;
   bool same_designs = false;  // every design has the same thickness and temperature

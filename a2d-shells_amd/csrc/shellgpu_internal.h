@@ -81,6 +81,9 @@ struct ElemArgs {
   // matrix modes: per element the blocks it writes rather than adds to
   // (first-touch bits, see shellgpu_ctx::d_first); null: add to every block
   const int *first;
+  // matrix modes, with `first`: per node the mask of its BC rows, which are
+  // written as rows of the identity; null: none
+  const int *bc;
   double *res;
   long res_stride;
   // kModeMassDV (state = phi): dv[e] += coef[d] phi^T dM_e/dt phi
