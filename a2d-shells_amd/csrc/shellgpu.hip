@@ -540,7 +540,7 @@ void shellgpu_destroy(shellgpu_ctx *ctx) {
   void *bufs[] = {ctx->d_conn, ctx->d_rowp,     ctx->d_cols,    ctx->d_blk, ctx->d_diag, ctx->d_tpos,
                   ctx->d_color_elems, ctx->d_X, ctx->d_bc_nodes, ctx->d_bc_mask,
                   ctx->d_bc_vals, ctx->d_thick, ctx->d_temp, ctx->d_coef, ctx->d_first,
-                  ctx->d_nptr, ctx->d_corner, ctx->d_xg, ctx->d_bc_rows};
+                  ctx->d_nptr, ctx->d_xg, ctx->d_bc_rows};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   drop_events(ctx->elem_ev);
@@ -647,8 +647,9 @@ int shellgpu_set_mesh(shellgpu_ctx *ctx, int nnodes, int nelems, const int *conn
   if (rc) return rc;
   if ((rc = upload(ctx, &ctx->d_conn, conn, 4L * nelems))) return rc;
   if ((rc = upload(ctx, &ctx->d_X, Xpts, 3L * nnodes))) return rc;
+  nep.insert(nep.end(), n2c.begin(), n2c.end());
   if ((rc = upload(ctx, &ctx->d_nptr, nep.data(), nep.size()))) return rc;
-  if ((rc = upload(ctx, &ctx->d_corner, n2c.data(), n2c.size()))) return rc;
+  ctx->d_corner = ctx->d_nptr + nnodes + 1;
   if ((rc = upload(ctx, &ctx->d_rowp, ctx->h_rowp.data(), ctx->h_rowp.size()))) return rc;
   if ((rc = upload(ctx, &ctx->d_cols, ctx->h_cols.data(), ctx->h_cols.size()))) return rc;
   if ((rc = upload(ctx, &ctx->d_blk, ctx->h_blk.data(), ctx->h_blk.size()))) return rc;

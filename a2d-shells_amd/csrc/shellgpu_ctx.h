@@ -28,8 +28,9 @@ struct shellgpu_ctx {
   int *d_first = nullptr;
   double *d_X = nullptr;
   // per node n the places 4 element + corner where it stands, in element
-  // order: d_corner[d_nptr[n]..d_nptr[n + 1])
-  int *d_nptr = nullptr, *d_corner = nullptr;
+  // order: d_corner[d_nptr[n]..d_nptr[n + 1]) (one allocation)
+  int *d_nptr = nullptr;
+  const int *d_corner = nullptr;
 
   // element colouring: 0 greedy first fit in element order, 1 greedy first
   // fit with the elements of most neighbours first (shellgpu_tune chooses)
