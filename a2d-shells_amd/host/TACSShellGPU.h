@@ -244,7 +244,7 @@ class TACSSchurMat : public TACSMat {
 
 // TACSPc (src/bpmat/KSM.h:209-230).  TACSSchurPc(mat, levFill, fill,
 // reorder) (src/bpmat/TACSSchurMat.h:59-214) factors the matrix it is
-// bound to; here that factorisation is the level-set block Cholesky of the
+// bound to; here that factorisation is the multifrontal Cholesky of the
 // shellgpu library whatever levFill says (a complete factorisation, which
 // is what levFill = 1e6 gives in the reference).
 class TACSPc : public TACSObject {

@@ -464,7 +464,7 @@ def stiffness_kernel_label(schedule):
     """The stiffness kernel the timed assembly ran: its tuned schedule."""
     elem = schedule.get("elem", {}).get("stiffness")
     if elem is None:
-        return "elem_kernel<0> (stiffness), default schedule 0: " + "two elements per workgroup"
+        return "elem_kernel<0> (stiffness), default schedule 4: wide workgroups"
     v = elem["schedule"]
     return f"elem_kernel<0> (stiffness), tuned schedule {v}: {schedule['schedules'][v]}" + (
         "" if v & 4 else ", two elements per workgroup")

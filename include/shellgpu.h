@@ -233,11 +233,12 @@ int shellgpu_vec_set_bcs(shellgpu_ctx *ctx, double *x);
 
 /* ---- direct solver (TACSPc, src/bpmat/KSM.h:209-230) ------------------ */
 /* Replaces TACSSchurPc's AMD-ordered complete block LU (src/bpmat/
- * TACSSchurMat.cpp:944-1652): nodes are ordered by breadth-first level sets
- * from a seed set, which makes the matrix block tridiagonal; the level
- * blocks are factored densely on the GPU for every design of the batch.
- * Seed nodes (e.g. one boundary ring) set the level structure; without a
- * seed a pseudo-peripheral node is used. */
+ * TACSSchurMat.cpp:944-1652): a multifrontal Cholesky over a nested
+ * dissection of the mesh, every front of a tree level and every design of the
+ * batch in one launch.  SHELLGPU_FACTOR=cr or thomas in the environment
+ * selects a block tridiagonal factor over breadth-first level sets instead;
+ * its levels start from the seed nodes (e.g. one boundary ring), without a
+ * seed from a pseudo-peripheral node. */
 int shellgpu_set_ordering_seed(shellgpu_ctx *ctx, int n, const int *nodes);
 int shellgpu_factor_create(shellgpu_ctx *ctx, shellgpu_factor **F);
 void shellgpu_factor_destroy(shellgpu_factor *F);
