@@ -335,7 +335,7 @@ __device__ __forceinline__ double mass_entry(const MassTile &m, int i, int j) {
 // workgroups the 32 lanes are half of one wavefront, whose LDS operations
 // complete in issue order: waiting for its own LDS operations and keeping
 // the compiler from moving memory operations across suffices, and the
-// workgroup's wavefronts then run their quadrature loops independently.
+// workgroup's wavefronts then run their products independently.
 template <int EPW>
 __device__ __forceinline__ void elem_sync() {
   if constexpr (EPW == 2) {
@@ -355,8 +355,8 @@ __device__ __forceinline__ void elem_sync() {
 //
 // VAR selects a compiled schedule of the same arithmetic (chosen per mode
 // and mesh by shellgpu_tune): bit 0 reads the lane's BSR block entries at
-// the scatter instead of before the quadrature loop (fewer live registers
-// through the loop).
+// the scatter instead of before the tile products (fewer live registers
+// through them).
 template <int MODE, int VAR, int EPW>
 __device__ __forceinline__ void elem_body(const ElemArgs &a) {
   using MT = ModeTraits<MODE>;
