@@ -2824,8 +2824,12 @@ __global__ __launch_bounds__(kLzThreads) void lz_update_kernel(int n, int k1, co
     if (r0 + 2 * kLzThreads * p < n) *reinterpret_cast<lzv2 *>(w + base + at[p]) = wv[p];
 }
 
-// beta = sqrt(w.kw) from the chunks' parts, w and kw scaled by 1 / beta (zero
-// where beta is)
+// beta = sqrt(w.kw) from the chunks' parts, w and kw scaled by 1 / beta.  In
+// the recurrence an exhausted basis leaves zero or less by round-off: beta and
+// the vectors are zero.  A start vector (null beta) of no positive norm is
+// scaled all the same, to NaN, and a NaN stays one: the projection then has no
+// eigenvalues, which the caller is told, instead of zeros that pass for
+// converged ones.
 __global__ __launch_bounds__(kLzThreads) void lz_scale_kernel(int n, const double *__restrict__ part, int chunks,
                                                               double *w, double *kw, double *beta, int ld_beta) {
   __shared__ double red[kLzThreads / 64];
@@ -2835,9 +2839,10 @@ __global__ __launch_bounds__(kLzThreads) void lz_scale_kernel(int n, const doubl
   s = wave_sum(s);
   if ((t & 63) == 0) red[t >> 6] = s;
   __syncthreads();
-  const double b = sqrt(fmax((red[0] + red[1]) + (red[2] + red[3]), 0.0));
+  const double ss = (red[0] + red[1]) + (red[2] + red[3]);
+  const double b = beta && ss < 0.0 ? 0.0 : sqrt(ss);
   if (blockIdx.x == 0 && t == 0 && beta) beta[(long)blockIdx.y * ld_beta] = b;
-  const double inv = b > 0.0 ? 1.0 / b : 0.0;
+  const double inv = !beta || b > 0.0 ? 1.0 / b : 0.0;
   const long base = (long)blockIdx.y * n;
 #pragma unroll
   for (int p = 0; p < kLzPairs; p++) {

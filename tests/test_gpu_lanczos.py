@@ -1,7 +1,8 @@
 """The Lanczos kernels at their edges: a vector shorter than one workgroup's
 rows (2,048), just below and above, more workgroups than the update adds up
 itself (16), more basis vectors than one tile (64), and odd design counts;
-loads against scipy on the assembled K and G."""
+loads against scipy on the assembled K and G; start vectors of no positive
+norm are refused."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -51,5 +52,44 @@ def test_loads_match_scipy(na, nc, nb, nev):
         for j in range(min(nev, 3)):
             phi = B.eigenvector(j)[d][free]
             assert abs(phi @ (k @ phi) - 1.0) <= 1e-8
+    B.destroy()
+    ctx.close()
+
+
+def _context(nb, rho=2700.0, same=False, clamped=False):
+    cyl = Cylinder(4, 8)
+    ctx = sg.Context(0)
+    ctx.set_mesh(cyl.conn, cyl.Xpts)
+    ctx.set_material(70e9, 0.3, rho)
+    if clamped:
+        ctx.set_bcs(np.arange(cyl.nnodes, dtype=np.int32), np.full(cyl.nnodes, 63, np.int32))
+    else:
+        ctx.set_bcs(*cyl.bcs())
+    ctx.set_designs(np.full((nb, cyl.nelems), 0.002) if same else
+                    np.random.default_rng(1).uniform(0.0015, 0.0025, (nb, cyl.nelems)))
+    return cyl, ctx
+
+
+@pytest.mark.parametrize("nb", [1, 2])
+@pytest.mark.parametrize("rho,clamped", [(0.0, False), (-2700.0, False), (2700.0, True)])
+def test_frequencies_without_a_positive_mass_are_refused(rho, clamped, nb):
+    """M zero or negative, or no free dof: the start vector's M norm is not
+    positive, and no frequencies exist."""
+    _, ctx = _context(nb, rho, clamped=clamped)
+    fr = ctx.frequency(sigma=0.0, nev=2, max_lanczos=40, tol=1e-10)
+    with pytest.raises(sg.ShellGPUError, match="error 6"):
+        fr.solve()
+    fr.destroy()
+    ctx.close()
+
+
+# sigma 0: buckling mode (identical designs) and shift estimate; 1e5: given shift
+@pytest.mark.parametrize("sigma", [0.0, 1e5])
+@pytest.mark.parametrize("nb,same", [(1, False), (2, False), (2, True)])
+def test_buckling_without_a_free_dof_is_refused(sigma, nb, same):
+    cyl, ctx = _context(nb, same=same, clamped=True)
+    B = ctx.buckling(sigma=sigma, nev=2, max_lanczos=40, tol=1e-10)
+    with pytest.raises(sg.ShellGPUError, match="error 6"):
+        B.solve(force=cyl.edge_load(1.0))
     B.destroy()
     ctx.close()
