@@ -964,6 +964,22 @@ hipError_t upload(T **dst, const std::vector<T> &src) {
   return e;
 }
 
+// workspace for F.chunk designs at once, for fewer where the memory left does
+// not hold it
+hipError_t alloc_work(NdFactor &F) {
+  for (;; F.chunk = (F.chunk + 1) / 2) {
+    hipError_t e = hipMalloc((void **)&F.Q, sizeof(double) * (size_t)F.q_len * F.chunk);
+    for (int k = 0; k < 2 && e == hipSuccess; k++)
+      e = hipMalloc((void **)&F.S[k], sizeof(double) * (size_t)F.s_len[k] * F.chunk);
+    if (e != hipErrorOutOfMemory || F.chunk == 1) return e;
+    (void)hipGetLastError();  // handled here
+    for (double **p : {&F.Q, &F.S[0], &F.S[1]}) {
+      if (*p) (void)hipFree(*p);
+      *p = nullptr;
+    }
+  }
+}
+
 }  // namespace
 
 std::string nd_create(int nn, const std::vector<int> &rowp, const std::vector<int> &cols, const double *X, int nbatch,
@@ -978,18 +994,16 @@ std::string nd_create(int nn, const std::vector<int> &rowp, const std::vector<in
   F.s_len[1] = L.s_len[1];
   blk_base = std::move(L.blk_base);
   blk_ld = std::move(L.blk_ld);
-  // workspace copies: as many designs at once as 4 GiB hold (16 designs of
-  // the 100 x 200 cylinder), which leaves no level short of workgroups
+  // workspace copies: at most as many designs at once as 4 GiB hold (15 of the
+  // 100 x 200 cylinder), which leaves no level short of workgroups
   const double ws = 8.0 * (F.q_len + F.s_len[0] + F.s_len[1]);
   F.chunk = std::max(1, (int)std::min<double>(nbatch, 4294967296.0 / ws));
   F.n = 6L * nn;
   hipError_t e = upload(&F.d_fronts, L.fronts);
   if (e == hipSuccess) e = upload(&F.d_lists, L.lists);
   if (e == hipSuccess) e = hipMalloc((void **)&F.M, sizeof(double) * (size_t)F.per_design * nbatch);
-  if (e == hipSuccess) e = hipMalloc((void **)&F.Q, sizeof(double) * (size_t)F.q_len * F.chunk);
-  for (int k = 0; k < 2 && e == hipSuccess; k++)
-    e = hipMalloc((void **)&F.S[k], sizeof(double) * (size_t)F.s_len[k] * F.chunk);
   if (e == hipSuccess) e = nd_reserve(F, nrhs);
+  if (e == hipSuccess) e = alloc_work(F);
   if (e != hipSuccess)
     return std::string("factor allocation (") + std::to_string((long)(8.0 * F.per_design * nbatch) >> 20) +
            " MiB): " + hipGetErrorString(e);

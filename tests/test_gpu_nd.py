@@ -1,7 +1,8 @@
 """The multifrontal factor (the default SHELLGPU_FACTOR) on matrices of known
 solution: meshes of one front, fronts shorter and longer than a pivot block,
 last blocks of every remainder, fronts longer than the staged vector pieces,
-batches of designs, several vectors per design, and the captured solve."""
+batches of designs, several vectors per design, the captured solve, and
+designs factored a few at a time where the memory left asks for it."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -201,3 +202,51 @@ def test_block_lanczos_solves_blocks(monkeypatch):
         B.destroy()
         ctx.close()
     assert np.abs(out[0] - out[1]).max() <= 1e-8 * np.abs(out[0]).max()
+
+
+def test_designs_are_factored_in_the_memory_that_is_left():
+    """Workspace for all designs at once does not fit beside the panels: the
+    factor takes fewer at a time, with the same bits."""
+    nb, gib = 12, 1 << 27  # gib: doubles
+    cyl = Cylinder(100, 200)
+    # per design 302 MiB of panels and 259 MiB of workspace (3.0 GiB for 12)
+    panels, work = nb * 302 / 1024, nb * 259 / 1024
+    ctx = make((cyl.conn, cyl.Xpts), nb)
+    rowp, cols = ctx.pattern()
+    base = spd_values(rowp, cols, 21)
+    scale = 1.0 + 0.1 * np.arange(nb)
+    x = np.random.default_rng(22).standard_normal((nb, 6 * cyl.nnodes))
+    free = ~bc_mask(cyl.nnodes)
+    x[:, ~free] = 0.0
+    A = sp.bsr_matrix((base, cols, rowp), shape=(6 * cyl.nnodes,) * 2)
+    b = np.stack([scale[d] * np.where(free, A @ x[d], 0.0) for d in range(nb)])
+    K = ctx.matrix()
+    K.set_values(base[None] * scale[:, None, None, None])
+    K.apply_bcs()
+    db, y = ctx.vector(b), ctx.vector()
+
+    def solve():
+        F = ctx.factor()
+        assert abs(F.info()[2] - panels) <= 0.02 * panels
+        F.compute(K)
+        F.apply(db, y)
+        F.destroy()
+        return y.download().reshape(nb, -1)
+
+    ref = solve()
+    assert np.linalg.norm(ref - x) <= TOL * np.linalg.norm(x)
+    # room for the panels and 0.7 of the workspace: for 6 designs, not for 12
+    room = sg.DeviceArray(ctx, int((panels + 0.7 * work) * gib))
+    held, size = [], 32 * gib
+    while size >= gib // 8:
+        try:
+            held.append(sg.DeviceArray(ctx, size))
+        except sg.ShellGPUError:
+            size //= 4
+    room.free()
+    try:
+        assert np.array_equal(solve(), ref)
+    finally:
+        for h in held:
+            h.free()
+    ctx.close()
