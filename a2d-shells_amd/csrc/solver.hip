@@ -101,7 +101,7 @@ struct CholNode {
 struct shellgpu_factor {
   shellgpu_ctx *ctx = nullptr;
   int nbatch = 0;
-  int nlevels = 0;
+  int nlevels = 0;  // of the dissection tree, or of the level order
   int n = 0;  // scalar dofs
   std::vector<int> m;        // dofs per level
   std::vector<long> voff;    // offset of level l in a level-ordered vector
@@ -115,7 +115,7 @@ struct shellgpu_factor {
   int *d_ct_src = nullptr;   // per entry: local index of the next-level node
   int *d_ct_blk = nullptr;   // per entry: the coupling block
   long per_design = 0;       // doubles per design
-  int maxm = 0;
+  int maxm = 0;              // dofs of the largest front or level
   long tmp_elems = 0;        // largest m_l * m_{l-1}
   double *buf = nullptr;     // nbatch * per_design
   double *tmp = nullptr;     // 2 * nbatch * tmp_elems (E P and its transpose)
@@ -997,69 +997,7 @@ int setup_plan(shellgpu_factor *F) {
   shellgpu_ctx *ctx = F->ctx;
   const int nn = ctx->nnodes;
   const std::vector<int> &rowp = ctx->h_rowp, &cols = ctx->h_cols;
-  // breadth-first levels from the seed set
-  std::vector<int> level(nn, -1), queue;
-  queue.reserve(nn);
-  std::vector<int> seeds = ctx->order_seed;
-  if (seeds.empty()) {
-    // pseudo-peripheral node: repeat BFS from the farthest node
-    int start = 0;
-    for (int it = 0; it < 4; it++) {
-      std::fill(level.begin(), level.end(), -1);
-      queue.clear();
-      level[start] = 0;
-      queue.push_back(start);
-      for (size_t h = 0; h < queue.size(); h++) {
-        int v = queue[h];
-        for (int p = rowp[v]; p < rowp[v + 1]; p++)
-          if (level[cols[p]] < 0) {
-            level[cols[p]] = level[v] + 1;
-            queue.push_back(cols[p]);
-          }
-      }
-      start = queue.back();
-    }
-    seeds.push_back(queue.front());
-  }
-  std::fill(level.begin(), level.end(), -1);
-  queue.clear();
-  for (int s : seeds) {
-    if (s < 0 || s >= nn) return ferr(ctx, 1, "ordering seed out of range");
-    if (level[s] < 0) {
-      level[s] = 0;
-      queue.push_back(s);
-    }
-  }
-  for (size_t h = 0; h < queue.size(); h++) {
-    int v = queue[h];
-    for (int p = rowp[v]; p < rowp[v + 1]; p++)
-      if (level[cols[p]] < 0) {
-        level[cols[p]] = level[v] + 1;
-        queue.push_back(cols[p]);
-      }
-  }
-  // unreached components start new level chains after the last level
-  int nl = 0;
-  for (int i = 0; i < nn; i++) nl = std::max(nl, level[i] + 1);
-  for (int i = 0; i < nn; i++)
-    if (level[i] < 0) return ferr(ctx, 1, "mesh graph is disconnected from the ordering seed");
-  F->nlevels = nl;
-  std::vector<int> cnt(nl, 0), node_pos(nn);
-  for (int i = 0; i < nn; i++) cnt[level[i]]++;
-  std::vector<int> noff(nl + 1, 0);
-  for (int l = 0; l < nl; l++) noff[l + 1] = noff[l] + cnt[l];
-  {
-    std::vector<int> fill(noff.begin(), noff.end() - 1);
-    for (int i = 0; i < nn; i++) node_pos[i] = fill[level[i]]++;
-  }
   F->n = 6 * nn;
-  F->m.assign(nl, 0);
-  F->voff.assign(nl + 1, 0);
-  for (int l = 0; l < nl; l++) {
-    F->m[l] = 6 * cnt[l];  // even: the level GEMVs load 16-byte pairs
-    F->voff[l + 1] = F->voff[l] + F->m[l];
-    F->maxm = std::max(F->maxm, F->m[l]);
-  }
 
   // BC dofs (symmetric elimination)
   std::vector<int> isbc(F->n, 0);
@@ -1073,17 +1011,36 @@ int setup_plan(shellgpu_factor *F) {
     return i == j ? mask | 1 << 12 : mask;
   };
 
+  // breadth-first levels from a node set
+  std::vector<int> level(nn), queue;
+  queue.reserve(nn);
+  auto breadth_first = [&](const std::vector<int> &from) {
+    std::fill(level.begin(), level.end(), -1);
+    queue.clear();
+    for (int s : from)
+      if (level[s] < 0) {
+        level[s] = 0;
+        queue.push_back(s);
+      }
+    for (size_t h = 0; h < queue.size(); h++) {
+      const int v = queue[h];
+      for (int p = rowp[v]; p < rowp[v + 1]; p++)
+        if (level[cols[p]] < 0) {
+          level[cols[p]] = level[v] + 1;
+          queue.push_back(cols[p]);
+        }
+    }
+  };
+  std::vector<int> seeds = ctx->order_seed;
+  for (int s : seeds)
+    if (s < 0 || s >= nn) return ferr(ctx, 1, "ordering seed out of range");
+  breadth_first(seeds.empty() ? std::vector<int>{0} : seeds);
+  if ((int)queue.size() < nn) return ferr(ctx, 1, "mesh graph is disconnected from the ordering seed");
+
   // The nested-dissection form (nd_factor.hip) for every mesh and batch; the
   // level forms below only where SHELLGPU_FACTOR asks for one of them.
-  // Factor and solve of one design, this form against the faster level form:
-  // 200 x 400 cylinder 24 and 0.67 ms against 340 and 4.3 ms (cyclic
-  // reduction), 16 designs of 61 x 119 15 against 110 ms, of 100 x 200 2.4
-  // against 4.0 ms per solve (sequential), and the whole analysis of a 20 x
-  // 40 cylinder 17 against 25 ms: no size was found where a level form wins.
-  {
-    const char *env = getenv("SHELLGPU_FACTOR");
-    F->nd = !(env && (strcmp(env, "thomas") == 0 || strcmp(env, "cr") == 0));
-  }
+  const char *env = getenv("SHELLGPU_FACTOR");
+  F->nd = !(env && (strcmp(env, "thomas") == 0 || strcmp(env, "cr") == 0));
   if (F->nd) {
     std::vector<double> X(3 * (size_t)nn);
     HIPCALL(ctx, hipMemcpyAsync(X.data(), ctx->d_X, sizeof(double) * X.size(), hipMemcpyDeviceToHost, ctx->stream));
@@ -1094,6 +1051,8 @@ int setup_plan(shellgpu_factor *F) {
         nd_create(nn, rowp, cols, X.data(), F->nbatch, F->nbatch == 1 ? std::min(kMaxRhs, ctx->nbatch) : 1, F->ndf, base, ld);
     if (!err.empty()) return ferr(ctx, 2, err);
     F->per_design = F->ndf.per_design;
+    F->nlevels = (int)F->ndf.levels.size();
+    for (const NdLevel &lv : F->ndf.levels) F->maxm = std::max(F->maxm, lv.max_m);
     for (int i = 0; i < nn; i++)
       for (int p = rowp[i]; p < rowp[i + 1]; p++) flag[p] = block_flag(i, cols[p]);
     HIPCALL(ctx, hipMalloc((void **)&F->d_bcflag, sizeof(int) * ctx->nnzb));
@@ -1105,31 +1064,37 @@ int setup_plan(shellgpu_factor *F) {
     return 0;
   }
 
-  // Block cyclic reduction when the padded factor (three M x M blocks per
-  // level and design) fits in 85 % of the free device memory, padding the
-  // levels to M adds at most half the unknowns, and the factor holds few
-  // designs; a factor of one design shared by the context's designs (load
-  // cases) solves their vectors together (up to 8, or 16) and reads
-  // itself once per solve.  Otherwise the sequential factorisation.
-  // SHELLGPU_FACTOR=thomas / =cr selects either (cr only where it fits).
+  // level forms: without a seed the levels start from a pseudo-peripheral
+  // node (the farthest from the last, three times)
+  if (seeds.empty())
+    for (int it = 0; it < 3; it++) breadth_first({queue.back()});
+  int nl = 0;
+  for (int i = 0; i < nn; i++) nl = std::max(nl, level[i] + 1);
+  F->nlevels = nl;
+  std::vector<int> cnt(nl, 0), node_pos(nn);
+  for (int i = 0; i < nn; i++) cnt[level[i]]++;
+  std::vector<int> noff(nl + 1, 0);
+  for (int l = 0; l < nl; l++) noff[l + 1] = noff[l] + cnt[l];
+  {
+    std::vector<int> fill(noff.begin(), noff.end() - 1);
+    for (int i = 0; i < nn; i++) node_pos[i] = fill[level[i]]++;
+  }
+  F->m.assign(nl, 0);
+  F->voff.assign(nl + 1, 0);
+  for (int l = 0; l < nl; l++) {
+    F->m[l] = 6 * cnt[l];  // even: the level GEMVs load 16-byte pairs
+    F->voff[l + 1] = F->voff[l] + F->m[l];
+    F->maxm = std::max(F->maxm, F->m[l]);
+  }
+
+  // block cyclic reduction where the padded factor (three M x M blocks per
+  // level and design) fits in 85 % of the free device memory
   {
     const long M = F->maxm;
     size_t freeb = 0, totalb = 0;
     HIPCALL(ctx, hipMemGetInfo(&freeb, &totalb));
     const double need = 3.0 * nl * (double)M * (double)M * 8.0 * F->nbatch;
-    const char *env = getenv("SHELLGPU_FACTOR");
-    const bool fits = nl >= 3 && need <= 0.85 * (double)freeb;
-    const bool uniform = (double)nl * M <= 1.5 * F->n;
-    // cyclic reduction pays off while one level's work is too small to fill
-    // the GPU and the level chain is long (its rounds batch the levels);
-    // with many vectors per solve the sequential factorisation is parallel
-    // enough and reads fewer bytes per solve (half of one inverse per
-    // level, where cyclic reduction reads three padded blocks)
-    const int per = ctx->nbatch / F->nbatch;  // vectors per design of one solve
-    const bool multi_ok = per == 1 || (F->nbatch == 1 && (per <= 8 || per == 16));
-    F->cr = fits && uniform && (long)F->nbatch * M <= 8192 && multi_ok;
-    if (env && strcmp(env, "thomas") == 0) F->cr = false;
-    if (env && strcmp(env, "cr") == 0) F->cr = fits;
+    F->cr = strcmp(env, "cr") == 0 && nl >= 3 && need <= 0.85 * (double)freeb;
   }
   if (F->cr) {
     const long M = F->maxm, M2 = M * M;

@@ -242,7 +242,9 @@ int shellgpu_vec_set_bcs(shellgpu_ctx *ctx, double *x);
 int shellgpu_set_ordering_seed(shellgpu_ctx *ctx, int n, const int *nodes);
 int shellgpu_factor_create(shellgpu_ctx *ctx, shellgpu_factor **F);
 void shellgpu_factor_destroy(shellgpu_factor *F);
-/* number of levels, largest level (dofs), factor memory (GiB, all designs) */
+/* levels of the dissection tree, dofs of the largest front (pivots and
+ * boundary), factor memory (GiB, all designs); under SHELLGPU_FACTOR=cr or
+ * thomas the levels of the mesh and the dofs of the largest */
 int shellgpu_factor_info(shellgpu_factor *F, int *nlevels, int *max_level_dofs, double *gib);
 /* TACSPc::factor (TACSSchurPc::factor, TACSSchurMat.cpp:1430-1510) */
 int shellgpu_factor_compute(shellgpu_factor *F, shellgpu_mat *A);

@@ -204,6 +204,43 @@ def test_block_lanczos_solves_blocks(monkeypatch):
     assert np.abs(out[0] - out[1]).max() <= 1e-8 * np.abs(out[0]).max()
 
 
+@pytest.mark.parametrize("mesh,levels,largest", [("1x3", 1, 36), ("4x8", 2, 192)])
+def test_info_describes_the_fronts(mesh, levels, largest):
+    """4 x 8: 40 nodes, a separator of 8 between leaves of 8 and of 24; the
+    largest front has 24 pivot and 8 boundary nodes."""
+    with make(MESHES[mesh](), 2) as ctx:
+        F = ctx.factor()
+        assert F.info()[:2] == (levels, largest)
+        F.destroy()
+
+
+def test_every_part_of_a_mesh_needs_a_seed():
+    """Two cylinders without a common node: refused until the ordering seed
+    reaches both; then each is solved."""
+    cyl = Cylinder(7, 13)
+    nn = cyl.nnodes
+    mesh = np.concatenate([cyl.conn, cyl.conn + nn]), np.concatenate([cyl.Xpts, cyl.Xpts + 3.0])
+    with make(mesh, 1) as ctx:
+        for seed in ([], [3]):
+            ctx.set_ordering_seed(seed)
+            with pytest.raises(sg.ShellGPUError, match="disconnected"):
+                ctx.factor()
+        ctx.set_ordering_seed([3, 2 * nn])
+        with pytest.raises(sg.ShellGPUError, match="out of range"):
+            ctx.factor()
+        ctx.set_ordering_seed([3, nn + 5])
+        vals, x, b = system(ctx, 1, True, 31)
+        A = ctx.matrix()
+        A.set_values(vals)
+        A.apply_bcs()
+        F = ctx.factor()
+        F.compute(A)
+        y = ctx.vector()
+        F.apply(ctx.vector(b), y)
+        assert np.linalg.norm(y.download() - x.ravel()) <= TOL * np.linalg.norm(x)
+        F.destroy()
+
+
 def test_designs_are_factored_in_the_memory_that_is_left():
     """Workspace for all designs at once does not fit beside the panels: the
     factor takes fewer at a time, with the same bits."""
