@@ -25,11 +25,14 @@ struct NdFactor {
   double *W = nullptr;  // interleaved right-hand sides and solutions of several vectors
 };
 
-// Order, structure and buffers for nbatch designs of the mesh graph; blk_base
-// and blk_ld receive, per BSR block, where it goes in M (base -1: the
-// transpose of a stored block).  Returns an empty string or the error.
-std::string nd_create(int nn, const std::vector<int> &rowp, const std::vector<int> &cols, const double *X, int nbatch,
-                      int nrhs, NdFactor &F, std::vector<long> &blk_base, std::vector<int> &blk_ld);
+// leaves of the dissection: 24 nodes (144 dofs).  Fewer, larger leaves give
+// fewer fronts but more fill (200 x 400 cylinder: 1.45 GB at 24 nodes, 1.33
+// at 16 with a third more fronts, 1.79 at 48)
+constexpr int kNdLeafNodes = 24;
+
+// Buffers of a factor of nbatch designs with the fronts of L, for solves of
+// nrhs vectors per design.  Returns an empty string or the error.
+std::string nd_create(int nn, const NdLayout &L, int nbatch, int nrhs, NdFactor &F);
 void nd_destroy(NdFactor &F);
 // factor the designs' matrices (nnzb blocks of 36 values each, placed by
 // blk_base, blk_ld and blk_flag: bits 6 + c for BC columns, bit 12 for a

@@ -49,10 +49,6 @@ typedef __attribute__((address_space(1))) double gdouble;
 typedef __attribute__((address_space(1))) const v2d gcv2d;
 
 constexpr int kB = 64;  // pivot block
-// leaves of the dissection: 24 nodes (144 dofs).  Fewer, larger leaves give
-// fewer fronts but more fill (200 x 400 cylinder: 1.45 GB at 24 nodes, 1.33
-// at 16 with a third more fronts, 1.79 at 48)
-constexpr int kLeafNodes = 24;
 
 struct LevelArgs {
   const NdDev *fronts;  // the level's first front
@@ -982,18 +978,14 @@ hipError_t alloc_work(NdFactor &F) {
 
 }  // namespace
 
-std::string nd_create(int nn, const std::vector<int> &rowp, const std::vector<int> &cols, const double *X, int nbatch,
-                      int nrhs, NdFactor &F, std::vector<long> &blk_base, std::vector<int> &blk_ld) {
-  NdLayout L = nd_layout(nn, rowp, cols, X, kLeafNodes);
+std::string nd_create(int nn, const NdLayout &L, int nbatch, int nrhs, NdFactor &F) {
   F.nbatch = nbatch;
-  F.levels = std::move(L.levels);
+  F.levels = L.levels;
   F.per_design = L.per_design;
   F.v_len = L.v_len;
   F.q_len = L.q_len;
   F.s_len[0] = L.s_len[0];
   F.s_len[1] = L.s_len[1];
-  blk_base = std::move(L.blk_base);
-  blk_ld = std::move(L.blk_ld);
   // workspace copies: at most as many designs at once as 4 GiB hold (15 of the
   // 100 x 200 cylinder), which leaves no level short of workgroups
   const double ws = 8.0 * (F.q_len + F.s_len[0] + F.s_len[1]);

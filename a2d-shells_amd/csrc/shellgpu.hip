@@ -593,6 +593,7 @@ int shellgpu_set_mesh(shellgpu_ctx *ctx, int nnodes, int nelems, const int *conn
   if (!ctx || nnodes <= 0 || nelems <= 0 || !conn || !Xpts) return set_err(ctx, 1, "invalid mesh arguments");
   for (long i = 0; i < 4L * nelems; i++)
     if (conn[i] < 0 || conn[i] >= nnodes) return set_err(ctx, 1, "connectivity entry out of range");
+  ctx->nd_layout.reset();
   ctx->nnodes = nnodes;
   ctx->nelems = nelems;
   ctx->h_conn.assign(conn, conn + 4L * nelems);
@@ -661,6 +662,7 @@ int shellgpu_set_mesh(shellgpu_ctx *ctx, int nnodes, int nelems, const int *conn
 int shellgpu_set_nodes(shellgpu_ctx *ctx, const double *Xpts) {
   if (!ctx || !Xpts) return set_err(ctx, 1, "invalid node arguments");
   if (ctx->nnodes <= 0 || !ctx->d_X) return set_err(ctx, 1, "set the mesh before the nodes");
+  ctx->nd_layout.reset();
   HIPCALL(ctx, hipMemcpyAsync(ctx->d_X, Xpts, sizeof(double) * 3 * (size_t)ctx->nnodes, hipMemcpyDeviceToDevice,
                               ctx->stream));
   return 0;

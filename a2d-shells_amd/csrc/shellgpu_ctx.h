@@ -3,11 +3,16 @@
 #pragma once
 
 #include <algorithm>
+#include <memory>
 #include <string>
 #include <utility>
 #include <vector>
 
 #include "shellgpu_internal.h"
+
+namespace shellgpu {
+struct NdLayout;
+}
 
 struct shellgpu_ctx {
   int device = 0;
@@ -77,6 +82,10 @@ struct shellgpu_ctx {
 
   // solver state
   std::vector<int> order_seed;  // BFS seed nodes of the level ordering
+  // nested-dissection order and front layout of the mesh, made by the first
+  // factor and shared by the later ones (an analysis has two); dropped with
+  // the mesh or the coordinates it was made from
+  std::shared_ptr<const shellgpu::NdLayout> nd_layout;
   void *blas = nullptr;         // rocblas_handle bound to `stream`
 };
 

@@ -1042,13 +1042,15 @@ int setup_plan(shellgpu_factor *F) {
   const char *env = getenv("SHELLGPU_FACTOR");
   F->nd = !(env && (strcmp(env, "thomas") == 0 || strcmp(env, "cr") == 0));
   if (F->nd) {
-    std::vector<double> X(3 * (size_t)nn);
-    HIPCALL(ctx, hipMemcpyAsync(X.data(), ctx->d_X, sizeof(double) * X.size(), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
-    std::vector<long> base;
-    std::vector<int> ld, flag(ctx->nnzb);
-    const std::string err =
-        nd_create(nn, rowp, cols, X.data(), F->nbatch, F->nbatch == 1 ? std::min(kMaxRhs, ctx->nbatch) : 1, F->ndf, base, ld);
+    if (!ctx->nd_layout) {
+      std::vector<double> X(3 * (size_t)nn);
+      HIPCALL(ctx, hipMemcpyAsync(X.data(), ctx->d_X, sizeof(double) * X.size(), hipMemcpyDeviceToHost, ctx->stream));
+      HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
+      ctx->nd_layout = std::make_shared<const NdLayout>(nd_layout(nn, rowp, cols, X.data(), kNdLeafNodes));
+    }
+    const NdLayout &L = *ctx->nd_layout;
+    std::vector<int> flag(ctx->nnzb);
+    const std::string err = nd_create(nn, L, F->nbatch, F->nbatch == 1 ? std::min(kMaxRhs, ctx->nbatch) : 1, F->ndf);
     if (!err.empty()) return ferr(ctx, 2, err);
     F->per_design = F->ndf.per_design;
     F->nlevels = (int)F->ndf.levels.size();
@@ -1059,8 +1061,8 @@ int setup_plan(shellgpu_factor *F) {
     HIPCALL(ctx, hipMalloc((void **)&F->d_blk_base, sizeof(long) * ctx->nnzb));
     HIPCALL(ctx, hipMalloc((void **)&F->d_blk_ld, sizeof(int) * ctx->nnzb));
     HIPCALL(ctx, hipMemcpy(F->d_bcflag, flag.data(), sizeof(int) * ctx->nnzb, hipMemcpyHostToDevice));
-    HIPCALL(ctx, hipMemcpy(F->d_blk_base, base.data(), sizeof(long) * ctx->nnzb, hipMemcpyHostToDevice));
-    HIPCALL(ctx, hipMemcpy(F->d_blk_ld, ld.data(), sizeof(int) * ctx->nnzb, hipMemcpyHostToDevice));
+    HIPCALL(ctx, hipMemcpy(F->d_blk_base, L.blk_base.data(), sizeof(long) * ctx->nnzb, hipMemcpyHostToDevice));
+    HIPCALL(ctx, hipMemcpy(F->d_blk_ld, L.blk_ld.data(), sizeof(int) * ctx->nnzb, hipMemcpyHostToDevice));
     return 0;
   }
 

@@ -214,6 +214,42 @@ def test_info_describes_the_fronts(mesh, levels, largest):
         F.destroy()
 
 
+def test_order_follows_the_mesh_and_its_nodes():
+    """The factors of a context share one order; new nodes or a new mesh get
+    the order, and so the bits, that a context made with them has."""
+    cyl = Cylinder(12, 20)
+    nodes = [cyl.Xpts, cyl.Xpts * np.array([1.0, 9.0, 0.2]), cyl.Xpts]
+    other = random_mesh(9, 10, 3)
+
+    def solves(ctx, seed):
+        vals, x, b = system(ctx, 1, False, seed)
+        A = ctx.matrix()
+        A.set_values(vals)
+        out = []
+        for _ in range(2):
+            F, y = ctx.factor(), ctx.vector()
+            F.compute(A)
+            F.apply(ctx.vector(b), y)
+            out.append(y.download())
+            assert np.linalg.norm(out[-1] - x.ravel()) <= TOL * np.linalg.norm(x)
+            F.destroy()
+        A.destroy()
+        assert np.array_equal(*out)
+        return out[0]
+
+    got = []
+    with make((cyl.conn, nodes[0]), 1, False) as ctx:
+        for X in nodes:
+            ctx.set_nodes(X)
+            got.append(solves(ctx, 41))
+        ctx.set_mesh(*other)
+        ctx.set_designs(np.full((1, len(other[0])), 0.002))
+        got.append(solves(ctx, 42))
+    for mesh, seed, g in [((cyl.conn, X), 41, h) for X, h in zip(nodes, got)] + [(other, 42, got[-1])]:
+        with make(mesh, 1, False) as ctx:
+            assert np.array_equal(solves(ctx, seed), g)
+
+
 def test_every_part_of_a_mesh_needs_a_seed():
     """Two cylinders without a common node: refused until the ordering seed
     reaches both; then each is solved."""
