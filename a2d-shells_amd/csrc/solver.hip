@@ -1571,7 +1571,7 @@ int shellgpu_factor_compute(shellgpu_factor *F, shellgpu_mat *A) {
   const long ps = F->per_design;
   F->factored = false;
   auto not_spd = [&](int b) {
-    return ferr(ctx, 5, "matrix not positive definite in the level Cholesky (design " + std::to_string(b) +
+    return ferr(ctx, 5, "matrix not positive definite in the Cholesky factorisation (design " + std::to_string(b) +
                             "): for K + sigma G the shift is above the first buckling load");
   };
   if (F->nd) {
@@ -1981,7 +1981,7 @@ static int factor_cr(shellgpu_factor *F) {
   HIPCALL(ctx, hipStreamSynchronize(ctx->stream));
   for (int b = 0; b < nb; b++)
     if (bad[b])
-      return ferr(ctx, 5, "matrix not positive definite in the level Cholesky (design " + std::to_string(b) +
+      return ferr(ctx, 5, "matrix not positive definite in the Cholesky factorisation (design " + std::to_string(b) +
                               "): for K + sigma G the shift is above the first buckling load");
   F->factored = true;
   return 0;

@@ -125,7 +125,7 @@ def test_indefinite_matrix_is_refused_and_named():
     A = ctx.matrix()
     F = ctx.factor()
     A.set_values(bad)
-    with pytest.raises(sg.ShellGPUError, match="design 1"):
+    with pytest.raises(sg.ShellGPUError, match=r"in the Cholesky factorisation \(design 1\)"):
         F.compute(A)
     with pytest.raises(sg.ShellGPUError):
         F.apply(ctx.vector(b), ctx.vector())
