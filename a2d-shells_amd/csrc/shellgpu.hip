@@ -1362,6 +1362,10 @@ int shellgpu_tune(shellgpu_ctx *ctx, int flags) {
     float t[kElemVariants];
     int best = 0;
     for (int v = 0; v < kElemVariants; v++) {
+      if (v & 2) {  // the kernel of schedule v - 2
+        t[v] = t[v & ~2];
+        continue;
+      }
       ctx->elem_variant[mode] = v;
       if ((rc = trial(mode, t[v]))) goto out;
       if (t[v] < t[best]) best = v;
@@ -1375,12 +1379,9 @@ int shellgpu_tune(shellgpu_ctx *ctx, int flags) {
     snprintf(buf + len, sizeof(buf) - len, "]}");
     rep += buf;
   }
-  rep += "}, \"schedules\": [\"block reads before the quadrature loop\", \"block reads at the scatter\", "
-         "\"reads before the loop, 2 wavefronts/SIMD register budget\", "
-         "\"reads at the scatter, 2 wavefronts/SIMD register budget\", "
-         "\"wide workgroups, reads before the loop\", \"wide workgroups, reads at the scatter\", "
-         "\"wide workgroups, reads before the loop, 2 wavefronts/SIMD\", "
-         "\"wide workgroups, reads at the scatter, 2 wavefronts/SIMD\"]}";
+  rep += "}, \"schedules\": [\"block reads before the tile products\", \"block reads at the scatter\", "
+         "\"as 0\", \"as 1\", \"wide workgroups, reads before the tile products\", "
+         "\"wide workgroups, reads at the scatter\", \"as 4\", \"as 5\"]}";
   ctx->schedule = rep;
 out:
   ctx->timing = timing;

@@ -437,7 +437,9 @@ int shellgpu_ks_aggregate(int n, double rho, const double *f, double *ks, double
  * the elements of most neighbours first), and keeps the fastest of each for
  * the context.  Results are the same arithmetic under every schedule. */
 int shellgpu_tune(shellgpu_ctx *ctx, int flags);
-/* the tuner's choices and timings as a JSON object ("{}" before tuning) */
+/* the tuner's choices and timings as a JSON object ("{}" before tuning);
+ * "us" lists schedules 0-7, those with bit 1 with the time of the same kernel
+ * without it */
 int shellgpu_get_schedule(shellgpu_ctx *ctx, char *buf, int len);
 /* force a schedule (0-7: bit 0 block reads at the scatter, bit 1 without
  * effect since every schedule keeps the two-wavefront register budget, bit 2

@@ -1,8 +1,8 @@
 """The autotuner's schedules: every compiled schedule of the matrix-assembly
-kernels (BSR block reads before the quadrature loop or at the scatter, one-
-or two-wavefront register budget, two elements per workgroup or wide
-workgroups of 4 with the geometry spread over them, on colours of
-ragged length) and both element colourings assemble the same matrices and
+kernels (BSR block reads before the tile products or at the scatter, two
+elements per workgroup or wide workgroups of 4 with the geometry spread over
+them, on colours of ragged length; schedules that differ in bit 1 are the same
+kernel, which the tuner times once) and both element colourings assemble the same matrices and
 residuals (the same arithmetic; within round-off of the default schedule,
 which the oracle tests pin), and shellgpu_tune reports and keeps valid
 choices, and that the timing counters count every colour launch."""
@@ -70,6 +70,11 @@ def test_tune_keeps_valid_choices_and_results():
         rep = ctx.tune(coloring=True)
         assert set(rep["elem"]) == {"stiffness", "tangent", "geometric", "jacobian_linear", "jacobian_nonlinear"}
         assert all(0 <= r["schedule"] < 8 and len(r["us"]) == 8 for r in rep["elem"].values())
+        # bit 1 selects nothing: such schedules are neither timed nor chosen
+        for r in rep["elem"].values():
+            assert r["schedule"] & 2 == 0
+            assert [r["us"][v] for v in (2, 3, 6, 7)] == [r["us"][v] for v in (0, 1, 4, 5)]
+        assert [rep["schedules"][v] for v in (2, 3, 6, 7)] == ["as 0", "as 1", "as 4", "as 5"]
         assert rep["coloring"]["colors"] == ctx.ncolors
         # the colouring in force: no two elements of a colour share a node
         col = ctx.colors()
