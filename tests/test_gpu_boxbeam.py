@@ -45,9 +45,13 @@ def make_ctx(b, thick):
     return ctx
 
 
-@pytest.mark.parametrize("factor", ["cr", "thomas"])
+@pytest.mark.parametrize("factor", ["nd", "cr", "thomas"])
 def test_box_beam_load_cases_match_oracle(factor, monkeypatch):
-    monkeypatch.setenv("SHELLGPU_FACTOR", factor)
+    # nd (nested dissection): the default
+    if factor == "nd":
+        monkeypatch.delenv("SHELLGPU_FACTOR", raising=False)
+    else:
+        monkeypatch.setenv("SHELLGPU_FACTOR", factor)
     b = small_beam()
     t = b.panel_thickness(4000)
     forces = np.stack([b.load_case(c) for c in CASES])

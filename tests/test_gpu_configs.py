@@ -5,8 +5,8 @@ B  200 x 400 cylinder (80,000 quads, 482,400 dof) with seeded thickness
    (seed 1234) and radial imperfection (seed 1235), unit axial edge load:
    5-step Newton on the nonlinear model, checked through the oracle's
    nonlinear residual; buckling about the final state, first 5 loads, run
-   with both factorisations (cyclic reduction and the sequential form), which
-   agree within 1e-10 (loads) and 1e-6 rad (principal angles of the modes,
+   with every factorisation (nested dissection, cyclic reduction and the
+   sequential form), which agree within 1e-10 (loads) and 1e-6 rad (principal angles of the modes,
    K inner product); every load within 1e-8 of the Rayleigh quotient of its
    mode with the oracle's K and G(u); K and G(u) themselves against the
    oracle's assembly (row-floored relative error 1e-10; G from the oracle's
@@ -121,8 +121,11 @@ def test_config_b_newton_and_buckling(cyl_b, monkeypatch):
     bc = bc_dofs(cyl.nnodes, cyl.bcs())
     m = O.material()
     runs = {}
-    for factor in ("cr", "thomas"):
-        monkeypatch.setenv("SHELLGPU_FACTOR", factor)
+    for factor in ("nd", "cr", "thomas"):
+        if factor == "nd":  # nested dissection: the default
+            monkeypatch.delenv("SHELLGPU_FACTOR", raising=False)
+        else:
+            monkeypatch.setenv("SHELLGPU_FACTOR", factor)
         log(f"config B (200x400): Newton + buckling, factorisation {factor}")
         with cyl_ctx(cyl, thick) as ctx:
             du, its, rel = ctx.newton_solve(f, nsteps=5, max_iters=20, rtol=1e-10)
@@ -146,15 +149,16 @@ def test_config_b_newton_and_buckling(cyl_b, monkeypatch):
             B.destroy()
         runs[factor] = out
 
-    cr, th = runs["cr"], runs["thomas"]
+    nd, cr, th = runs["nd"], runs["cr"], runs["thomas"]
     log("config B: oracle residual, K, G(u), Rayleigh quotients")
-    # the Newton state solves the oracle's nonlinear residual
-    r = O.assemble_res(1, m, cyl.Xpts, cyl.conn, thick[0], u=cr["u"]) - f
-    r[bc] = 0.0
+    # the Newton states solve the oracle's nonlinear residual
     fr = f.copy()
     fr[bc] = 0.0
-    log(f"  |R_nl(u) - f| / |f| = {np.linalg.norm(r) / np.linalg.norm(fr):.2e}")
-    assert np.linalg.norm(r) <= 1e-9 * np.linalg.norm(fr)
+    for run in (nd, cr):
+        r = O.assemble_res(1, m, cyl.Xpts, cyl.conn, thick[0], u=run["u"]) - f
+        r[bc] = 0.0
+        log(f"  |R_nl(u) - f| / |f| = {np.linalg.norm(r) / np.linalg.norm(fr):.2e}")
+        assert np.linalg.norm(r) <= 1e-9 * np.linalg.norm(fr)
     # K and G(u) against the oracle's assembly at full size
     Kref = O.bsr_apply_bcs(O.assemble_mat(O.KIND_K, 0, m, cyl.Xpts, cyl.conn, thick[0], rowp, cols), rowp, cols,
                            *cyl.bcs())
@@ -167,22 +171,24 @@ def test_config_b_newton_and_buckling(cyl_b, monkeypatch):
     log(f"  K parity {ek:.2e}, G(u) parity {eg:.2e}")
     assert ek <= 1e-10 and eg <= 1e-10
     # each load is the Rayleigh quotient of its mode with the oracle's matrices
-    for j in range(5):
-        p = cr["phi"][j]
-        rq = -(p @ O.bsr_matvec(rowp, cols, Kref, p)) / (p @ O.bsr_matvec(rowp, cols, Gref, p))
-        log(f"  load {j}: {cr['lam'][j]:.12e}, Rayleigh quotient {rq:.12e}")
-        assert abs(rq - cr["lam"][j]) <= 1e-8 * abs(cr["lam"][j])
-    # both factorisations: the same loads and modes
-    dl = np.abs(cr["lam"] - th["lam"]).max() / np.abs(cr["lam"]).max()
-    log(f"  cyclic reduction vs sequential factor: loads {dl:.2e}")
-    assert dl <= 1e-10
-    groups = clusters(cr["lam"])
-    if len(groups) > 1:
-        groups = groups[:-1]  # the last cluster may continue past the 5th load
-    for g in groups:
-        a = k_angle(cr["phi"][g], th["phi"][g], rowp, cols, Kref)
-        log(f"  modes {g}: principal angle {a:.2e} rad")
-        assert a <= 1e-6
+    for run in (nd, cr):
+        for j in range(5):
+            p = run["phi"][j]
+            rq = -(p @ O.bsr_matvec(rowp, cols, Kref, p)) / (p @ O.bsr_matvec(rowp, cols, Gref, p))
+            log(f"  load {j}: {run['lam'][j]:.12e}, Rayleigh quotient {rq:.12e}")
+            assert abs(rq - run["lam"][j]) <= 1e-8 * abs(run["lam"][j])
+    # all factorisations: the same loads and modes
+    for name, run in (("sequential factor", th), ("nested dissection", nd)):
+        dl = np.abs(cr["lam"] - run["lam"]).max() / np.abs(cr["lam"]).max()
+        log(f"  cyclic reduction vs {name}: loads {dl:.2e}")
+        assert dl <= 1e-10
+        groups = clusters(cr["lam"])
+        if len(groups) > 1:
+            groups = groups[:-1]  # the last cluster may continue past the 5th load
+        for g in groups:
+            a = k_angle(cr["phi"][g], run["phi"][g], rowp, cols, Kref)
+            log(f"  modes {g}: principal angle {a:.2e} rad")
+            assert a <= 1e-6
 
 
 # ---------------------------------------------------------------------------

@@ -1,7 +1,7 @@
 """The multifrontal factor (the default SHELLGPU_FACTOR) on matrices of known
 solution: meshes of one front, fronts shorter and longer than a pivot block,
-last blocks of every remainder, fronts longer than the staged vector pieces,
-batches of designs, several vectors per design, the captured solve, and
+last blocks of every remainder, fronts longer than the staged vector pieces, the
+stiffness of a shell of large fronts, batches of designs, several vectors per design, the captured solve, and
 designs factored a few at a time where the memory left asks for it."""
 import numpy as np
 import pytest
@@ -110,6 +110,43 @@ def test_known_solutions(mesh, nb, bcs):
     y = ctx.vector(b)
     F.apply(y, y)
     assert np.array_equal(y.download().reshape(nb, -1), got)
+    F.destroy()
+    ctx.close()
+
+
+def test_shell_stiffness_of_large_fronts():
+    """K of a 201 x 402 cylinder, fronts of 2,400 pivots: one vector, and
+    eleven through the factor of one design.  The solve multiplies by explicit
+    inverses of the fronts' Cholesky factors, whose residuals grow with their
+    condition, at most the root of K's (below 1e9); 1e3 covers the sums'
+    lengths (up to 3,600 terms, 14 levels): 1e3 x 3.2e4 eps."""
+    cyl = Cylinder(201, 402)
+    thick = np.random.default_rng(51).uniform(0.0015, 0.0025, (1, cyl.nelems))
+    ctx = sg.Context(0)
+    ctx.set_mesh(cyl.conn, cyl.Xpts)
+    ctx.set_material(70e9, 0.3)
+    ctx.set_bcs(*cyl.bcs())
+    ctx.set_designs(thick)
+    K = ctx.matrix()
+    ctx.assemble_mattype(sg.STIFFNESS, K)
+    rowp, cols = ctx.pattern()
+    n = 6 * cyl.nnodes
+    A = sp.bsr_matrix((K.design_values(0), cols, rowp), shape=(n, n)).tocsr()
+    F = ctx.factor()
+    F.compute(K)
+    norm = abs(A).sum(1).max()
+    for vectors in (1, 11):
+        ctx.set_designs(np.repeat(thick, vectors, 0))  # one factor, so many vectors
+        b = np.random.default_rng(52).standard_normal((vectors, n))
+        db = ctx.vector(b)
+        ctx.vec_zero_bcs(db)
+        b = db.download().reshape(vectors, n)
+        y = ctx.vector()
+        F.apply(db, y)
+        for x, r in zip(y.download().reshape(vectors, n), b):
+            eta = np.abs(A @ x - r).max() / (norm * np.abs(x).max() + np.abs(r).max())
+            print(vectors, "vectors: backward error", eta)
+            assert eta <= 1e3 * 3.2e4 * 2.3e-16
     F.destroy()
     ctx.close()
 

@@ -13,10 +13,14 @@ pytestmark = pytest.mark.gpu
 
 
 def set_factor(monkeypatch, factor):
-    """cr: block cyclic reduction; thomas: the sequential level factorisation;
-    -block: with block Lanczos (blocks of 4 vectors; cyclic reduction then
-    solves the 4 vectors of a block together)"""
-    monkeypatch.setenv("SHELLGPU_FACTOR", factor.split("-")[0])
+    """nd: the default, the nested-dissection factor; cr: block cyclic
+    reduction; thomas: the sequential level factorisation; -block: with block
+    Lanczos (blocks of 4 vectors; nested dissection and cyclic reduction then
+    solve the 4 vectors of a block together)"""
+    if factor.startswith("nd"):
+        monkeypatch.delenv("SHELLGPU_FACTOR", raising=False)
+    else:
+        monkeypatch.setenv("SHELLGPU_FACTOR", factor.split("-")[0])
     if factor.endswith("-block"):
         monkeypatch.setenv("SHELLGPU_LANCZOS_BLOCK", "4")
 
@@ -31,11 +35,11 @@ def make_ctx(cyl, thick):
     return ctx
 
 
-@pytest.mark.parametrize("factor", ["cr", "thomas"])
+@pytest.mark.parametrize("factor", ["nd", "cr", "thomas"])
 def test_direct_solve_and_gmres(factor, monkeypatch):
-    # cr: block cyclic reduction over the (uniform) ring levels;
-    # thomas: the sequential level Cholesky
-    monkeypatch.setenv("SHELLGPU_FACTOR", factor)
+    # nd: fronts of a nested dissection; cr: block cyclic reduction over the
+    # (uniform) ring levels; thomas: the sequential level Cholesky
+    set_factor(monkeypatch, factor)
     cyl = Cylinder(10, 20)
     thick = np.random.default_rng(1).uniform(0.0015, 0.0025, cyl.nelems)
     ctx = make_ctx(cyl, thick)
@@ -43,7 +47,8 @@ def test_direct_solve_and_gmres(factor, monkeypatch):
     ctx.assemble_mattype(sg.STIFFNESS, K)
     F = ctx.factor()
     nl, mx, _ = F.info()
-    assert nl == cyl.na + 1 and mx == 6 * cyl.nc  # one level per ring
+    if factor != "nd":
+        assert nl == cyl.na + 1 and mx == 6 * cyl.nc  # one level per ring
     F.compute(K)
     rng = np.random.default_rng(2)
     b = rng.standard_normal(6 * cyl.nnodes)
@@ -54,7 +59,7 @@ def test_direct_solve_and_gmres(factor, monkeypatch):
     Kref = O.bsr_apply_bcs(O.assemble_mat(O.KIND_K, 0, O.material(), cyl.Xpts, cyl.conn, thick, rowp, cols),
                            rowp, cols, *cyl.bcs())
     r = O.bsr_matvec(rowp, cols, Kref, x) - b
-    # explicit level inverses: the true residual floor is ~cond * eps
+    # explicit inverses (of the levels, of the fronts): the true residual floor is ~cond * eps
     assert np.linalg.norm(r) <= 1e-6 * np.linalg.norm(b)
     xr = O.band_solve(rowp, cols, Kref, b)
     assert np.abs(x - xr).max() <= 1e-8 * np.abs(xr).max()
@@ -67,7 +72,7 @@ def _subspace_angle(V, W, rowp, cols, Kvals):
     return float(np.arccos(min(1.0, s.min())))
 
 
-@pytest.mark.parametrize("factor", ["cr", "thomas", "thomas-block", "cr-block"])
+@pytest.mark.parametrize("factor", ["nd", "nd-block", "cr", "thomas", "thomas-block", "cr-block"])
 @pytest.mark.parametrize("na,nc", [(20, 40)])
 def test_buckling_matches_oracle(na, nc, factor, monkeypatch):
     set_factor(monkeypatch, factor)
@@ -101,7 +106,7 @@ def test_buckling_matches_oracle(na, nc, factor, monkeypatch):
         i = j
 
 
-@pytest.mark.parametrize("factor", ["cr", "thomas", "thomas-block"])
+@pytest.mark.parametrize("factor", ["nd", "nd-block", "cr", "thomas", "thomas-block"])
 def test_batched_designs_match_single_designs(factor, monkeypatch):
     set_factor(monkeypatch, factor)
     cyl = Cylinder(8, 16, imperfection=(2e-4, 2, 3))
@@ -116,13 +121,14 @@ def test_batched_designs_match_single_designs(factor, monkeypatch):
         assert np.abs(out["lambda"][b] - lam).max() <= 1e-8 * np.abs(lam).max()
 
 
-def test_batched_designs_converging_at_different_steps(monkeypatch):
+@pytest.mark.parametrize("factor", ["nd", "thomas"])
+def test_batched_designs_converging_at_different_steps(factor, monkeypatch):
     """Designs of one batch whose wanted pairs converge at different Lanczos
-    steps (thickness x1, x1.4, x2 under one shift): with the sequential
-    factorisation each design stops solving at its own convergence, and its
-    loads and Ritz residuals still match the oracle's and its own
-    single-design run's."""
-    set_factor(monkeypatch, "thomas")
+    steps (thickness x1, x1.4, x2 under one shift): with the nested-dissection
+    and the sequential factorisation each design stops solving at its own
+    convergence, and its loads and Ritz residuals still match the oracle's and
+    its own single-design run's."""
+    set_factor(monkeypatch, factor)
     cyl = Cylinder(8, 16, imperfection=(2e-4, 2, 3))
     base = np.random.default_rng(29).uniform(0.0015, 0.0025, cyl.nelems)
     thick = np.stack([base, 1.4 * base, 2.0 * base])
@@ -146,7 +152,7 @@ def test_batched_designs_converging_at_different_steps(monkeypatch):
     assert len(set(steps)) > 1, steps
 
 
-@pytest.mark.parametrize("factor", ["cr", "thomas"])
+@pytest.mark.parametrize("factor", ["nd", "cr", "thomas"])
 def test_solve_graph_replays_match_direct_launches(factor, monkeypatch):
     """The captured solve graph (SHELLGPU_GRAPH=1), replayed with eager work
     between replays and after a refactorisation with new values, gives
