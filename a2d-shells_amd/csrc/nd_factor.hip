@@ -626,9 +626,11 @@ constexpr int kBatch = 8;     // columns of M per wavefront in flight
 // per lane), the columns split over the NW wavefronts.  A level's launch is a
 // chain of memory latencies, so the loads of M (which need nothing of the
 // vector) and the children's part of the rows are issued before the vector is
-// staged, and each batch of columns before the products of the last: a solve
-// of the 200 x 400 cylinder 0.67 -> 0.61 ms (5.0 TB/s over both sweeps), of 16
-// designs of 100 x 200 2.39 -> 2.04 ms.
+// staged, and each batch of columns before the products of the last: solves of
+// the 200 x 400 cylinder, several streams at once, 0.67 -> 0.61 ms each, of 16
+// designs of 100 x 200 2.39 -> 2.04 ms.  With the downward sweep as it is now
+// 0.59 (4.9 TB/s over both sweeps) and 1.96; solves of one stream, whose levels
+// wait for each other, take 0.81 and 2.16.
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void nd_up_kernel(SolveArgs a) {
   __shared__ double vj[kStage];
@@ -680,9 +682,14 @@ __global__ __launch_bounds__(64 * NW) void nd_up_kernel(SolveArgs a) {
 }
 
 // downward sweep: x_J = M^T [y ; x_B], CW columns per wavefront, lanes along
-// the rows (two per lane), the loads of M ahead of the vector as above
-template <int CW>
+// the rows (two per lane), the loads of M ahead of the vector as above.  Four
+// columns at every size: eight take 156 registers instead of 88, three
+// wavefronts per SIMD instead of five, and no size gains by them (a solve of
+// 200 x 400 831 us with eight where a level has 32,768 columns, 805 with four;
+// of 64 designs of 61 x 119 3,196 and 2,921; of 256 of 20 x 40 1,168 and 1,075;
+// of 1,000 of 4 x 8 149 and 126).
 __global__ __launch_bounds__(256) void nd_down_kernel(SolveArgs a) {
+  constexpr int CW = 4;
   constexpr int kRows = 2 * kStage;
   __shared__ __align__(16) double z[kRows];
   const int f = blockIdx.x / a.tiles, c0 = 4 * CW * (blockIdx.x - f * a.tiles);
@@ -1156,14 +1163,8 @@ hipError_t nd_solve(const NdFactor &F, const double *b, double *x, long n, int n
   for (size_t l = F.levels.size(); l-- > 0;) {
     const NdLevel &lv = F.levels[l];
     a.fronts = F.d_fronts + lv.f0;
-    const long cols = (long)lv.nf * lv.max_ns * ne;
-    if (cols >= 32768) {
-      a.tiles = (lv.max_ns + 31) / 32;
-      hipLaunchKernelGGL(nd_down_kernel<8>, dim3((unsigned)(lv.nf * a.tiles), ne), dim3(256), 0, stream, a);
-    } else {
-      a.tiles = (lv.max_ns + 15) / 16;
-      hipLaunchKernelGGL(nd_down_kernel<4>, dim3((unsigned)(lv.nf * a.tiles), ne), dim3(256), 0, stream, a);
-    }
+    a.tiles = (lv.max_ns + 15) / 16;
+    hipLaunchKernelGGL(nd_down_kernel, dim3((unsigned)(lv.nf * a.tiles), ne), dim3(256), 0, stream, a);
   }
   return hipGetLastError();
 }
