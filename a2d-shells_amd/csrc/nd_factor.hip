@@ -628,9 +628,9 @@ constexpr int kBatch = 8;     // columns of M per wavefront in flight
 // vector) and the children's part of the rows are issued before the vector is
 // staged, and each batch of columns before the products of the last: solves of
 // the 200 x 400 cylinder, several streams at once, 0.67 -> 0.61 ms each, of 16
-// designs of 100 x 200 2.39 -> 2.04 ms.  With the launch lines as they are now
-// 0.58 (5.0 TB/s over both sweeps) and 1.89; solves of one stream, whose levels
-// wait for each other, take 0.78 and 2.12.
+// designs of 100 x 200 2.39 -> 2.04 ms.  With the downward sweep as it is now
+// 0.59 (4.9 TB/s over both sweeps) and 1.96; solves of one stream, whose levels
+// wait for each other, take 0.81 and 2.16.
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void nd_up_kernel(SolveArgs a) {
   __shared__ double vj[kStage];
@@ -753,7 +753,7 @@ __global__ __launch_bounds__(256) void nd_down_kernel(SolveArgs a) {
 // panels are read once for up to 16 of them, as matrix products with 16
 // columns (v_mfma_f64_16x16x4f64).  The vectors are interleaved, entry i of
 // vector v at 16 i + v, so every gather along a node list moves whole 128-byte
-// lines.  16 vectors of a 32,000-quad box beam: 0.70 ms a solve (2.3 ms with
+// lines.  16 vectors of a 32,000-quad box beam: 0.79 ms a solve (2.3 ms with
 // the single-vector kernels run once per vector).
 constexpr int kNv = 16;
 
@@ -1113,16 +1113,11 @@ hipError_t nd_solve(const NdFactor &F, const double *b, double *x, long n, int n
       const long rows = (long)lv.nf * F.nbatch * ((lv.max_m + 31) / 32);
       // 32-row pieces of the level: enough of them fill the GPU with whole
       // columns, fewer split the columns over the wavefronts of a workgroup
-      // (16 vectors, us.  First line at 256 / 1,024 / 4,096 / none: 61 x 119
-      // 290 / 283 / 293 / 293, 131 x 211 708 / 683 / 718 / 755, 200 x 400 1,794 /
-      // 1,749 / 1,764 / 1,972, 32,000-quad box beam 727 / 699 / 700 / 759.
-      // Second at 0 / 256 / 1,024: 318 / 283 / 309, 737 / 683 / 718, 1,827 / 1,748 /
-      // 1,766, 740 / 698 / 714)
-      if (rows >= 1024) {
+      if (rows >= 8192) {
         a.tiles = (lv.max_m + 127) / 128;
         hipLaunchKernelGGL((nd_up_multi_kernel<4, 1>), dim3((unsigned)(lv.nf * a.tiles), F.nbatch), dim3(256), 0,
                            stream, a);
-      } else if (rows >= 256) {
+      } else if (rows >= 1024) {
         a.tiles = (lv.max_m + 63) / 64;
         hipLaunchKernelGGL((nd_up_multi_kernel<2, 4>), dim3((unsigned)(lv.nf * a.tiles), F.nbatch), dim3(512), 0,
                            stream, a);
@@ -1137,8 +1132,8 @@ hipError_t nd_solve(const NdFactor &F, const double *b, double *x, long n, int n
       a.fronts = F.d_fronts + lv.f0;
       const long cols = (long)lv.nf * F.nbatch * ((lv.max_ns + 15) / 16);
       // 16-column pieces: many split the rows over 4 wavefronts, few over 16
-      // (16 vectors; line at 0 / 512 / none, us: 61 x 119 327 / 283 / 285, 100 x
-      // 200 611 / 549 / 568, 200 x 400 1,840 / 1,749 / 1,793).  Whole rows per
+      // (16 vectors; line at 0 / 512 / none, us: 61 x 119 363 / 320 / 322, 100 x
+      // 200 676 / 613 / 631, 200 x 400 1,936 / 1,845 / 1,886).  Whole rows per
       // wavefront, tried from 4,096 pieces on, are slower: 200 x 400 1,999
       // against 1,845, 32,000-quad box beam 816 against 762.
       if (cols >= 512) {
@@ -1160,11 +1155,8 @@ hipError_t nd_solve(const NdFactor &F, const double *b, double *x, long n, int n
     a.tiles = (lv.max_m + 127) / 128;
     const long groups = (long)lv.nf * a.tiles * ne;
     // few row tiles (the fronts near the root): more wavefronts share a
-    // tile's columns, so that enough loads are in flight (line at 0 / 256 /
-    // 1,024 / none, us: 61 x 119 147 / 144 / 148 / 148, 100 x 200 284 / 277 / 285 /
-    // 294, 200 x 400 802 / 783 / 792 / 867, 16 designs of 20 x 40 108 / 108 / 114 /
-    // 114, of 61 x 119 788 / 786 / 791 / 875)
-    if (groups < 256)
+    // tile's columns, so that enough loads are in flight
+    if (groups < 1024)
       hipLaunchKernelGGL(nd_up_kernel<16>, dim3((unsigned)(lv.nf * a.tiles), ne), dim3(1024), 0, stream, a);
     else
       hipLaunchKernelGGL(nd_up_kernel<4>, dim3((unsigned)(lv.nf * a.tiles), ne), dim3(256), 0, stream, a);
