@@ -1131,12 +1131,11 @@ hipError_t nd_solve(const NdFactor &F, const double *b, double *x, long n, int n
       const NdLevel &lv = F.levels[l];
       a.fronts = F.d_fronts + lv.f0;
       const long cols = (long)lv.nf * F.nbatch * ((lv.max_ns + 15) / 16);
-      // 16-column pieces: many split the rows over 4 wavefronts, few over 16
-      // (16 vectors; line at 0 / 512 / none, us: 61 x 119 363 / 320 / 322, 100 x
-      // 200 676 / 613 / 631, 200 x 400 1,936 / 1,845 / 1,886).  Whole rows per
-      // wavefront, tried from 4,096 pieces on, are slower: 200 x 400 1,999
-      // against 1,845, 32,000-quad box beam 816 against 762.
-      if (cols >= 512) {
+      if (cols >= 4096) {
+        a.tiles = (lv.max_ns + 127) / 128;
+        hipLaunchKernelGGL((nd_down_multi_kernel<8, 1>), dim3((unsigned)(lv.nf * a.tiles), F.nbatch), dim3(512), 0,
+                           stream, a);
+      } else if (cols >= 512) {
         a.tiles = (lv.max_ns + 31) / 32;
         hipLaunchKernelGGL((nd_down_multi_kernel<2, 4>), dim3((unsigned)(lv.nf * a.tiles), F.nbatch), dim3(512), 0,
                            stream, a);
