@@ -26,7 +26,9 @@
 //
 // The short separators are what this form is for: a band (level) order of the
 // 200 x 400 cylinder stores 27.7 GB and needs 10.6 Tflop, this order 1.45 GB
-// and 0.17 Tflop, and the largest front has 2,400 pivots.  A factorisation is
+// and 0.165 Tflop (0.074 for the panels with their inverses, 0.091 for the
+// Schur complements; a plain Cholesky factor 0.128), and the largest front has
+// 2,400 pivots.  A factorisation is
 // bound by the chain of about 100 pivot blocks of its levels (latency), a
 // solve by the two reads of M and the chain of 2 x 14 levels.
 //
@@ -753,7 +755,7 @@ __global__ __launch_bounds__(256) void nd_down_kernel(SolveArgs a) {
 // panels are read once for up to 16 of them, as matrix products with 16
 // columns (v_mfma_f64_16x16x4f64).  The vectors are interleaved, entry i of
 // vector v at 16 i + v, so every gather along a node list moves whole 128-byte
-// lines.  16 vectors of a 32,000-quad box beam: 0.79 ms a solve (2.3 ms with
+// lines.  16 vectors of a 32,000-quad box beam: 0.82 ms a solve (2.3 ms with
 // the single-vector kernels run once per vector).
 constexpr int kNv = 16;
 
@@ -1113,6 +1115,12 @@ hipError_t nd_solve(const NdFactor &F, const double *b, double *x, long n, int n
       const long rows = (long)lv.nf * F.nbatch * ((lv.max_m + 31) / 32);
       // 32-row pieces of the level: enough of them fill the GPU with whole
       // columns, fewer split the columns over the wavefronts of a workgroup
+      // (16 vectors, us.  First line at 1,024 / 8,192 / none: 61 x 119 309 / 319 /
+      // 319, 200 x 400 1,923 / 1,998 / 2,148, 32,000-quad box beam 771 / 817 / 831.
+      // Second at 0 / 1,024 / 4,096: 329 / 319 / 355, 2,061 / 1,999 / 2,162, 841 /
+      // 816 / 907).  The lines here and below also set the order of the sums: the
+      // lower ones that would be faster move box-beam KS gradients, which lose
+      // digits to cancellation, by 2e-9.
       if (rows >= 8192) {
         a.tiles = (lv.max_m + 127) / 128;
         hipLaunchKernelGGL((nd_up_multi_kernel<4, 1>), dim3((unsigned)(lv.nf * a.tiles), F.nbatch), dim3(256), 0,
@@ -1131,6 +1139,11 @@ hipError_t nd_solve(const NdFactor &F, const double *b, double *x, long n, int n
       const NdLevel &lv = F.levels[l];
       a.fronts = F.d_fronts + lv.f0;
       const long cols = (long)lv.nf * F.nbatch * ((lv.max_ns + 15) / 16);
+      // 16-column pieces: many split the rows over fewer wavefronts (16 vectors,
+      // us.  First line at 512 / 4,096 / none: 61 x 119 322 / 319 / 319, 200 x 400
+      // 2,014 / 2,001 / 1,845, box beam 841 / 816 / 762: whole rows per wavefront
+      // are not the faster form, but see above.  Second at 0 / 512 / 4,096: 363 /
+      // 319 / 320, 2,095 / 2,001 / 1,974, 872 / 817 / 809)
       if (cols >= 4096) {
         a.tiles = (lv.max_ns + 127) / 128;
         hipLaunchKernelGGL((nd_down_multi_kernel<8, 1>), dim3((unsigned)(lv.nf * a.tiles), F.nbatch), dim3(512), 0,
@@ -1154,7 +1167,10 @@ hipError_t nd_solve(const NdFactor &F, const double *b, double *x, long n, int n
     a.tiles = (lv.max_m + 127) / 128;
     const long groups = (long)lv.nf * a.tiles * ne;
     // few row tiles (the fronts near the root): more wavefronts share a
-    // tile's columns, so that enough loads are in flight
+    // tile's columns, so that enough loads are in flight (line at 0 / 256 /
+    // 1,024 / none, us: 61 x 119 147 / 144 / 148 / 148, 100 x 200 284 / 277 / 285 /
+    // 294, 200 x 400 802 / 783 / 792 / 867, 16 designs of 20 x 40 108 / 108 / 114 /
+    // 114, of 61 x 119 788 / 786 / 791 / 875)
     if (groups < 1024)
       hipLaunchKernelGGL(nd_up_kernel<16>, dim3((unsigned)(lv.nf * a.tiles), ne), dim3(1024), 0, stream, a);
     else

@@ -955,9 +955,14 @@ int shellgpu_mat_mult(shellgpu_mat *A, const double *x, double *y) {
 
 // The BC rows an element kernel can write itself: where it writes blocks at
 // their first touch it reaches every block of a row, so the rows need no
-// launch of their own.  Worth a launch while the assembly is short: K of a 4 x 8
-// cylinder 18.5 -> 15.0 us, of 60 x 120 58.9 -> 57.9, of 100 x 150 77.7 -> 75.6;
-// but 243 -> 248 us at 200 x 400, where every lane loads a mask for it.
+// launch of their own, at the price of a mask that every lane loads.  Worth it
+// while the assembly is short (with the launch / without, us, K and G): 4 x 8
+// cylinder K 18.5 / 15.0; 60 x 120 58.1 / 56.6 and 107.2 / 105.0; 90 x 160 74.4 /
+// 72.1 and 187.5 / 185.4; 120 x 240 131.4 / 129.8 and 301.1 / 300.8; even from 140
+// x 280 (147.1 / 144.2 and 374.1 / 374.5) to 160 x 320 (188.1 / 187.6 and 467.6 /
+// 469.2); slower at 200 x 400, 258.1 / 260.3 and 693.2 / 696.7.  The line lies
+// where every matrix type and batch (16 designs of 20 x 40: 73.0 / 70.4 and 185.7
+// / 183.5) gains 1 us or more.
 static const int *bc_rows(const shellgpu_ctx *ctx) {
   const bool small = (long)ctx->nelems * ctx->nbatch <= 16384;
   return small && ctx->d_first && ctx->nbc > 0 && ctx->bc_rows == ctx->nnodes ? ctx->d_bc_rows : nullptr;

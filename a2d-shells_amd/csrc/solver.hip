@@ -34,11 +34,12 @@
 // relative on shell stiffness matrices of condition 1e9 (about ten times
 // smaller than a partial-pivoting LU solve).
 //
-// Block cyclic reduction (below) for a few designs of long level chains.
+// Block cyclic reduction (below) where it is asked for and its blocks fit.
 //
 // A failed Cholesky (non-positive pivot) reports a shift above the first
-// eigenvalue, in every form.  The solve is exact for right-hand sides that vanish on BC
-// dofs (all solves of the buckling path); GMRES corrects the remainder.
+// eigenvalue, in every form.  The solve is exact for right-hand sides that
+// vanish on BC dofs (all solves of the buckling path); GMRES corrects the
+// remainder.
 //
 // GMRES.  Right-preconditioned restarted GMRES with Givens rotations
 // (GMRES::solve, src/bpmat/KSM.cpp:785-955), FP64, preconditioned by the
@@ -132,7 +133,7 @@ struct shellgpu_factor {
   int rhs_cap = 1;           // vectors per design that vb, vz, vx and part hold
   hipGraphExec_t solve_graph = nullptr;  // the single-vector solve body, captured
   bool graph_off = false;
-  // single-vector solves of the sequential form: only designs d_act[0 ..
+  // single-vector solves, but for cyclic reduction: only designs d_act[0 ..
   // nact) when nact >= 0 (Lanczos stops solving for converged designs)
   int *d_act = nullptr;
   int nact = -1;
@@ -1038,7 +1039,14 @@ int setup_plan(shellgpu_factor *F) {
   if ((int)queue.size() < nn) return ferr(ctx, 1, "mesh graph is disconnected from the ordering seed");
 
   // The nested-dissection form (nd_factor.hip) for every mesh and batch; the
-  // level forms below only where SHELLGPU_FACTOR asks for one of them.
+  // level forms below only where SHELLGPU_FACTOR asks for one of them.  Factor
+  // and solve in ms, against the faster level form: 200 x 400 cylinder 12.6 and
+  // 0.80 against 338 and 4.6 (cyclic reduction), 16 designs of 100 x 200 34 and
+  // 2.2 against 339 and 6.3, 64 of 20 x 40 3.0 and 0.31 against 10.4 and 0.67
+  // (sequential).  Solves alone are slower than the sequential form's for
+  // thousands of tiny meshes, whose leaves hold more than their rings do (1,000
+  // designs of 8 x 16 5.1 and 0.63 against 7.8 and 0.38, 4,000 of 4 x 8 3.8 and
+  // 0.50 against 5.9 and 0.28); whole analyses of these take the same time.
   const char *env = getenv("SHELLGPU_FACTOR");
   F->nd = !(env && (strcmp(env, "thomas") == 0 || strcmp(env, "cr") == 0));
   if (F->nd) {
@@ -1644,7 +1652,7 @@ static int gemv_batch(shellgpu_factor *F, bool trans, int m, int n, const double
 // stride nv): one vector per design reads half of P, several read it in
 // full once for all (nrhs <= 8 or 16)
 // vectors per pass when a factor of one design solves n vectors: 16 while
-// there are that many (P read once for 16), else up to 8
+// there are that many (P read once for 16), else up to 8, in every form
 inline int rhs_chunk(int n) { return n >= kMaxRhs ? kMaxRhs : std::min(8, n); }
 static int symv(shellgpu_factor *F, int l, const double *x, double alpha, const double *c, double beta, double *y,
                 int nrhs) {
@@ -2252,7 +2260,7 @@ int apply_block(shellgpu_factor *F, const double *b, double *x, int nrhs, bool m
   shellgpu_ctx *ctx = F->ctx;
   const int nb = F->nbatch;
   const long nv = F->nv, n = F->n;
-  // a Lanczos run may restrict single-vector solves of the sequential form
+  // a Lanczos run may restrict single-vector solves (not of cyclic reduction)
   // to the designs it has not converged yet (the others keep x unchanged)
   const int *act = (!F->cr && nrhs == 1 && F->nact >= 0) ? F->d_act : nullptr;
   if (act && F->nact == 0) return 0;
@@ -2871,7 +2879,7 @@ struct LanczosOut {
 // sigma (mode 2).  Mode 3 is mode 1 with the wanted values the nev smallest
 // |lambda| of either sign (mode 1 wants the smallest positive loads).  Stops
 // when the nev wanted Ritz values have relative residual <= tol.  With a
-// factor of the sequential form per design, a design whose wanted values
+// factor per design, but for cyclic reduction, a design whose wanted values
 // have converged keeps its basis size (lo.ns) and its later solves are
 // skipped; its later basis vectors and projection entries are not used.
 // Otherwise (one factor, or cyclic reduction) every design keeps the whole
@@ -3286,10 +3294,10 @@ int lanczos_block(shellgpu_ctx *ctx, shellgpu_factor *F, shellgpu_mat *K, shellg
 }
 
 // Vectors per Lanczos block: 1 (the single-vector recurrence) unless
-// SHELLGPU_LANCZOS_BLOCK=b (2 ... 8) asks for blocks, which the sequential
-// factorisation and a cyclic-reduction factor of one design solve together
-// (one pass over the factor per block).  Measured on 64 designs of the
-// 100 x 200 cylinder, blocks of 4 read the level inverses 2.5 times less
+// SHELLGPU_LANCZOS_BLOCK=b (2 ... 8) asks for blocks, which the multifrontal
+// and sequential factors and a cyclic-reduction factor of one design solve
+// together (one pass over the factor per block).  Measured on 64 designs of the
+// 100 x 200 cylinder in the sequential form, blocks of 4 read the level inverses 2.5 times less
 // per vector but need a basis as large as the single-vector run's, and the
 // block Gram-Schmidt products (tall, skinny, transposed GEMMs) cost more
 // than the saving.
